@@ -177,7 +177,7 @@ struct bmx_ctx {
   DevBuf<double> d_vpart;      // [slot][vstride] max dt*|vel| per wave/block
   DevBuf<unsigned long long> d_slotmax;  // per-slot maxima (skin check)
   int32_t vmax_slots = 1;
-  int32_t vstride = 1;         // waves of ncap particles (blocks of 64)
+  int32_t vstride = 1;         // tiles (flat_tile) of ncap particles
   int32_t row_nblk = 0;        // blocks of the last row build
   // pinned: err, max row, total (2 words), ..., guard periods' errors
   // (8, 9), the chemistry's size maxima (16..19), the adjoint forward's
@@ -425,15 +425,18 @@ bmx_status ensure_rows(bmx_ctx *c) {
 }
 
 // Per-block partial arrays sized for the smallest block size; the skin
-// check reads every slot, so unused tails stay zero.
+// check reads every slot, so unused tails stay zero.  A displacement slot
+// holds one entry per tile (ensure_rows sets flat_tile first): sphere passes
+// store one per wave of 64 particles, segment passes one per block, and a
+// one-wave block of the segment pass is one tile of 32.
 bmx_status alloc_partials(bmx_ctx *c) {
   c->vmax_slots = std::max(1, c->nbp.rebuild_every);
-  c->vstride = std::max(1, row_blocks(c->ncap, 64));
+  c->vstride = std::max(1, row_blocks(c->ncap, c->flat_tile));
   hipError_t e = c->d_vpart.alloc((size_t)c->vmax_slots * c->vstride);
   if (e == hipSuccess)
     e = launch_fill_u64(reinterpret_cast<unsigned long long *>(c->d_vpart.p),
                         (int64_t)c->vmax_slots * c->vstride, 0ull, c->stream);
-  if (e == hipSuccess) e = c->d_bstats.alloc(2 * (size_t)c->vstride);
+  if (e == hipSuccess) e = c->d_bstats.alloc(2 * (size_t)row_blocks(c->ncap, 64));
   if (e == hipSuccess) e = c->d_slotmax.alloc(c->vmax_slots);
   if (e == hipSuccess)
     e = launch_fill_u64(c->d_slotmax.p, c->vmax_slots, 0ull, c->stream);
@@ -2737,7 +2740,7 @@ constexpr size_t kNaBytes =
     + na_align(4 * kNaFlat) + na_align(kNaFlat)  // cidx, cown
     + 2 * na_align(4 * (kNaBins + 1))            // count, start
     + na_align(4 * ((kNaBins + 2047) / 2048 + 2))  // scan tile sums
-    + na_align(8 * (kNaParticles / 64 + 1) * kNaRebuild)  // displacement slots
+    + na_align(8 * kNaTiles * kNaRebuild)        // displacement slots
     + na_align(8 * kNaRebuild)                   // slot maxima
     + na_align(4 * 2 * (kNaParticles / 64 + 1))  // row-build block stats
     + na_align(4) + na_align(16) + na_align(8) + na_align(64)  // err, stats, total, ustats
@@ -2796,7 +2799,7 @@ bmx_status na_setup(NaDevice &d, int dev) {
   na_slice(c.d_count, cur, (size_t)kNaBins + 1);
   na_slice(c.d_start, cur, (size_t)kNaBins + 1);
   na_slice(c.d_scan, cur, (size_t)(kNaBins + 2047) / 2048 + 2);
-  na_slice(c.d_vpart, cur, (N / 64 + 1) * (size_t)kNaRebuild);
+  na_slice(c.d_vpart, cur, kNaTiles * (size_t)kNaRebuild);
   na_slice(c.d_slotmax, cur, (size_t)kNaRebuild);
   na_slice(c.d_bstats, cur, 2 * (N / 64 + 1));
   na_slice(c.d_err, cur, 1);

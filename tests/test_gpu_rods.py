@@ -201,3 +201,44 @@ def test_reference_single_segment_decks(bmx, oracle, gpu, fname):
         close_fc(ctx.fc(), fo)
     close_traj(ctx, orecs, 0.128)
     assert orecs["pos"][0, 2] != recs["pos"][0, 2]   # it moved
+
+
+@pytest.mark.parametrize("block", [64, 256])
+def test_skin_check_sees_the_last_tiles(bmx, gpu, block):
+    """The displacement record of a Verlet period holds every tile of 32
+    segments at every block size: only the last segments in sorted order
+    move, and the summed bound is compared with skin / 2 from both sides."""
+    n, gap = 512, 1.0e-2                       # 32 x 16 segments, out of reach
+    hi = [32 * gap, 16 * gap, 1.6e-2]
+    recs = bmx.generate_hyphae(n, n, 30e-4, 2e-4, 0.0, 30.0, 60.0, 3, [0, 0, 0], hi, 0.0)
+    k = np.arange(n)
+    recs["pos"][:, 0] = (k % 32 + 0.5) * gap
+    recs["pos"][:, 1] = (k // 32 + 0.5) * gap
+    recs["pos"][:, 2] = 4.0e-3                 # above the surface's reach
+    recs["rdata"][:, 3] = 0.0
+    recs["pos"][-1] = recs["pos"][-2] + [0.0, 0.0, 2.0e-4]   # the last two cross
+    recs["rdata"][-1, 3] = 0.5 * np.pi
+
+    def run(skin, steps):
+        ctx = bmx.Context(0)
+        ctx.set_launch_params(block, 1)
+        ctx.set_force_params(W.hyphae_fpar(0.0))
+        ctx.set_geometry([0, 0, 0], hi, (1, 1, 0), (160, 80, 8))
+        ctx.set_neighbor_params(mode=bmx.NBR_VERLET, rebuild_every=2, skin=skin,
+                                max_neighbors=64)
+        ctx.bind(recs.copy())
+        try:
+            ctx.evolve(W.DT, steps)
+            return W.DT * np.linalg.norm(ctx.fc()[:3], axis=0)
+        finally:
+            ctx.close()
+
+    d = [run(1.0e-3, steps) for steps in (1, 2)]
+    for v in d:
+        assert set(np.argsort(v)[-2:]) == {n - 2, n - 1}
+        assert v[-1] > 100 * v[:-2].max()
+    bound = d[0].max() + d[1].max()
+    run(2.0 * 1.01 * bound, 2)                 # just inside
+    with pytest.raises(bmx.BMXError) as e:
+        run(2.0 * 0.99 * bound, 2)
+    assert e.value.code == 6                   # BMX_ERR_SKIN
