@@ -63,9 +63,8 @@ __global__ __launch_bounds__(kAdjBlock) void k_adj_loss(
   if (threadIdx.x == 0) lpart[blockIdx.x] = sh[0];
 }
 
-// One adjoint step over the flat rows (tiles of 64 particles, one per
-// wave; thread i of block b owns particle 256 b + i as in a row-by-row
-// pass).  Per window of 128 entries the lanes apply the pair test
+// One adjoint step over the flat rows, one tile (64 particles or fewer) per
+// wave; lanes below the tile size own a particle.  Per window of 128 entries the lanes apply the pair test
 // (r_lm - small_number, then r < R_A); the pairs that pass are packed in
 // entry order and their nine terms formed 64 at a time into LDS; every
 // owner adds its own terms in row order.  The owner sums, the surface term
@@ -87,26 +86,27 @@ union AdjLds {
 __global__ __launch_bounds__(kAdjBlock) void k_adj_step(
     const double4 *__restrict__ pos, const int32_t *__restrict__ cidx,
     const uint8_t *__restrict__ cown, const int32_t *__restrict__ wtot,
-    const int32_t *__restrict__ ncnt, int32_t maxn,
+    const int32_t *__restrict__ ncnt, int tsize, int32_t maxn,
     const int32_t *__restrict__ oid, int64_t n, BoxGeom g, ForceParams fp,
     const double4 *__restrict__ lam_in, double4 *__restrict__ lam_out,
     double *__restrict__ grad_r, double *__restrict__ acc) {
   __shared__ AdjLds lds;
   const int lane = threadIdx.x & 63;
   AdjWave &L = lds.w[threadIdx.x / 64];
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const bool active = t < n;
+  const int64_t tile = (int64_t)blockIdx.x * (kAdjBlock / 64) + threadIdx.x / 64;
+  const int64_t t0 = tile * tsize, t = t0 + lane;
+  const bool active = lane < tsize && t < n;
   // Every load that does not depend on another is issued here, before
   // anything waits, from indexes valid for every lane (the last particle
   // for lanes past n, tile 0 for a wave past n): the row length, the wave's
   // entry count, the particle, its adjoint and the first window of entries
   // (a tile's region, and the padding after the last one, is always
   // readable; entries past the count are masked below).
-  const bool live = t - lane < n;  // the wave's tile holds at least one particle
-  const int64_t B = live ? (t / 64) * (int64_t)64 * maxn : 0;
+  const bool live = t0 < n;  // the wave's tile holds at least one particle
+  const int64_t B = live ? t0 * maxn : 0;
   const int64_t tc = active ? t : n - 1;
   const int32_t raw = ncnt[tc];
-  const int32_t T_l = wtot[live ? t / 64 : 0];
+  const int32_t T_l = wtot[live ? tile : 0];
   const double4 p_l = pos[tc];
   const double4 li_l = lam_in[tc];
   int fu[2], fo[2];
@@ -307,27 +307,28 @@ int blocks(int64_t n, int b) {
 
 }  // namespace
 
-int32_t adj_blocks(int64_t n) { return blocks(n, kAdjBlock); }
+int32_t adj_blocks(int64_t n, int tile) { return blocks(n, tile * (kAdjBlock / 64)); }
+int32_t adj_loss_blocks(int64_t n) { return blocks(n, kAdjBlock); }
 
 hipError_t launch_adj_loss(const double4 *pos, const int32_t *oid,
                            const double *target, int64_t n, BoxGeom g,
                            double4 *lam, double *lpart, hipStream_t s) {
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_adj_loss, dim3(blocks(n, kAdjBlock)), dim3(kAdjBlock), 0,
+  hipLaunchKernelGGL(k_adj_loss, dim3(adj_loss_blocks(n)), dim3(kAdjBlock), 0,
                      s, pos, oid, target, n, g, 1.0 / (double)n, lam, lpart);
   return hipGetLastError();
 }
 
 hipError_t launch_adj_step(const double4 *pos, const int32_t *cidx,
                            const uint8_t *cown, const int32_t *wtot,
-                           const int32_t *ncnt, int32_t maxn,
+                           const int32_t *ncnt, int tile, int32_t maxn,
                            const int32_t *oid, int64_t n, BoxGeom g,
                            ForceParams fp, const double4 *lam_in,
                            double4 *lam_out, double *grad_r, double *acc,
                            hipStream_t s) {
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_adj_step, dim3(blocks(n, kAdjBlock)), dim3(kAdjBlock), 0,
-                     s, pos, cidx, cown, wtot, ncnt, maxn, oid, n, g, fp,
+  hipLaunchKernelGGL(k_adj_step, dim3(adj_blocks(n, tile)), dim3(kAdjBlock), 0,
+                     s, pos, cidx, cown, wtot, ncnt, tile, maxn, oid, n, g, fp,
                      lam_in, lam_out, grad_r, acc);
   return hipGetLastError();
 }

@@ -128,11 +128,11 @@ struct bmx_ctx {
   bool count_clear = false;  // d_count holds zeros (the scan resets it)
   DevBuf<unsigned long long> d_permk;
   int32_t maxn = 96;
-  DevBuf<int32_t> d_nbr, d_ncnt;
+  DevBuf<int32_t> d_nbr, d_ncnt;  // row entries past the staged ones; lengths
   // flat row layout of the force pass: per-tile entry totals and bases,
   // entries back to back, the particle's place in its tile per entry
   int flat_tile = 64;
-  DevBuf<int32_t> d_wtot, d_cidx;
+  DevBuf<int32_t> d_wtot, d_cidx, d_roff;
   DevBuf<uint8_t> d_cown;
   DevBuf<int8_t> d_redo;  // segment tiles left to the row loop this step
   // species A, B, C and volume, and their exchange increments, in original
@@ -403,16 +403,37 @@ bmx_status setup_boxes(bmx_ctx *c) {
   return BMX_OK;
 }
 
+// Entries an average row will hold, from the density over all boxes: for
+// Verlet rows the spheres whose centres fit between contact and the list
+// radius, for stencil rows those of the 27 cells (within 'neighborhood').
+// Only the tile size depends on it.
+double row_estimate(const bmx_ctx *c) {
+  double vol = 0.0, cell = 0.0;
+  for (const BoxGeom &b : c->boxes) {
+    const double v = b.L[0] * b.L[1] * b.L[2];
+    vol += v;
+    cell = std::max(cell, v / ((double)b.nbin[0] * b.nbin[1] * b.nbin[2]));
+  }
+  auto ball = [](double r) { return 4.18879020478639 * r * r * r; };
+  double near;
+  if (c->nbp.mode == BMX_NBR_VERLET)
+    near = ball(c->verlet_radius) - ball(2.0 * c->rmax);
+  else
+    near = std::min(27.0 * cell, ball(std::sqrt(std::max(c->crit, 0.0))));
+  return vol > 0.0 ? (double)c->n / vol * near : 0.0;
+}
+
 // Row arrays for ncap particles and maxn entries per row.  A failure leaves
 // the context unbound (the rows would be smaller than the kernels assume).
 bmx_status ensure_rows(bmx_ctx *c) {
   c->have_list = false;
   size_t need = (size_t)c->maxn * (size_t)c->ncap;
-  c->flat_tile = flat_tile(c->any_fungi ? 1 : 0);
+  c->flat_tile = flat_tile(c->any_fungi ? 1 : 0, c->n, row_estimate(c));
   const int64_t nw = (c->ncap + c->flat_tile - 1) / c->flat_tile;
   const int64_t nflat = flat_entries(c->ncap, c->flat_tile, c->maxn);
   hipError_t e = c->d_nbr.alloc(need);
   if (e == hipSuccess) e = c->d_ncnt.alloc(c->ncap);
+  if (e == hipSuccess) e = c->d_roff.alloc(c->ncap);
   if (e == hipSuccess) e = c->d_wtot.alloc(nw + 1);
   if (e == hipSuccess) e = c->d_redo.alloc(nw + 1);
   if (e == hipSuccess) e = c->d_cidx.alloc(nflat);
@@ -424,19 +445,18 @@ bmx_status ensure_rows(bmx_ctx *c) {
   return BMX_OK;
 }
 
-// Per-block partial arrays sized for the smallest block size; the skin
-// check reads every slot, so unused tails stay zero.  A displacement slot
-// holds one entry per tile (ensure_rows sets flat_tile first): sphere passes
-// store one per wave of 64 particles, segment passes one per block, and a
-// one-wave block of the segment pass is one tile of 32.
+// Partial arrays with one entry per tile (ensure_rows sets flat_tile first):
+// the force passes store one displacement maximum and the row build the row
+// statistics of each tile.  The skin check reads every entry, so unused
+// tails stay zero.
 bmx_status alloc_partials(bmx_ctx *c) {
   c->vmax_slots = std::max(1, c->nbp.rebuild_every);
-  c->vstride = std::max(1, row_blocks(c->ncap, c->flat_tile));
+  c->vstride = tile_count(c->ncap, c->flat_tile);
   hipError_t e = c->d_vpart.alloc((size_t)c->vmax_slots * c->vstride);
   if (e == hipSuccess)
     e = launch_fill_u64(reinterpret_cast<unsigned long long *>(c->d_vpart.p),
                         (int64_t)c->vmax_slots * c->vstride, 0ull, c->stream);
-  if (e == hipSuccess) e = c->d_bstats.alloc(2 * (size_t)row_blocks(c->ncap, 64));
+  if (e == hipSuccess) e = c->d_bstats.alloc(2 * (size_t)c->vstride);
   if (e == hipSuccess) e = c->d_slotmax.alloc(c->vmax_slots);
   if (e == hipSuccess)
     e = launch_fill_u64(c->d_slotmax.p, c->vmax_slots, 0ull, c->stream);
@@ -448,7 +468,7 @@ bmx_status alloc_partials(bmx_ctx *c) {
 }
 
 FlatRows flat_rows(bmx_ctx *c) {
-  return FlatRows{c->flat_tile, c->d_cidx.p, c->d_cown.p, c->d_wtot.p};
+  return FlatRows{c->flat_tile, c->d_cidx.p, c->d_cown.p, c->d_wtot.p, c->d_roff.p};
 }
 
 bool verlet_checked(const bmx_ctx *c) {
@@ -472,11 +492,8 @@ bmx_status close_run(bmx_ctx *c) {
 // in force, the displacements since that list was built are checked against
 // skin/2 first and their partials cleared, so every caller that rebuilds
 // (steps, exchange, fusion, InitBonds) starts the next period from zero.
-// check_skin = false is for passes that repeat checked arithmetic.  The
-// force and adjoint passes read the flat rows only; cols = true also writes
-// the column-major rows of a sphere context, for the passes that walk rows
-// that way (segment contexts always have them).
-bmx_status rebuild(bmx_ctx *c, bool check_skin = true, bool cols = false) {
+// check_skin = false is for passes that repeat checked arithmetic.
+bmx_status rebuild(bmx_ctx *c, bool check_skin = true) {
   hipStream_t s = c->stream;
   if (c->timing) {
     bmx_status st = close_run(c);
@@ -522,9 +539,8 @@ bmx_status rebuild(bmx_ctx *c, bool check_skin = true, bool cols = false) {
                           c->n, c->nbp.mode == BMX_NBR_STENCIL ? 1 : 0,
                           c->crit, c->fpar[0], c->nbp.skin, c->d_nbr.p,
                           c->d_ncnt.p, c->ncap, c->maxn, c->d_err.p,
-                          c->d_bstats.p, flat_rows(c), cols ? 1 : 0, shape(c),
-                          s));
-  c->row_nblk = row_blocks(c->n, c->lp.block_size);
+                          c->d_bstats.p, flat_rows(c), c->lp.xcd_remap, s));
+  c->row_nblk = tile_count(c->n, c->flat_tile);
   if (c->timing) {
     HIPCHK(hipEventRecord(e1, s));
     c->ev_rebuild.push_back({e0, e1});
@@ -559,15 +575,14 @@ bmx_status enqueue_step(bmx_ctx *c, double dt, bool write_fc) {
   if (!c->any_fungi) {
     HIPCHK(launch_force_sphere_flat(
         c->pos[c->cd].p, c->pos[1 - c->cd].p, c->d_cidx.p, c->d_cown.p,
-        c->d_wtot.p, c->d_ncnt.p, c->n, c->maxn,
+        c->d_wtot.p, c->d_ncnt.p, c->n, c->flat_tile, c->maxn,
         multi ? c->col[c->cs].p : nullptr, c->d_boxes.p, c->boxes[0], multi,
         fp, fc, c->oid[c->cs].p, vm, c->d_err.p, shape(c), s));
   } else {
     HIPCHK(launch_force_general(
         dyn_arrays(c, c->cd), dyn_arrays(c, 1 - c->cd), static_arrays(c, c->cs),
-        c->d_cidx.p, c->d_cown.p, c->d_wtot.p, c->d_redo.p, c->d_nbr.p,
-        c->d_ncnt.p, c->ncap, c->n, c->maxn, c->d_boxes.p, c->boxes[0], multi,
-        fp, fc, vm, c->d_err.p, shape(c), s));
+        flat_rows(c), c->d_redo.p, c->d_ncnt.p, c->n, c->maxn, c->d_boxes.p,
+        c->boxes[0], multi, fp, fc, vm, c->d_err.p, shape(c), s));
   }
   if (c->timing) c->run_n++;
   c->cd = 1 - c->cd;
@@ -586,7 +601,7 @@ bmx_status enqueue_force_only(bmx_ctx *c, double dt, int slot) {
                    : nullptr;
   HIPCHK(launch_force_sphere_flat(
       c->pos[c->cd].p, c->pos[1 - c->cd].p, c->d_cidx.p, c->d_cown.p,
-      c->d_wtot.p, c->d_ncnt.p, c->n, c->maxn, nullptr, c->d_boxes.p,
+      c->d_wtot.p, c->d_ncnt.p, c->n, c->flat_tile, c->maxn, nullptr, c->d_boxes.p,
       c->boxes[0], 0, fp, nullptr, nullptr, vm, c->d_err.p, shape(c),
       c->stream));
   c->cd = 1 - c->cd;
@@ -958,6 +973,7 @@ void bmx_ctx_destroy(bmx_ctx *c) {
   c->d_scan.release();
   c->d_permk.release();
   c->d_nbr.release();
+  c->d_roff.release();
   c->d_ncnt.release();
   c->d_wtot.release();
   c->d_redo.release();
@@ -1223,7 +1239,7 @@ bmx_status bmx_init_bonds(bmx_ctx *c) {
   if (st != BMX_OK) return st;
   if (c->any_fungi)
     HIPCHK(launch_init_bonds(dyn_arrays(c, c->cd), static_arrays(c, c->cs),
-                             c->d_nbr.p, c->d_ncnt.p, c->ncap, c->n,
+                             flat_rows(c), c->maxn, c->d_ncnt.p, c->n,
                              c->d_boxes.p, c->boxes[0], c->ncol > 1,
                              force_params(c, 0.0), c->d_err.p, c->stream));
   // the first evolve step rebuilds, as EvolveParticles does after InitBonds
@@ -1700,9 +1716,9 @@ bmx_status bmx_adjoint(bmx_ctx *c, double dt, int32_t nsteps,
   HIPCHK(A.lam1.alloc(cap));
   HIPCHK(A.lamo.alloc(cap));
   HIPCHK(A.fin.alloc(cap));
-  const int32_t nblk = adj_blocks(n);
+  const int32_t nblk = adj_blocks(n, c->flat_tile), nloss = adj_loss_blocks(n);
   HIPCHK(A.acc.alloc(3 * (size_t)nblk));
-  HIPCHK(A.lpart.alloc((size_t)nblk));
+  HIPCHK(A.lpart.alloc((size_t)nloss));
   HIPCHK(A.out.alloc(4));
   double *d_gr = A.gr.p, *d_acc = A.acc.p, *d_lpart = A.lpart.p, *d_out = A.out.p;
   double4 *d_ckpt = A.ckpt.p, *d_lamo = A.lamo.p, *d_final = A.fin.p;
@@ -1797,7 +1813,7 @@ bmx_status bmx_adjoint(bmx_ctx *c, double dt, int32_t nsteps,
         HIPCHK(launch_force_sphere_flat(
             H.pos.p + (size_t)t * cap, H.pos.p + (size_t)(t + 1) * cap,
             c->d_cidx.p, c->d_cown.p, c->d_wtot.p, c->d_ncnt.p, c->n,
-            c->maxn, nullptr, c->d_boxes.p, c->boxes[0], 0, fp, nullptr,
+            c->flat_tile, c->maxn, nullptr, c->d_boxes.p, c->boxes[0], 0, fp, nullptr,
             nullptr, nullptr, c->d_err.p, shape(c), s));
     }
     HIPCHK(hipEventRecord(A.rdone[hs], s));
@@ -1811,7 +1827,7 @@ bmx_status bmx_adjoint(bmx_ctx *c, double dt, int32_t nsteps,
       HIPCHK(launch_adj_step(H.pos.p + (size_t)t * cap, H.idx.p + (size_t)r * rowbuf,
                              H.own.p + (size_t)r * rowbuf,
                              H.tot.p + (size_t)r * tilebuf,
-                             H.cnt.p + (size_t)r * cap, c->maxn, oid, n,
+                             H.cnt.p + (size_t)r * cap, c->flat_tile, c->maxn, oid, n,
                              c->boxes[0], fp, lam_in, lam_out, d_gr, d_acc, s2));
       std::swap(lam_in, lam_out);
       if (t % K == 0 && t > 0) {  // back across a rebuild: reorder lambda
@@ -1827,7 +1843,7 @@ bmx_status bmx_adjoint(bmx_ctx *c, double dt, int32_t nsteps,
   HIPCHK(hipEventRecord(A.join, s2));
   HIPCHK(hipStreamWaitEvent(s, A.join, 0));
   HIPCHK(launch_sum_partials(d_acc, nblk, 3, d_out, s));
-  HIPCHK(launch_sum_partials(d_lpart, nblk, 1, d_out + 3, s));
+  HIPCHK(launch_sum_partials(d_lpart, nloss, 1, d_out + 3, s));
   HIPCHK(hipEventRecord(e2, s));
   // leave the context in the final forward state
   HIPCHK(launch_from_orig4(d_final, c->oid[c->cs].p, n, c->pos[c->cd].p, s));
@@ -2054,10 +2070,10 @@ extern "C" bmx_status bmx_exchange(bmx_ctx *c, const double xpar[3], double dt) 
   st = load_chem(c);
   if (st != BMX_OK) return st;
   // the rows are rebuilt at the current positions (xchng.cpp:68-77)
-  st = rebuild(c, true, true);
+  st = rebuild(c);
   if (st != BMX_OK) return st;
   HIPCHK(launch_exchange(c->pos[c->cd].p, c->type[c->cs].p, c->topo[c->cd].p,
-                         c->d_nbr.p, c->d_ncnt.p, c->ncap, c->n,
+                         flat_rows(c), c->maxn, c->d_ncnt.p, c->n,
                          c->d_chemst[c->cc].p, xpar, dt, s));
   return check_flags(c);
 }
@@ -2628,7 +2644,7 @@ extern "C" bmx_status bmx_fusion(bmx_ctx *c, const bmx_fusion_params *fp,
   // records and rows at the current positions (EvaluateTipFusion rebuilds)
   st = pack_records(c);
   if (st != BMX_OK) return st;
-  st = rebuild(c, true, true);
+  st = rebuild(c);
   if (st != BMX_OK) return st;
   st = check_flags(c);
   if (st != BMX_OK) return st;
@@ -2644,7 +2660,7 @@ extern "C" bmx_status bmx_fusion(bmx_ctx *c, const bmx_fusion_params *fp,
   HIPCHK(ttau.alloc((size_t)n + 1));
   HIPCHK(launch_fill_i32(flag.p, 1, 0, s));
   HIPCHK(launch_tip_fusion(c->recs, c->lay, n, c->pos[c->cd].p,
-                           c->oid[c->cs].p, c->d_nbr.p, c->d_ncnt.p, c->ncap, g0,
+                           c->oid[c->cs].p, flat_rows(c), c->maxn, c->d_ncnt.p, g0,
                            wa, fus, seed, call, tgt.p, ttau.p, flag.p, s));
   int32_t any = 0;
   HIPCHK(hipMemcpyAsync(&any, flag.p, sizeof any, hipMemcpyDeviceToHost, s));
@@ -2665,7 +2681,7 @@ extern "C" bmx_status bmx_fusion(bmx_ctx *c, const bmx_fusion_params *fp,
   HIPCHK(dec.alloc((size_t)n));
   HIPCHK(dtau.alloc((size_t)n));
   HIPCHK(launch_interior_fusion(c->recs, c->lay, n, c->pos[c->cd].p,
-                                c->oid[c->cs].p, c->d_nbr.p, c->d_ncnt.p, c->ncap,
+                                c->oid[c->cs].p, flat_rows(c), c->maxn, c->d_ncnt.p,
                                 g0, wa, cnt.p, dec.p, dtau.p, one.p, s));
   HIPCHK(launch_scan(one.p, start.p, n, scratch.p, s));
   int32_t total = 0;
@@ -2687,12 +2703,12 @@ extern "C" bmx_status bmx_fusion(bmx_ctx *c, const bmx_fusion_params *fp,
   if (st != BMX_OK) return st;
   grown.release();
   // cleanup over rows rebuilt with the new segments
-  st = rebuild(c, true, true);
+  st = rebuild(c);
   if (st != BMX_OK) return st;
   st = check_flags(c);
   if (st != BMX_OK) return st;
   HIPCHK(launch_fusion_cleanup(c->recs, c->lay, c->n, c->pos[c->cd].p,
-                               c->oid[c->cs].p, c->d_nbr.p, c->d_ncnt.p, c->ncap,
+                               c->oid[c->cs].p, flat_rows(c), c->maxn, c->d_ncnt.p,
                                c->boxes[0], fus[2], 1.5 * fus[3], s));
   HIPCHK(hipStreamSynchronize(s));
   void *user = c->user_aos;
@@ -2724,8 +2740,8 @@ constexpr int kNaDevices = 64;
 constexpr size_t na_align(size_t b) { return (b + 255) / 256 * 256; }
 
 // Bytes of each slice of the scratch, in carve order.
-constexpr size_t kNaTiles = (size_t)(kNaParticles + 31) / 32 + 1;  // tiles of 32
-constexpr size_t kNaFlat = (size_t)kNaTiles * 32 * kNaNeighbors + 2 * 64;
+constexpr size_t kNaTiles = (size_t)(kNaParticles + 3) / 4 + 1;  // the smallest tiles
+constexpr size_t kNaFlat = (size_t)(kNaParticles + 64) * kNaNeighbors + 2 * 64;
 constexpr size_t kNaBytes =
     2 * 3 * na_align(4 * kNaParticles)           // oid, type, key
     + 2 * na_align(8 * kNaParticles)             // bscale
@@ -2734,15 +2750,15 @@ constexpr size_t kNaBytes =
     + 2 * na_align(4 * kNaParticles)             // keytmp, rank
     + na_align(8 * kNaParticles)                 // permk
     + na_align(8 * 6 * kNaParticles)             // fc
-    + na_align(4 * kNaNeighbors * kNaParticles)  // nbr (column-major rows)
-    + na_align(4 * kNaParticles)                 // ncnt
+    + na_align(4 * kNaNeighbors * kNaParticles)  // nbr (long rows)
+    + 2 * na_align(4 * kNaParticles)             // ncnt, roff
     + na_align(4 * kNaTiles) + na_align(kNaTiles)  // wtot, redo
     + na_align(4 * kNaFlat) + na_align(kNaFlat)  // cidx, cown
     + 2 * na_align(4 * (kNaBins + 1))            // count, start
     + na_align(4 * ((kNaBins + 2047) / 2048 + 2))  // scan tile sums
     + na_align(8 * kNaTiles * kNaRebuild)        // displacement slots
     + na_align(8 * kNaRebuild)                   // slot maxima
-    + na_align(4 * 2 * (kNaParticles / 64 + 1))  // row-build block stats
+    + na_align(4 * 2 * kNaTiles)                 // row-build block stats
     + na_align(4) + na_align(16) + na_align(8) + na_align(64)  // err, stats, total, ustats
     + na_align(sizeof(BoxGeom));
 
@@ -2792,6 +2808,7 @@ bmx_status na_setup(NaDevice &d, int dev) {
   na_slice(c.d_fc, cur, 6 * N);
   na_slice(c.d_nbr, cur, (size_t)kNaNeighbors * N);
   na_slice(c.d_ncnt, cur, N);
+  na_slice(c.d_roff, cur, N);
   na_slice(c.d_wtot, cur, kNaTiles);
   na_slice(c.d_redo, cur, kNaTiles);
   na_slice(c.d_cidx, cur, kNaFlat);
@@ -2801,7 +2818,7 @@ bmx_status na_setup(NaDevice &d, int dev) {
   na_slice(c.d_scan, cur, (size_t)(kNaBins + 2047) / 2048 + 2);
   na_slice(c.d_vpart, cur, kNaTiles * (size_t)kNaRebuild);
   na_slice(c.d_slotmax, cur, (size_t)kNaRebuild);
-  na_slice(c.d_bstats, cur, 2 * (N / 64 + 1));
+  na_slice(c.d_bstats, cur, 2 * kNaTiles);
   na_slice(c.d_err, cur, 1);
   na_slice(c.d_stats, cur, 4);
   na_slice(c.d_total, cur, 1);

@@ -87,9 +87,9 @@ __device__ __forceinline__ double species_flux(double c1, double c2, double area
 __global__ void k_exchange_rows(const double4 *__restrict__ pos,
                                 const int32_t *__restrict__ type,
                                 const Topo *__restrict__ topo,
-                                const int32_t *__restrict__ nbr,
-                                const int32_t *__restrict__ ncnt, int64_t ncap,
-                                int64_t n, double *__restrict__ state,
+                                FlatRows flat, int32_t maxn,
+                                const int32_t *__restrict__ ncnt, int64_t n,
+                                double *__restrict__ state,
                                 double mtA, double mtB, double mtC, double dt) {
   int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= n || type[t] != rec::FUNGI) return;
@@ -98,9 +98,9 @@ __global__ void k_exchange_rows(const double4 *__restrict__ pos,
   const double4 c1 = *reinterpret_cast<const double4 *>(state + t * chem::stride);
   double ia = 0.0, ib = 0.0, ic = 0.0;  // initExchange
   const int c = ncnt[t] & ((1 << 28) - 1);  // bits 28..30: image axes
-  const int32_t *rp = nbr + t;
-  for (int k = 0; k < c; k++, rp += ncap) {
-    const int u = *rp;
+  const int32_t *row = flat.cidx + row_base(flat, maxn, t);
+  for (int k = 0; k < c; k++) {
+    const int u = row[k];
     if (type[u] != rec::FUNGI) continue;
     const Topo tj = topo[u];
     int bi, bj;
@@ -162,13 +162,12 @@ hipError_t launch_chem_pack(uint8_t *aos, AosLayout lay, int64_t n,
 }
 
 hipError_t launch_exchange(const double4 *pos, const int32_t *type,
-                           const Topo *topo,
-                           const int32_t *nbr, const int32_t *ncnt,
-                           int64_t ncap, int64_t n, double *state,
+                           const Topo *topo, FlatRows flat, int32_t maxn,
+                           const int32_t *ncnt, int64_t n, double *state,
                            const double xpar[3], double dt, hipStream_t s) {
   if (n <= 0) return hipSuccess;
   hipLaunchKernelGGL(k_exchange_rows, dim3(grid256(n)), dim3(256), 0, s, pos,
-                     type, topo, nbr, ncnt, ncap, n, state, xpar[0],
+                     type, topo, flat, maxn, ncnt, n, state, xpar[0],
                      xpar[1], xpar[2], dt);
   hipLaunchKernelGGL(k_exchange_apply, dim3(grid256(n)), dim3(256), 0, s, type,
                      n, state);

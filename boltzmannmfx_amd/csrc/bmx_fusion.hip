@@ -148,8 +148,8 @@ __device__ void tip_apply(double *ir, int32_t *ii, int32_t j_id, int32_t j_cpu,
 __global__ void k_tip_decide(const uint8_t *__restrict__ aos, AosLayout lay,
                              int64_t n, const double4 *__restrict__ pos,
                              const int32_t *__restrict__ oid,
-                             const int32_t *__restrict__ nbr,
-                             const int32_t *__restrict__ ncnt, int64_t ncap,
+                             FlatRows flat, int32_t maxn,
+                             const int32_t *__restrict__ ncnt,
                              BoxGeom g, double wa, FusionParams P,
                              uint64_t seed, uint32_t call,
                              int32_t *__restrict__ tgt,
@@ -170,8 +170,9 @@ __global__ void k_tip_decide(const uint8_t *__restrict__ aos, AosLayout lay,
   const int32_t cpu = *reinterpret_cast<const int32_t *>(base + lay.cpu);
   uint32_t draw = 0;
   const int c = ncnt[t] & ((1 << 28) - 1);
+  const int32_t *row = flat.cidx + row_base(flat, maxn, t);
   for (int k = 0; k < c; k++) {
-    const int u = nbr[(int64_t)k * ncap + t];
+    const int u = row[k];
     RecP b = recp(ab, lay, oid[u]);
     double d[3];
     separation(pi, pos[u], g, d);
@@ -207,9 +208,8 @@ __global__ void k_tip_apply(uint8_t *__restrict__ aos, AosLayout lay, int64_t n,
 __global__ void k_interior_decide(uint8_t *__restrict__ aos, AosLayout lay,
                                   int64_t n, const double4 *__restrict__ pos,
                                   const int32_t *__restrict__ oid,
-                                  const int32_t *__restrict__ nbr,
-                                  const int32_t *__restrict__ ncnt,
-                                  int64_t ncap, BoxGeom g, double wa,
+                                  FlatRows flat, int32_t maxn,
+                                  const int32_t *__restrict__ ncnt, BoxGeom g, double wa,
                                   int32_t *__restrict__ cnt,
                                   int4 *__restrict__ dec,
                                   double *__restrict__ dtau) {
@@ -223,8 +223,9 @@ __global__ void k_interior_decide(uint8_t *__restrict__ aos, AosLayout lay,
   if (a.ip[rec::position] != rec::TIP) {
     const double4 pi = pos[t];
     const int c = ncnt[t] & ((1 << 28) - 1);
+    const int32_t *row = flat.cidx + row_base(flat, maxn, t);
     for (int k = 0; k < c; k++) {
-      const int u = nbr[(int64_t)k * ncap + t];
+      const int u = row[k];
       RecP b = recp(aos, lay, oid[u]);
       if (!(b.ip[rec::fuse_flag] == 1)) continue;
       double d[3];
@@ -461,9 +462,8 @@ __device__ void cleanup_bond(int32_t *ip, const int32_t *jp) {
 __global__ void k_fusion_cleanup(uint8_t *__restrict__ aos, AosLayout lay,
                                  int64_t n, const double4 *__restrict__ pos,
                                  const int32_t *__restrict__ oid,
-                                 const int32_t *__restrict__ nbr,
-                                 const int32_t *__restrict__ ncnt,
-                                 int64_t ncap, BoxGeom g, double scale_inc,
+                                 FlatRows flat, int32_t maxn,
+                                 const int32_t *__restrict__ ncnt, BoxGeom g, double scale_inc,
                                  double reach) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= n) return;
@@ -476,8 +476,9 @@ __global__ void k_fusion_cleanup(uint8_t *__restrict__ aos, AosLayout lay,
   if (a.rd[rec::bond_scale] >= 1.0) a.ip[rec::fuse_tip] = 0;
   const double4 pi = pos[t];
   const int c = ncnt[t] & ((1 << 28) - 1);
+  const int32_t *row = flat.cidx + row_base(flat, maxn, t);
   for (int k = 0; k < c; k++) {
-    const int u = nbr[(int64_t)k * ncap + t];
+    const int u = row[k];
     double d[3];
     separation(pi, pos[u], g, d);
     const double r2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
@@ -492,15 +493,15 @@ int grid_of(int64_t n) { return (int)((n + 255) / 256 > 0 ? (n + 255) / 256 : 1)
 
 hipError_t launch_tip_fusion(uint8_t *aos, AosLayout lay, int64_t n,
                              const double4 *pos, const int32_t *oid,
-                             const int32_t *nbr, const int32_t *ncnt,
-                             int64_t ncap, const BoxGeom &g, double wa,
+                             FlatRows flat, int32_t maxn,
+                             const int32_t *ncnt, const BoxGeom &g, double wa,
                              const double fus[4], uint64_t seed, uint32_t call,
                              int32_t *tgt, double *ttau, int32_t *fused,
                              hipStream_t s) {
   if (n <= 0) return hipSuccess;
   FusionParams P{fus[0], fus[1], fus[2], fus[3]};
   hipLaunchKernelGGL(k_tip_decide, dim3(grid_of(n)), dim3(256), 0, s, aos, lay, n,
-                     pos, oid, nbr, ncnt, ncap, g, wa, P, seed, call, tgt, ttau,
+                     pos, oid, flat, maxn, ncnt, g, wa, P, seed, call, tgt, ttau,
                      fused);
   hipLaunchKernelGGL(k_tip_apply, dim3(grid_of(n)), dim3(256), 0, s, aos, lay, n,
                      oid, tgt, ttau);
@@ -509,13 +510,13 @@ hipError_t launch_tip_fusion(uint8_t *aos, AosLayout lay, int64_t n,
 
 hipError_t launch_interior_fusion(uint8_t *aos, AosLayout lay, int64_t n,
                                   const double4 *pos, const int32_t *oid,
-                                  const int32_t *nbr, const int32_t *ncnt,
-                                  int64_t ncap, const BoxGeom &g, double wa,
+                                  FlatRows flat, int32_t maxn,
+                                  const int32_t *ncnt, const BoxGeom &g, double wa,
                                   int32_t *cnt, int4 *dec, double *dtau,
                                   int32_t *one, hipStream_t s) {
   if (n <= 0) return hipSuccess;
   hipLaunchKernelGGL(k_interior_decide, dim3(grid_of(n)), dim3(256), 0, s, aos,
-                     lay, n, pos, oid, nbr, ncnt, ncap, g, wa, cnt, dec, dtau);
+                     lay, n, pos, oid, flat, maxn, ncnt, g, wa, cnt, dec, dtau);
   hipLaunchKernelGGL(k_interior_apply, dim3(grid_of(n)), dim3(256), 0, s, aos,
                      lay, n, cnt, dec, dtau, one);
   return hipGetLastError();
@@ -532,13 +533,13 @@ hipError_t launch_fusion_split(uint8_t *aos, AosLayout lay, int64_t n,
 
 hipError_t launch_fusion_cleanup(uint8_t *aos, AosLayout lay, int64_t n,
                                  const double4 *pos, const int32_t *oid,
-                                 const int32_t *nbr, const int32_t *ncnt,
-                                 int64_t ncap, const BoxGeom &g,
+                                 FlatRows flat, int32_t maxn,
+                                 const int32_t *ncnt, const BoxGeom &g,
                                  double scale_inc, double reach,
                                  hipStream_t s) {
   if (n <= 0) return hipSuccess;
   hipLaunchKernelGGL(k_fusion_cleanup, dim3(grid_of(n)), dim3(256), 0, s, aos,
-                     lay, n, pos, oid, nbr, ncnt, ncap, g, scale_inc, reach);
+                     lay, n, pos, oid, flat, maxn, ncnt, g, scale_inc, reach);
   return hipGetLastError();
 }
 

@@ -11,16 +11,24 @@ struct LaunchShape {
 };
 
 // Flat row layout written by the list build: each tile of 'tile' particles
-// (64 for spheres, 32 for segment contexts) has its rows back to back in
-// cidx from the start of its own region (tile index * tile * maxn), tot[tile]
-// entries, with the particle's place in the tile beside every entry in
-// cown.  cidx == nullptr builds no flat rows.
+// (flat_tile) has its rows back to back in cidx from the start of its own
+// region (tile index * tile * maxn), tot[tile] entries, with the particle's
+// place in the tile beside every entry in cown.  Particle t's row starts at
+// roff[t] of its tile's region (row_base).
 struct FlatRows {
   int tile;
   int32_t *cidx;
   uint8_t *cown;
   int32_t *tot;
+  int32_t *roff;
 };
+__device__ __forceinline__ int64_t row_base(const FlatRows &f, int32_t maxn,
+                                            int64_t t) {
+  return t / f.tile * f.tile * (int64_t)maxn + f.roff[t];
+}
+// Particles per tile for a context of n particles whose rows hold about
+// 'row' entries (4 to 64; segment and mixed contexts: 4 to 16).
+int flat_tile(int segments, int64_t n, double row);
 // Entries to allocate for the flat rows of ncap particles.
 int64_t flat_entries(int64_t ncap, int tile, int32_t maxn);
 
@@ -92,10 +100,9 @@ hipError_t launch_sort_gather(const unsigned long long *permk,
                               const double *chem_src = nullptr,
                               double *chem_dst = nullptr);
 
-// ---- neighbor list: flat rows (FlatRows) always; column-major rows
-// nbr[k*ncap + i] for segment contexts, and for sphere contexts only when
-// cols = 1 (the passes that walk rows that way: exchange, fusion); ncnt
-// holds the row length, bits 28..30 the axes that may need a periodic image
+// ---- neighbor list: flat rows (FlatRows); nbr: maxn * ncap entries of
+// scratch for rows longer than the build stages on chip; ncnt holds the row
+// length, bits 28..30 the axes that may need a periodic image
 // mode 0: r2 <= (reach_i + reach_j + wa + skin)^2 (reach = radius, or 1.5 *
 // c_length for segments); mode 1: r2 <= crit (the neighborhood value)
 hipError_t launch_build_nbr(const double4 *pos, const int32_t *col,
@@ -105,27 +112,24 @@ hipError_t launch_build_nbr(const double4 *pos, const int32_t *col,
                             int64_t n, int mode, double crit, double wa,
                             double skin, int32_t *nbr, int32_t *ncnt,
                             int64_t ncap, int32_t maxn, int32_t *err,
-                            int32_t *bstats, FlatRows flat, int cols,
-                            LaunchShape ls, hipStream_t s);
-// Particles per tile of the flat row layout: 64 for spheres, 32 for
-// segment (and mixed) contexts.
-int flat_tile(int segments);
+                            int32_t *bstats, FlatRows flat, int remap,
+                            hipStream_t s);
 // Sphere force + overdamped update, fused, over the flat row layout.  fc
 // (6*ncap, original order: fc[oid + c*ncap]) is written when non-null,
-// with fc_oid the original index of each sorted row; vmax[wave] receives
-// the wave's max dt*|vel| when non-null.
+// with fc_oid the original index of each sorted row; vmax[tile] receives
+// the tile's max dt*|vel| when non-null.
 hipError_t launch_force_sphere_flat(const double4 *pos_in, double4 *pos_out,
                                     const int32_t *cidx, const uint8_t *cown,
                                     const int32_t *wtot, const int32_t *ncnt,
-                                    int64_t n, int32_t maxn,
+                                    int64_t n, int tile, int32_t maxn,
                                     const int32_t *col,
                                     const BoxGeom *boxes, BoxGeom g0, int multi,
                                     ForceParams fp, double *fc,
                                     const int32_t *fc_oid, double *vmax,
                                     int32_t *err, LaunchShape ls,
                                     hipStream_t s);
-// blocks of a row build / force launch over n particles (partial arrays)
-int32_t row_blocks(int64_t n, int block);
+// tiles of n particles (at least one)
+int32_t tile_count(int64_t n, int tile);
 // The end of a call in one launch: row statistics (nblk > 0), then err,
 // longest row and entry total (low, high word) into host_out (host memory
 // mapped for the device), err cleared.
@@ -138,22 +142,20 @@ hipError_t launch_reduce_rowstats(const int32_t *bstats, int32_t nblk,
                                   hipStream_t s);
 
 // ---- segment (and mixed) force + overdamped update, fused: fc and vmax
-// as for launch_force_sphere_flat, vmax per block.
+// as for launch_force_sphere_flat.
 hipError_t launch_force_general(DynArrays in, DynArrays out, StaticArrays st,
-                                const int32_t *cidx, const uint8_t *cown,
-                                const int32_t *wtot, int8_t *redo_tile,
-                                const int32_t *nbr, const int32_t *ncnt,
-                                int64_t ncap, int64_t n, int32_t maxn,
+                                FlatRows flat, int8_t *redo_tile,
+                                const int32_t *ncnt, int64_t n, int32_t maxn,
                                 const BoxGeom *boxes, BoxGeom g0, int multi,
                                 ForceParams fp, double *fc, double *vmax,
                                 int32_t *err, LaunchShape ls, hipStream_t s);
-hipError_t launch_init_bonds(DynArrays dy, StaticArrays st, const int32_t *nbr,
-                             const int32_t *ncnt, int64_t ncap, int64_t n,
+hipError_t launch_init_bonds(DynArrays dy, StaticArrays st, FlatRows flat,
+                             int32_t maxn, const int32_t *ncnt, int64_t n,
                              const BoxGeom *boxes, BoxGeom g0, int multi,
                              ForceParams fp, int32_t *err, hipStream_t s);
 // Displacement record of the Verlet skin check: one slot of `stride`
-// doubles per step since the last rebuild; force kernels store each wave's
-// (or block's) largest dt*|vel| at its index in their step's slot.
+// doubles per step since the last rebuild; force kernels store each tile's
+// largest dt*|vel| at its index in their step's slot.
 // sum over slots of max over the slot > limit -> err |= ERRBIT_SKIN;
 // clear = 1 zeroes the partials (at a rebuild).  slotmax: nslots zeroed
 // words of scratch (left zeroed).
@@ -180,13 +182,14 @@ hipError_t launch_export_counts(const int32_t *ncnt, const int32_t *oid,
                                 hipStream_t s);
 
 // ---- adjoint of the sphere step (bmx_adjoint.hip)
-int32_t adj_blocks(int64_t n);
+int32_t adj_blocks(int64_t n, int tile);  // of a reverse step
+int32_t adj_loss_blocks(int64_t n);       // of the loss
 hipError_t launch_adj_loss(const double4 *pos, const int32_t *oid,
                            const double *target, int64_t n, BoxGeom g,
                            double4 *lam, double *lpart, hipStream_t s);
 hipError_t launch_adj_step(const double4 *pos, const int32_t *cidx,
                            const uint8_t *cown, const int32_t *wtot,
-                           const int32_t *ncnt, int32_t maxn,
+                           const int32_t *ncnt, int tile, int32_t maxn,
                            const int32_t *oid, int64_t n, BoxGeom g,
                            ForceParams fp, const double4 *lam_in,
                            double4 *lam_out, double *grad_r, double *acc,
@@ -226,9 +229,8 @@ hipError_t launch_chem_pack(uint8_t *aos, AosLayout lay, int64_t n,
                             hipStream_t s);
 // ParticleExchange (bmx_exchange.hip) on the chemistry state
 hipError_t launch_exchange(const double4 *pos, const int32_t *type,
-                           const Topo *topo,
-                           const int32_t *nbr, const int32_t *ncnt,
-                           int64_t ncap, int64_t n, double *state,
+                           const Topo *topo, FlatRows flat, int32_t maxn,
+                           const int32_t *ncnt, int64_t n, double *state,
                            const double xpar[3], double dt, hipStream_t s);
 
 // ---- particle <-> mesh (bmx_mesh.hip), over the sorted arrays
@@ -280,16 +282,16 @@ hipError_t launch_split_apply(uint8_t *aos, AosLayout lay, int64_t n,
 // applies the decisions
 hipError_t launch_tip_fusion(uint8_t *aos, AosLayout lay, int64_t n,
                              const double4 *pos, const int32_t *oid,
-                             const int32_t *nbr, const int32_t *ncnt,
-                             int64_t ncap, const BoxGeom &g, double wa,
+                             FlatRows flat, int32_t maxn, const int32_t *ncnt,
+                             const BoxGeom &g, double wa,
                              const double fus[4], uint64_t seed, uint32_t call,
                              int32_t *tgt, double *ttau, int32_t *fused,
                              hipStream_t s);
 // cnt[o]: tips that fused into o; one[o] = (cnt[o] == 1), the new segments
 hipError_t launch_interior_fusion(uint8_t *aos, AosLayout lay, int64_t n,
                                   const double4 *pos, const int32_t *oid,
-                                  const int32_t *nbr, const int32_t *ncnt,
-                                  int64_t ncap, const BoxGeom &g, double wa,
+                                  FlatRows flat, int32_t maxn,
+                                  const int32_t *ncnt, const BoxGeom &g, double wa,
                                   int32_t *cnt, int4 *dec, double *dtau,
                                   int32_t *one, hipStream_t s);
 hipError_t launch_fusion_split(uint8_t *aos, AosLayout lay, int64_t n,
@@ -297,8 +299,8 @@ hipError_t launch_fusion_split(uint8_t *aos, AosLayout lay, int64_t n,
                                int32_t next_id, int32_t cpu, hipStream_t s);
 hipError_t launch_fusion_cleanup(uint8_t *aos, AosLayout lay, int64_t n,
                                  const double4 *pos, const int32_t *oid,
-                                 const int32_t *nbr, const int32_t *ncnt,
-                                 int64_t ncap, const BoxGeom &g,
+                                 FlatRows flat, int32_t maxn,
+                                 const int32_t *ncnt, const BoxGeom &g,
                                  double scale_inc, double reach,
                                  hipStream_t s);
 

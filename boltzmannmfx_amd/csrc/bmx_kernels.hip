@@ -4,9 +4,9 @@
 // (floor((x - plo) * dxi), src/interpolation/bmx_interp_K.H:55-56), counts
 // bins with atomics, scans the counts, scatters (original index, slot)
 // pairs, orders each bin by original index, gathers every per-particle array
-// into the new order and builds column-major neighbor rows over the +-1 bin
-// stencil (spheres: then copied into a flat layout, each wave's rows back to
-// back).  Rows are visited in a fixed order (stencil offsets dz, dy, dx
+// into the new order and builds the neighbor rows over the +-1 bin stencil
+// in a flat layout, the rows of a force wave's tile of particles back to
+// back.  Rows are visited in a fixed order (stencil offsets dz, dy, dx
 // lexicographic, ascending original index inside a bin), so the force pass
 // sums each particle's pair terms in an order that does not depend on
 // thread scheduling.  The force kernel is a gather: particle i reads its row
@@ -14,6 +14,7 @@
 // does (src/des/bmx_pc_interaction.cpp:170-279), then applies the overdamped
 // update (src/des/bmx_pc_interaction.cpp:311-449) in the same launch,
 // writing the next state into the other half of a ping-pong pair.
+#include <algorithm>
 #include <type_traits>
 
 #include "bmx_device.h"
@@ -592,51 +593,6 @@ __device__ __forceinline__ double sep_m(double xi, double xj, const BoxGeom &g) 
   return xi - xj;
 }
 
-// Scans one contiguous candidate range [ua, ub) of the sorted arrays and
-// appends the accepted candidates to the row (out walks the column-major
-// row, one stride of ncap per entry).  The candidate loop is branch-free
-// apart from the append: loads past the range end repeat the last entry and
-// are masked out with the self pair.  Bit a of M asks for the periodic image
-// test along axis a; an axis left out is one along which no candidate of
-// the wave can need an image.  was = W_A + skin.
-template <bool RODS, int M>
-__device__ __forceinline__ void scan_range(
-    int ua, int ub, int t, const double4 &p, double reach_i,
-    const BoxGeom &g, const double4 *__restrict__ pos,
-    const int32_t *__restrict__ type, const double4 *__restrict__ rod,
-    int mode, double crit, double was, int32_t *&out, int64_t ncap,
-    int32_t maxn, int &cnt) {
-  for (int u0 = ua; u0 < ub; u0++) {
-    double4 o[1];
-    o[0] = pos[u0];
-    {
-      const int j = 0, u = u0;
-      const double d0 = sep_m<M, 0>(p.x, o[j].x, g);
-      const double d1 = sep_m<M, 1>(p.y, o[j].y, g);
-      const double d2 = sep_m<M, 2>(p.z, o[j].z, g);
-      double r2 = d0 * d0 + d1 * d1 + d2 * d2;
-      bool ok;
-      if (mode == 1) {
-        ok = r2 <= crit;  // BMXCheckPair (src/des/bmx_pc.H:76)
-      } else {
-        double rj = RODS ? reach_of<true>(o[j], type[min(u, ub - 1)], rod,
-                                          min(u, ub - 1))
-                         : o[j].w;
-        double cut = reach_i + rj + was;
-        ok = r2 <= cut * cut;
-      }
-      if (ok && u < ub && u != t) {
-        if (cnt < maxn) {
-          *out = u;
-          out += ncap;
-        }
-        cnt++;
-      }
-    }
-  }
-}
-
-
 // A particle's bin stencil as memory ranges of the sorted arrays, in the
 // canonical order (oz, then oy, then ox).  Each (oz, oy) row of bins is one
 // or two ranges: the x window [bx - 1, bx + 1] is contiguous in memory
@@ -719,127 +675,6 @@ __device__ __forceinline__ int2 stencil_range(const Stencil st, int k,
   return make_int2(start[row + xa], start[row + xb]);
 }
 
-// Where a sphere build puts a particle's row while it grows: the first
-// kStage entries in LDS (entry k at stage[k * stride], one word per thread
-// and entry, so the lanes of a wave write neighbouring banks), the rest in
-// the column-major row (entry k at col[k * ncap]).  With cols, every entry
-// also goes to the column-major row, for the passes that read rows that way
-// (exchange, fusion).  The flat rows are copied from here at the end.
-constexpr int kStage = 8;
-struct RowSink {
-  int32_t *stage;
-  int stride;
-  int32_t *col;
-  int64_t ncap;
-  int cols;
-};
-__device__ __forceinline__ void row_put(const RowSink &sk, int k, int32_t u) {
-  if (k < kStage) {
-    sk.stage[k * sk.stride] = u;
-    if (sk.cols) sk.col[(int64_t)k * sk.ncap] = u;
-  } else {
-    sk.col[(int64_t)k * sk.ncap] = u;
-  }
-}
-__device__ __forceinline__ int32_t row_get(const RowSink &sk, int k) {
-  return k < kStage ? sk.stage[k * sk.stride] : sk.col[(int64_t)k * sk.ncap];
-}
-
-// Scans a particle's stencil as one sequence of candidates and appends the
-// accepted ones to its row (through the row sink).  Each lane moves on to its
-// next range as soon as its current one ends, so a wave takes as many
-// iterations as its longest stencil rather than the sum over ranges of the
-// longest range; the next range's bounds are loaded one range ahead.  An
-// iteration tests NC candidates of the range: two for one box (three or
-// four spill at 64 VGPRs), one for several boxes (two spill there).
-// Candidates visited are capped at scan_cap per particle (a range
-// that would pass it is dropped and the row reported as overflowing).  Bit
-// a of M asks for the periodic image
-// test along axis a; an axis left out is one along which no candidate of
-// the wave can need an image.  CRIT: the stencil policy's test of the
-// squared distance against crit; otherwise the Verlet test against the
-// reaches plus was = W_A + skin (a sphere's reach is its radius).
-template <int M, bool CRIT, int NC>
-__device__ __forceinline__ void scan_stencil(
-    const Stencil sc, const BoxGeom &g, const int32_t *__restrict__ start,
-    int64_t scan_cap, int t, const double4 &p,
-    const double4 *__restrict__ pos, double crit, double was,
-    const RowSink &sk, int32_t maxn, int &cnt) {
-  const int nq = 9 << sc.two;
-  // 32-bit count of the candidates taken; once a range would pass the cap,
-  // it and every later range are dropped (scanned sticks above the cap)
-  const int cap = scan_cap < (1 << 30) ? (int)scan_cap : (1 << 30);
-  int scanned = 0;
-  int q = 0;
-  const int2 first = stencil_range(sc, 0, start);
-  int2 next = stencil_range(sc, 1, start);
-  int u = first.x, e = first.y;
-  if (e - u > cap) {
-    cnt = maxn + 1;
-    e = u;
-    scanned = cap + 1;
-  } else {
-    scanned = e - u;
-  }
-  for (;;) {
-    while (u >= e && q + 1 < nq) {
-      q++;
-      u = next.x;
-      e = next.y;
-      const int len = e - u;
-      if (len > cap - scanned) {
-        cnt = maxn + 1;  // reported as overflow
-        e = u;
-        scanned = cap + 1;
-      } else {
-        scanned += len;
-      }
-      if (q + 1 < nq) next = stencil_range(sc, q + 1, start);
-    }
-    if (u >= e) break;
-    // NC = 2: two candidates of the range per iteration (the second only
-    // when the range holds it), appended in order
-    const bool two = NC == 2 && u + 1 < e;
-    const int u1 = two ? u + 1 : u;
-    const double4 o = pos[u];
-    bool ok, ok1 = false;
-    {
-      const double d0 = sep_m<M, 0>(p.x, o.x, g);
-      const double d1 = sep_m<M, 1>(p.y, o.y, g);
-      const double d2 = sep_m<M, 2>(p.z, o.z, g);
-      const double r2 = d0 * d0 + d1 * d1 + d2 * d2;
-      if (CRIT) {
-        ok = r2 <= crit;  // BMXCheckPair (src/des/bmx_pc.H:76)
-      } else {
-        const double cut = p.w + o.w + was;
-        ok = r2 <= cut * cut;
-      }
-    }
-    if (NC == 2) {
-      const double4 o1 = pos[u1];
-      const double d0 = sep_m<M, 0>(p.x, o1.x, g);
-      const double d1 = sep_m<M, 1>(p.y, o1.y, g);
-      const double d2 = sep_m<M, 2>(p.z, o1.z, g);
-      const double r2 = d0 * d0 + d1 * d1 + d2 * d2;
-      if (CRIT) {
-        ok1 = r2 <= crit;
-      } else {
-        const double cut = p.w + o1.w + was;
-        ok1 = r2 <= cut * cut;
-      }
-    }
-    if (ok && u != t) {
-      if (cnt < maxn) row_put(sk, cnt, u);
-      cnt++;
-    }
-    if (two && ok1 && u1 != t) {
-      if (cnt < maxn) row_put(sk, cnt, u1);
-      cnt++;
-    }
-    u += two ? 2 : 1;
-  }
-}
-
 // Bits 28..30 of a row count mark the axes (x, y, z) along which a neighbor
 // of the particle can need a periodic image before the next rebuild: the
 // axis is periodic and the particle's bin is within two bins of a face (or
@@ -856,8 +691,39 @@ __device__ __forceinline__ int wave_or3(int m) {
 }
 
 
-template <bool MULTI, bool RODS>
-__global__ __launch_bounds__(512, 8) void k_build_nbr(
+// Axes (bits) along which a candidate of a list build over the +-1 stencil of
+// bin b3 (scan) or a neighbor before the next rebuild (force) can need a
+// periodic image.
+__device__ __forceinline__ void image_axes(const int b3[3], const BoxGeom &g,
+                                           int &scan_img, int &force_img) {
+#pragma unroll
+  for (int a = 0; a < 3; a++) {
+    if (!g.periodic[a]) continue;
+    const int nb = g.nbin[a];
+    if (!(nb >= 4 && b3[a] >= 1 && b3[a] + 1 < nb)) scan_img |= 1 << a;
+    if (!(nb >= 6 && b3[a] >= 2 && b3[a] + 2 < nb)) force_img |= 1 << a;
+  }
+}
+
+// One block builds the rows of one tile (blockDim.x / G particles), G lanes
+// to a particle.  The lanes of a group load the bounds of the particle's 9
+// (18 next to a periodic x face) stencil ranges at once, leave their running
+// ends in LDS, and then test candidates k = sub, sub + G, ... of the
+// concatenated ranges, kBuildUnroll of them in flight; a ballot gives the
+// accepted ones their places, which keeps the rows in candidate order.
+// Entries past the staged ones pass through global memory (nbr).
+constexpr int kBuildRanges = 18;
+constexpr int kBuildUnroll = 2;
+__host__ __device__ constexpr int build_stage(int tile) {
+  return tile >= 64 ? 9 : (tile >= 32 ? 17 : 33);
+}
+size_t build_lds(int tile) {
+  return (size_t)tile * (sizeof(int2) * kBuildRanges +
+                         sizeof(int32_t) * build_stage(tile));
+}
+
+template <bool MULTI, bool RODS, int G>
+__global__ __launch_bounds__(256, 8) void k_build_rows(
     const double4 *__restrict__ pos, const int32_t *__restrict__ col,
     const int32_t *__restrict__ type, const double4 *__restrict__ rod,
     const BoxGeom *__restrict__ boxes, BoxGeom g0,
@@ -865,175 +731,197 @@ __global__ __launch_bounds__(512, 8) void k_build_nbr(
     int64_t n, int mode, double crit, double wa, double skin,
     int32_t *__restrict__ nbr, int32_t *__restrict__ ncnt, int64_t ncap,
     int32_t maxn, int32_t *__restrict__ err, int32_t *__restrict__ bstats,
-    FlatRows flat, int cols, int remap) {
-  const int64_t t = tile_of(remap) * blockDim.x + threadIdx.x;
-  const int ti = (int)t;  // n < 2^31
+    FlatRows flat, int remap) {
+  extern __shared__ __align__(8) int32_t build_words[];
+  const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
+  const int nwv = blockDim.x / kWave, T = flat.tile;  // T = blockDim.x / G
+  const int place = threadIdx.x / G, sub = threadIdx.x & (G - 1);
+  const int S = build_stage(T);
+  int2 *rng = reinterpret_cast<int2 *>(build_words) + place * kBuildRanges;
+  int32_t *stage = build_words + 2 * kBuildRanges * T + place * S;
+  const int64_t tile = tile_of(remap);
+  const int64_t t = tile * T + place;
   const double was = wa + skin;
-  int32_t *out = nbr + t;
-  // sphere builds stage the first entries of each row in LDS (kStage words
-  // per thread, launched with that much dynamic LDS)
-  extern __shared__ int32_t srow[];
-  const RowSink sk{srow + threadIdx.x, (int)blockDim.x, nbr + t, ncap,
-                   (cols || !flat.cidx) ? 1 : 0};
-  int cnt = 0;
   // Candidates visited per particle are capped (a pile of particles in a few
-  // bins would otherwise make this quadratic); hitting the cap is reported
-  // as an overflow.  After a non-finite force no rows are built.
+  // bins would otherwise make this quadratic): a range that would pass the
+  // cap is dropped with every later one, and the row reported as an
+  // overflow.  After a non-finite force no rows are built.
   const int64_t scan_cap = 64 * (int64_t)maxn + 4096;
+  const int cap = scan_cap < (1 << 30) ? (int)scan_cap : (1 << 30);
   const bool active = t < n && !(*err & ERRBIT_NAN);
+  const int64_t tc = t < n ? t : n - 1;
+  const unsigned long long gmask = ((1ull << G) - 1ull) << (lane & ~(G - 1));
+  const unsigned long long below = (1ull << lane) - 1ull;
+  int cnt = 0;
   // The row build over box g.  Several boxes: a wave whose particles all
   // lie in one box (all but the waves at colony boundaries) reads that box
   // once into scalar registers; the others read each particle's box.
   auto build = [&](const BoxGeom &g) {
-    const int nbx = g.nbin[0], nby = g.nbin[1], nbz = g.nbin[2];
-    int bx = 0, by = 0, bz = 0;
-    double4 p = make_double4(0.0, 0.0, 0.0, 0.0);
-    double reach_i = 0.0;
-    // axes along which a candidate of this list build (scan) or a neighbor
-    // before the next rebuild (force) can need a periodic image
+    const double4 p = pos[tc];
+    const double reach_i = RODS ? reach_of<true>(p, type[tc], rod, tc) : p.w;
+    const int nbx = g.nbin[0], nby = g.nbin[1];
+    const int lb = key[tc] - g.bin_offset;
+    const int rr = lb / nbx;
+    const int b3[3] = {lb % nbx, rr % nby, rr / nby};
     int scan_img = 0, force_img = 0;
-    if (active) {
-      p = pos[t];
-      reach_i = RODS ? reach_of<true>(p, type[t], rod, t) : p.w;
-      int lb = key[t] - g.bin_offset;
-      bx = lb % nbx;
-      int rr = lb / nbx;
-      by = rr % nby;
-      bz = rr / nby;
-      const int b3[3] = {bx, by, bz};
-      for (int a = 0; a < 3; a++) {
-        if (!g.periodic[a]) continue;
-        int nb = g.nbin[a];
-        if (!(nb >= 4 && b3[a] >= 1 && b3[a] + 1 < nb)) scan_img |= 1 << a;
-        if (!(nb >= 6 && b3[a] >= 2 && b3[a] + 2 < nb)) force_img |= 1 << a;
+    image_axes(b3, g, scan_img, force_img);
+    const Stencil sc = make_stencil(b3[0], b3[1], b3[2], g);
+    const int nq = active ? 9 << sc.two : 0;
+    // the ranges' bounds, then rng[r] = (running end, first - begin)
+    int total = 0;
+    bool over = false;
+    auto bounds = [&](auto nb_tag) {
+      constexpr int NB = decltype(nb_tag)::value;
+      int2 se[NB];
+#pragma unroll
+      for (int b = 0; b < NB; b++) {
+        const int r = b * G + sub;
+        se[b] = r < nq ? stencil_range(sc, r, start) : make_int2(0, 0);
       }
-    }
-    const int wave_img = wave_or3(scan_img);
-    if (active) {
-      if (RODS) {
-        // Segment builds (sparse mesh-cell bins): range by range, all lanes
-        // together, which measured faster there than the flattened scan.
-        int64_t scanned = 0;
-        for (int oz = -1; oz <= 1; oz++) {
-          int cz = bz + oz;
-          if (g.periodic[2]) {
-            cz = (cz + nbz) % nbz;
-          } else if (cz < 0 || cz >= nbz) {
-            continue;
-          }
-          for (int oy = -1; oy <= 1; oy++) {
-            int cy = by + oy;
-            if (g.periodic[1]) {
-              cy = (cy + nby) % nby;
-            } else if (cy < 0 || cy >= nby) {
-              continue;
-            }
-            int row = g.bin_offset + (cz * nby + cy) * nbx;
-            // up to three x-ranges; one contiguous range when no x wrap
-            int ranges[3][2];
-            int nr = 0;
-            if (bx >= 1 && bx + 1 < nbx) {
-              ranges[0][0] = start[row + bx - 1];
-              ranges[0][1] = start[row + bx + 2];
-              nr = 1;
-            } else {
-              for (int ox = -1; ox <= 1; ox++) {
-                int cx = bx + ox;
-                if (g.periodic[0]) {
-                  cx = (cx + nbx) % nbx;
-                } else if (cx < 0 || cx >= nbx) {
-                  continue;
-                }
-                ranges[nr][0] = start[row + cx];
-                ranges[nr][1] = start[row + cx + 1];
-                nr++;
-              }
-            }
-            for (int q = 0; q < nr; q++) {
-              int64_t len = ranges[q][1] - ranges[q][0];
-              if (scanned + len > scan_cap) {
-                cnt = maxn + 1;  // reported as overflow below
-                ranges[q][1] = ranges[q][0];
-              }
-              scanned += len;
-              if (wave_img == 0)
-                scan_range<RODS, 0>(ranges[q][0], ranges[q][1], ti, p, reach_i, g,
-                                    pos, type, rod, mode, crit, was, out, ncap,
-                                    maxn, cnt);
-              else if (wave_img == 1)
-                scan_range<RODS, 1>(ranges[q][0], ranges[q][1], ti, p, reach_i, g,
-                                    pos, type, rod, mode, crit, was, out, ncap,
-                                    maxn, cnt);
-              else
-                scan_range<RODS, 7>(ranges[q][0], ranges[q][1], ti, p, reach_i, g,
-                                    pos, type, rod, mode, crit, was, out, ncap,
-                                    maxn, cnt);
-            }
-          }
+      int run = 0;
+#pragma unroll
+      for (int b = 0; b < NB; b++) {
+        const int r = b * G + sub;
+        const int len = se[b].y - se[b].x;
+        int incl = len;
+#pragma unroll
+        for (int o = 1; o < G; o <<= 1) {
+          const int w = __shfl_up(incl, o, G);
+          if (sub >= o) incl += w;
         }
-      } else {
-        const Stencil sc = make_stencil(bx, by, bz, g);
-        auto run = [&](auto crit_tag) {
-          constexpr bool C = decltype(crit_tag)::value;
-          constexpr int NC = MULTI ? 1 : 2;
-          if (wave_img == 0)
-            scan_stencil<0, C, NC>(sc, g, start, scan_cap, ti, p, pos, crit, was, sk,
-                                   maxn, cnt);
-          else if (wave_img == 1)
-            scan_stencil<1, C, NC>(sc, g, start, scan_cap, ti, p, pos, crit, was, sk,
-                                   maxn, cnt);
-          else
-            scan_stencil<7, C, NC>(sc, g, start, scan_cap, ti, p, pos, crit, was, sk,
-                                   maxn, cnt);
-        };
-        if (mode == 1)
-          run(std::true_type{});
-        else
-          run(std::false_type{});
+        const int end = run + incl;
+        if (r < nq) {
+          rng[r] = make_int2(end, se[b].x - (end - len));
+          if (end <= cap) total = end;
+        }
+        run += __shfl(incl, G - 1, G);
       }
-      ncnt[t] = (cnt < maxn ? cnt : maxn) | (force_img << kImgShift);
+      over = run > cap;
+    };
+    if (__any(nq > 9))
+      bounds(std::integral_constant<int, (18 + G - 1) / G>{});
+    else
+      bounds(std::integral_constant<int, (9 + G - 1) / G>{});
+#pragma unroll
+    for (int o = G >> 1; o > 0; o >>= 1) {
+      const int w = __shfl_xor(total, o, G);
+      total = w > total ? w : total;
+    }
+    wave_lds_sync();
+    auto scan = [&](auto m_tag, auto crit_tag) {
+      constexpr int M = decltype(m_tag)::value;
+      constexpr bool CRIT = decltype(crit_tag)::value;
+      int r = 0;
+      int2 cur = rng[0];
+      for (int k0 = sub; __any(k0 < total); k0 += kBuildUnroll * G) {
+        int u[kBuildUnroll];
+        bool ok[kBuildUnroll];
+        double4 o[kBuildUnroll];
+        double rj[kBuildUnroll];
+#pragma unroll
+        for (int j = 0; j < kBuildUnroll; j++) {
+          const int k = k0 + j * G;
+          ok[j] = k < total;
+          while (ok[j] && k >= cur.x) cur = rng[++r];
+          u[j] = ok[j] ? k + cur.y : (int)tc;
+          o[j] = pos[u[j]];
+          if (!CRIT) rj[j] = RODS ? reach_of<true>(o[j], type[u[j]], rod, u[j]) : o[j].w;
+        }
+#pragma unroll
+        for (int j = 0; j < kBuildUnroll; j++) {
+          const double d0 = sep_m<M, 0>(p.x, o[j].x, g);
+          const double d1 = sep_m<M, 1>(p.y, o[j].y, g);
+          const double d2 = sep_m<M, 2>(p.z, o[j].z, g);
+          const double r2 = d0 * d0 + d1 * d1 + d2 * d2;
+          bool in;
+          if (CRIT) {
+            in = r2 <= crit;  // BMXCheckPair (src/des/bmx_pc.H:76)
+          } else {
+            const double cut = reach_i + rj[j] + was;
+            in = r2 <= cut * cut;
+          }
+          in = in && ok[j] && u[j] != (int)t;
+          const unsigned long long m = __ballot(in) & gmask;
+          const int k = cnt + __popcll(m & below);
+          if (in && k < maxn) {
+            if (k < S)
+              stage[k] = u[j];
+            else
+              nbr[tc + (int64_t)k * ncap] = u[j];
+          }
+          cnt += __popcll(m);
+        }
+      }
+    };
+    const bool img = wave_or3(active ? scan_img : 0) != 0;
+    auto run = [&](auto crit_tag) {
+      if (img)
+        scan(std::integral_constant<int, 7>{}, crit_tag);
+      else
+        scan(std::integral_constant<int, 0>{}, crit_tag);
+    };
+    if (mode == 1)
+      run(std::true_type{});
+    else
+      run(std::false_type{});
+    if (over && cnt <= maxn) cnt = maxn + 1;  // reported as an overflow
+    if (sub == 0 && t < n) {
+      ncnt[t] = active ? (cnt < maxn ? cnt : maxn) | (force_img << kImgShift) : 0;
       if (cnt > maxn) atomicOr(err, ERRBIT_OVERFLOW);
-    } else if (t < n) {
-      ncnt[t] = 0;
     }
   };
   if (MULTI) {
-    const int32_t cl = col[t < n ? t : n - 1];
+    const int32_t cl = col[tc];
     const int cw = __builtin_amdgcn_readfirstlane(cl);
     if (__all(t >= n || cl == cw)) {
       const BoxGeom gw = boxes[cw];
       build(gw);
     } else {
-      build(boxes[active ? col[t] : 0]);
+      build(boxes[cl]);
     }
   } else {
     build(g0);
   }
-  if (flat.cidx) {
-    // Flat row layout: the tile's rows back to back from the start of the
-    // tile's own region (tile * maxn entries per tile).
-    const int tile = flat.tile, place = threadIdx.x & (tile - 1);
-    const int kept = cnt < maxn ? cnt : maxn;
-    const int incl = wave_incl_scan(kept, tile);
-    const int tot = __shfl(incl, tile - 1, tile);
-    if (place == 0 && t < n) flat.tot[t / tile] = tot;
-    const int64_t b = (t / tile) * (int64_t)tile * maxn + (incl - kept);
-    for (int k = 0; k < kept; k++) {
-      flat.cidx[b + k] = RODS ? nbr[t + (int64_t)k * ncap] : row_get(sk, k);
-      flat.cown[b + k] = (uint8_t)place;
-    }
+  // the rows back to back: offsets over the tile's particles, wave totals
+  // through LDS, with the row statistics
+  __shared__ int32_t wsum[256 / kWave], wmax[256 / kWave], wall[256 / kWave];
+  const int kept = cnt < maxn ? cnt : maxn;
+  int incl = wave_incl_scan64(sub == 0 ? kept : 0);
+  int all = incl;
+  if (__any(cnt > kept)) all = wave_incl_scan64(sub == 0 ? cnt : 0);
+  int mx = cnt;
+#pragma unroll
+  for (int o = kWave / 2; o >= G; o >>= 1) {
+    const int w = __shfl_xor(mx, o, kWave);
+    mx = w > mx ? w : mx;
   }
-  __shared__ int32_t shi[16];
-  int m = block_max(cnt, shi);
+  if (lane == kWave - 1) {
+    wsum[wv] = incl;
+    wmax[wv] = mx;
+    wall[wv] = all;
+  }
+  // (also orders the staged entries, and those in global memory, before
+  // other lanes read them)
   __syncthreads();
-  int sm = block_sum(cnt, shi);
+  for (int w = 0; w < wv; w++) incl += wsum[w];
   if (threadIdx.x == 0) {
+    int tot = wsum[0], m = wmax[0], a = wall[0];
+    for (int w = 1; w < nwv; w++) {
+      tot += wsum[w];
+      m = wmax[w] > m ? wmax[w] : m;
+      a += wall[w];
+    }
+    flat.tot[tile] = tot;
     bstats[2 * blockIdx.x] = m;
-    bstats[2 * blockIdx.x + 1] = sm;
+    bstats[2 * blockIdx.x + 1] = a;
+  }
+  if (sub == 0 && t < n) flat.roff[t] = incl - kept;
+  const int64_t b = tile * (int64_t)T * maxn + (incl - kept);
+  for (int k = sub; k < kept; k += G) {
+    flat.cidx[b + k] = k < S ? stage[k] : nbr[tc + (int64_t)k * ncap];
+    flat.cown[b + k] = (uint8_t)place;
   }
 }
-
-
 
 // Reduces the per-block row statistics of the last build.
 __global__ __launch_bounds__(1024) void k_reduce_rowstats(
@@ -1059,13 +947,6 @@ __global__ __launch_bounds__(1024) void k_reduce_rowstats(
 
 // ------------------------------------------------------- force + update ---
 
-// Largest step displacement dt*|vel| of the block, one store per block.
-__device__ __forceinline__ void block_vmax(double v2, double dt, double *vpart) {
-  __shared__ double shd[16];
-  double m = block_max(v2, shd);
-  if (threadIdx.x == 0) vpart[blockIdx.x] = dt * sqrt(m);
-}
-
 // Separation of two spheres along the axes, with the image test of sep_m.
 template <int M>
 __device__ __forceinline__ void sphere_sep(const double4 &p, const double4 &o,
@@ -1080,8 +961,9 @@ __device__ __forceinline__ void sphere_sep(const double4 &p, const double4 &o,
 //
 // The sphere step (force lambda PCI:170-279 with the sphere law K.H:243-276
 // and the wall K.H:1009-1030, then the update PCI:311-449) over the flat row
-// layout.  Lane l of a wave takes list entries l and l + 64 of each window
-// of 128: it loads the neighbor index and its owner lane, gathers the
+// layout, one tile (64 particles or fewer, see flat_tile) per wave; lanes
+// below the tile size own a particle.  Lane l takes list entries l and l + 64
+// of each window of 128: it loads the neighbor index and its owner lane, gathers the
 // neighbor, reads the owner's position from LDS and applies the interaction
 // test (K.H:23-40 with PCI:212).  Interacting pairs are packed into LDS
 // slots by ballot, entry 0 of every lane first, so slot order is entry
@@ -1094,14 +976,13 @@ constexpr size_t kFlatWaveBytes =
     kWave * sizeof(double4) + 4 * kFlatWin * sizeof(double);
 
 // Largest step displacement dt*|vel| of the wave, one store per wave at its
-// wave index (the partial arrays hold one slot per 64 particles), with no
-// block barrier: waves that finish early do not wait for the block's
-// slowest.  (One atomic maximum per wave into a few shared words instead
+// tile's index (the partial arrays hold one entry per tile), with no block
+// barrier: waves that finish early do not wait for the block's slowest.  (One atomic maximum per wave into a few shared words instead
 // measured 2.4 times slower on the 1M-sphere step: the atomics serialize.)
 __device__ __forceinline__ void wave_vmax(double v2, double dt, double *vpart,
-                                          int64_t t, int lane, int64_t n) {
+                                          int64_t tile, int lane, bool live) {
   const double m = wave_max_f64(v2);
-  if (lane == 0 && t < n) vpart[t / kWave] = dt * sqrt(m);
+  if (lane == 0 && live) vpart[tile] = dt * sqrt(m);
 }
 
 
@@ -1195,7 +1076,7 @@ __global__ __launch_bounds__(512, 6) void k_force_sphere_flat(
     const double4 *__restrict__ pos_in, double4 *__restrict__ pos_out,
     const int32_t *__restrict__ cidx, const uint8_t *__restrict__ cown,
     const int32_t *__restrict__ wtot, const int32_t *__restrict__ ncnt,
-    int64_t n, int32_t maxn, const int32_t *__restrict__ col,
+    int64_t n, int tsize, int32_t maxn, const int32_t *__restrict__ col,
     const BoxGeom *__restrict__ boxes, BoxGeom g0, ForceParams fp,
     double *__restrict__ fc, const int32_t *__restrict__ fc_oid,
     double *__restrict__ vmax, int32_t *__restrict__ err, int remap) {
@@ -1208,9 +1089,10 @@ __global__ __launch_bounds__(512, 6) void k_force_sphere_flat(
   double *q1s = q0s + kFlatWin, *q2s = q1s + kFlatWin, *qrs = q2s + kFlatWin;
   int32_t *scol = reinterpret_cast<int32_t *>(flat_lds + nwv * kFlatWaveBytes) +
                   wv * kWave;
-  const int64_t t = tile_of(remap) * blockDim.x + threadIdx.x;
-  const bool active = t < n;
-  // The wave's entries start at its region (64 * maxn entries per wave).
+  const int64_t tile = tile_of(remap) * nwv + wv;
+  const int64_t t0 = tile * tsize, t = t0 + lane;
+  const bool active = lane < tsize && t < n;
+  // The wave's entries start at its tile's region (tsize * maxn entries).
   // Every load that does not depend on another is issued here, before
   // anything waits, from indexes valid for every lane (the last particle
   // for lanes past n, tile 0 for a wave past n): the row length, the wave's
@@ -1218,11 +1100,11 @@ __global__ __launch_bounds__(512, 6) void k_force_sphere_flat(
   // tile's region, and the padding after the last one, is always
   // readable).  The one-box path takes the first window from these; the
   // per-entry-box path, which would spill with them live, reloads it.
-  const bool live = t - lane < n;  // the wave holds at least one particle
-  const int64_t B = live ? (t / kWave) * (int64_t)kWave * maxn : 0;
+  const bool live = t0 < n;  // the tile holds at least one particle
+  const int64_t B = live ? t0 * maxn : 0;
   const int64_t tc = active ? t : n - 1;
   const int32_t raw_l = ncnt[tc];
-  const int32_t T_l = wtot[live ? t / kWave : 0];
+  const int32_t T_l = wtot[live ? tile : 0];
   const double4 p_l = pos_in[tc];
   const int32_t col_l = MULTI ? col[tc] : 0;
   const int f0u = cidx[B + lane], f1u = cidx[B + kWave + lane];
@@ -1294,27 +1176,26 @@ __global__ __launch_bounds__(512, 6) void k_force_sphere_flat(
     if (!(isfinite(a0) && isfinite(a1) && isfinite(a2))) atomicOr(err, ERRBIT_NAN);
     v2 = vx * vx + vy * vy + vz * vz;
   }
-  if (vmax) wave_vmax(v2, fp.dt, vmax, t, lane, n);
+  if (vmax) wave_vmax(v2, fp.dt, vmax, tile, lane, live);
 }
 
-// Serial pass over one particle's column-major row (the reference's
-// per-particle neighbor loop): sphere pairs for yeast, segment pairs for
+// Serial pass over one particle's row (the reference's per-particle
+// neighbor loop): sphere pairs for yeast, segment pairs for
 // hyphae, summed into acc in row order; ti is the particle's evolving
 // record (rod_pair_i may repair a bond or promote a second segment).
 template <bool MULTI>
 __device__ void general_rows(int64_t t, const BoxGeom &g, const DynArrays &in,
-                             const StaticArrays &st,
-                             const int32_t *__restrict__ nbr,
-                             const int32_t *__restrict__ ncnt, int64_t ncap,
+                             const StaticArrays &st, const FlatRows &flat,
+                             int32_t maxn, const int32_t *__restrict__ ncnt,
                              const ForceParams &fp, double acc[6], Topo &ti) {
   const int ty = st.type[t];
   const double4 p = in.pos[t];
   const double4 rod_i = in.rod[t];
   const int c = row_len(ncnt[t]);
-  const int32_t *row = nbr + t;
+  const int32_t *row = flat.cidx + row_base(flat, maxn, t);
   if (ty == rec::YEAST) {
     for (int k = 0; k < c; k++) {
-      int u = row[(int64_t)k * ncap];
+      int u = row[k];
       if (st.type[u] != rec::YEAST) continue;  // r_lm = 0 (K.H:39)
       double4 o = in.pos[u];
       double d0 = sep_axis(p.x, o.x, g.L[0], g.halfL[0], g.periodic[0]);
@@ -1330,7 +1211,7 @@ __device__ void general_rows(int64_t t, const BoxGeom &g, const DynArrays &in,
     RodSelf S;
     rod_self_init(S, rod_i, in.trig[t], p.w, st.bscale[t], fp.visc);
     for (int k = 0; k < c; k++) {
-      int u = row[(int64_t)k * ncap];
+      int u = row[k];
       if (st.type[u] != rec::FUNGI) continue;
       double4 o = in.pos[u];
       double4 rod_j = in.rod[u];
@@ -1411,12 +1292,12 @@ __device__ double general_finish(int64_t t, const BoxGeom &g,
 
 // ------------------------------------------------ flat general force ---
 //
-// Segments (and mixed colonies) over the flat row layout with tiles of
-// kGTile particles, one tile per wave.  Per window of 128 entries a light
+// Segments (and mixed colonies) over the flat row layout with tiles of at
+// most kGTile particles, one tile per wave.  Per window of 128 entries a light
 // pass (neighbor position, length and type) applies the interaction test;
 // the interacting entries are packed by ballot, in entry order, and only
 // they load the heavy data and run the pair law (rod_pair_i, sphere_pair),
-// each term into its LDS slot.  The tile's particles (lanes 0..kGTile-1)
+// each term into its LDS slot.  The tile's particles (the first lanes)
 // then add their runs of terms in row order.  The pair law is evaluated
 // with the particle's record as it stands before its row; that is what the
 // row loop sees unless an earlier pair of the row repaired a bond.  A tile
@@ -1463,7 +1344,7 @@ __global__ __launch_bounds__(256, 4) void k_force_general_flat(
     DynArrays in, DynArrays out, StaticArrays st,
     const int32_t *__restrict__ cidx, const uint8_t *__restrict__ cown,
     const int32_t *__restrict__ wtot, int8_t *__restrict__ redo_tile,
-    const int32_t *__restrict__ ncnt, int64_t n, int32_t maxn,
+    const int32_t *__restrict__ ncnt, int64_t n, int tsize, int32_t maxn,
     const BoxGeom *__restrict__ boxes, BoxGeom g0,
     ForceParams fp, double *__restrict__ fc, double *__restrict__ vmax,
     int32_t *__restrict__ err, int remap) {
@@ -1476,13 +1357,13 @@ __global__ __launch_bounds__(256, 4) void k_force_general_flat(
   int32_t *po = pu + kGWin;
   int32_t *pf = po + kGWin;
   const int64_t tile = tile_of(remap) * nwv + wv;
-  const int64_t t0 = tile * kGTile;
+  const int64_t t0 = tile * tsize;
   const int64_t t = t0 + lane;
-  const bool active = lane < kGTile && t < n;
+  const bool active = lane < tsize && t < n;
   int64_t B = 0;
   int T = 0;
   if (t0 < n) {
-    B = tile * (int64_t)kGTile * maxn;
+    B = t0 * maxn;
     T = wtot[tile];
   }
   const int c = active ? row_len(ncnt[t]) : 0;
@@ -1603,7 +1484,7 @@ __global__ __launch_bounds__(256, 4) void k_force_general_flat(
     }
     v2 = general_finish(t, g, in, out, st, fp, acc, ti, fc, err);
   }
-  if (vmax) block_vmax(v2, fp.dt, vmax);
+  if (vmax) wave_vmax(v2, fp.dt, vmax, tile, lane, t0 < n);
 }
 
 // The row loop for the particles of the tiles that the flat pass marked
@@ -1613,17 +1494,17 @@ __global__ __launch_bounds__(256, 4) void k_force_general_flat(
 template <bool MULTI>
 __global__ __launch_bounds__(256) void k_force_general_redo(
     DynArrays in, DynArrays out, StaticArrays st,
-    const int8_t *__restrict__ redo_tile, const int32_t *__restrict__ nbr,
-    const int32_t *__restrict__ ncnt, int64_t ncap, int64_t n,
+    const int8_t *__restrict__ redo_tile, FlatRows flat, int32_t maxn,
+    const int32_t *__restrict__ ncnt, int64_t n,
     const BoxGeom *__restrict__ boxes, BoxGeom g0, ForceParams fp,
     double *__restrict__ fc, double *__restrict__ vmax,
     int32_t *__restrict__ err) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n || !redo_tile[t / kGTile]) return;
+  if (t >= n || !redo_tile[t / flat.tile]) return;
   const BoxGeom &g = MULTI ? boxes[st.col[t]] : g0;
   Topo ti = in.topo[t];
   double acc[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-  general_rows<MULTI>(t, g, in, st, nbr, ncnt, ncap, fp, acc, ti);
+  general_rows<MULTI>(t, g, in, st, flat, maxn, ncnt, fp, acc, ti);
   const double v2 = general_finish(t, g, in, out, st, fp, acc, ti, fc, err);
   if (vmax)
     atomicMax(reinterpret_cast<unsigned long long *>(vmax), dbits(fp.dt * sqrt(v2)));
@@ -1632,9 +1513,8 @@ __global__ __launch_bounds__(256) void k_force_general_redo(
 // InitBonds: per segment, scan the row in order and append a bond for the
 // first site pair closer than rlim (K.H:1285-1444 with rlim = 1e-7, PCI:508).
 template <bool MULTI>
-__global__ void k_init_bonds(DynArrays dy, StaticArrays st,
-                             const int32_t *__restrict__ nbr,
-                             const int32_t *__restrict__ ncnt, int64_t ncap,
+__global__ void k_init_bonds(DynArrays dy, StaticArrays st, FlatRows flat,
+                             int32_t maxn, const int32_t *__restrict__ ncnt,
                              int64_t n, const BoxGeom *__restrict__ boxes,
                              BoxGeom g0, ForceParams fp,
                              int32_t *__restrict__ err) {
@@ -1649,8 +1529,9 @@ __global__ void k_init_bonds(DynArrays dy, StaticArrays st,
   double nxi = tr.y * tr.z, nyi = tr.y * tr.w, nzi = tr.x;
   Topo ti = dy.topo[t];
   int c = row_len(ncnt[t]);
+  const int32_t *row = flat.cidx + row_base(flat, maxn, t);
   for (int k = 0; k < c; k++) {
-    int u = nbr[(int64_t)k * ncap + t];
+    int u = row[k];
     if (st.type[u] != rec::FUNGI) continue;
     double4 o = dy.pos[u];
     double4 rod_j = dy.rod[u];
@@ -1782,8 +1663,7 @@ __global__ void k_export_counts(const int32_t *__restrict__ ncnt,
   if (t >= n) return;
   out[oid[t]] = row_len(ncnt[t]);
 }
-// Rows from the flat layout: particle t's row starts after the rows of the
-// particles before it in its tile.
+// Rows from the flat layout, in original order.
 __global__ void k_export_nbr(FlatRows flat, int32_t maxn,
                              const int32_t *__restrict__ ncnt,
                              const int32_t *__restrict__ oid, int64_t n,
@@ -1791,9 +1671,7 @@ __global__ void k_export_nbr(FlatRows flat, int32_t maxn,
                              int32_t *__restrict__ out) {
   int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= n) return;
-  const int64_t t0 = t / flat.tile * flat.tile;
-  int64_t b = t0 * maxn;
-  for (int64_t u = t0; u < t; u++) b += row_len(ncnt[u]);
+  const int64_t b = row_base(flat, maxn, t);
   int64_t base = row_off[oid[t]];
   int c = row_len(ncnt[t]);
   for (int k = 0; k < c; k++) out[base + k] = oid[flat.cidx[b + k]];
@@ -1899,6 +1777,30 @@ hipError_t launch_sort_gather(const unsigned long long *permk,
   return hipGetLastError();
 }
 
+int32_t tile_count(int64_t n, int tile) { return grid_for(n, tile); }
+
+namespace {
+// blocks of a force launch, one wave per tile
+int force_blocks(int64_t n, int tile, int block) {
+  return grid_for(tile_count(n, tile), block / kWave);
+}
+// Lanes per particle of the row build.  More lanes shorten each particle's
+// chain of dependent loads, until the waves they make no longer fit the chip
+// at once.  Whole rebuilds, in us, 1.1-entry sphere rows unless said:
+//   n = 2,000:   16 lanes 29.6, 8 lanes 30.3, 4 lanes 32.0, 2 lanes 36.9
+//   24,000:      33.7, 32.8, 34.1, 37.7     (one lane per particle: 55)
+//   120,000:     8 lanes 49.5, 4 lanes 45.1, 2 lanes 46.1 (one lane: 58)
+//   300,000:     4 lanes 65.4, 2 lanes 67.2 (one lane: 68)
+//   1,000,000:   4 lanes 149.6, 2 lanes 139.1 (one lane: 146.8)
+//   segments, stencil rows, 20,000: 8 lanes 27.7, 4 lanes 29.8;
+//   200,000: 8 lanes 61.8, 4 lanes 55.8, 2 lanes 61.0
+// A block is one tile of at most 256 threads and at least one wave.
+int build_lanes(int tile, int64_t n) {
+  const int g = n > 400000 ? 2 : (n > 60000 ? 4 : (n > 8000 ? 8 : 16));
+  return std::min(std::max(g, kWave / tile), 256 / tile);
+}
+}  // namespace
+
 hipError_t launch_build_nbr(const double4 *pos, const int32_t *col,
                             const int32_t *type, const double4 *rod,
                             const BoxGeom *boxes, BoxGeom g0, int multi,
@@ -1906,29 +1808,39 @@ hipError_t launch_build_nbr(const double4 *pos, const int32_t *col,
                             int64_t n, int mode, double crit, double wa,
                             double skin, int32_t *nbr, int32_t *ncnt,
                             int64_t ncap, int32_t maxn, int32_t *err,
-                            int32_t *bstats, FlatRows flat, int cols,
-                            LaunchShape ls, hipStream_t s) {
+                            int32_t *bstats, FlatRows flat, int remap,
+                            hipStream_t s) {
   if (n <= 0) return hipSuccess;
-  int b = ls.block;
-  const size_t stage = rods ? 0 : sizeof(int32_t) * kStage * (size_t)b;
-#define BMX_BUILD(M, RD)                                                      \
-  hipLaunchKernelGGL((k_build_nbr<M, RD>), dim3(grid_for(n, b)), dim3(b),     \
-                     stage, s, pos, col, type, rod, boxes, g0, start, key, n, \
-                     mode, crit, wa, skin, nbr, ncnt, ncap, maxn, err, bstats, \
-                     flat, cols, ls.remap)
+  const int G = build_lanes(flat.tile, n);
+#define BMX_BUILD(M, RD, G_)                                                  \
+  hipLaunchKernelGGL((k_build_rows<M, RD, G_>), dim3(tile_count(n, flat.tile)), \
+                     dim3(flat.tile * G_), build_lds(flat.tile), s, pos, col, \
+                     type, rod, boxes, g0, start, key, n, mode, crit, wa,     \
+                     skin, nbr, ncnt, ncap, maxn, err, bstats, flat, remap)
+#define BMX_BUILD_G(M, RD)                                                    \
+  do {                                                                        \
+    if (G == 2)                                                               \
+      BMX_BUILD(M, RD, 2);                                                    \
+    else if (G == 4)                                                          \
+      BMX_BUILD(M, RD, 4);                                                    \
+    else if (G == 8)                                                          \
+      BMX_BUILD(M, RD, 8);                                                    \
+    else                                                                      \
+      BMX_BUILD(M, RD, 16);                                                   \
+  } while (0)
   if (multi && rods)
-    BMX_BUILD(true, true);
+    BMX_BUILD_G(true, true);
   else if (multi)
-    BMX_BUILD(true, false);
+    BMX_BUILD_G(true, false);
   else if (rods)
-    BMX_BUILD(false, true);
+    BMX_BUILD_G(false, true);
   else
-    BMX_BUILD(false, false);
+    BMX_BUILD_G(false, false);
+#undef BMX_BUILD_G
 #undef BMX_BUILD
   return hipGetLastError();
 }
 
-int32_t row_blocks(int64_t n, int block) { return grid_for(n, block); }
 
 // The tail of a call in one launch: the row statistics of the last build
 // (nblk > 0), then the error word (OR-ed in: calls enqueued back to back
@@ -1990,7 +1902,7 @@ size_t flat_lds_bytes(int block, int multi) {
 hipError_t launch_force_sphere_flat(const double4 *pos_in, double4 *pos_out,
                                     const int32_t *cidx, const uint8_t *cown,
                                     const int32_t *wtot, const int32_t *ncnt,
-                                    int64_t n, int32_t maxn,
+                                    int64_t n, int tile, int32_t maxn,
                                     const int32_t *col,
                                     const BoxGeom *boxes, BoxGeom g0, int multi,
                                     ForceParams fp, double *fc,
@@ -2000,65 +1912,88 @@ hipError_t launch_force_sphere_flat(const double4 *pos_in, double4 *pos_out,
   if (n <= 0) return hipSuccess;
   const int b = ls.block;
   const size_t lds = flat_lds_bytes(b, multi);
+  const int grid = force_blocks(n, tile, b);
   if (multi)
-    hipLaunchKernelGGL(k_force_sphere_flat<true>, dim3(grid_for(n, b)), dim3(b),
-                       lds, s, pos_in, pos_out, cidx, cown, wtot, ncnt, n, maxn,
+    hipLaunchKernelGGL(k_force_sphere_flat<true>, dim3(grid), dim3(b), lds, s,
+                       pos_in, pos_out, cidx, cown, wtot, ncnt, n, tile, maxn,
                        col, boxes, g0, fp, fc, fc_oid, vmax, err, ls.remap);
   else
-    hipLaunchKernelGGL(k_force_sphere_flat<false>, dim3(grid_for(n, b)), dim3(b),
-                       lds, s, pos_in, pos_out, cidx, cown, wtot, ncnt, n, maxn,
+    hipLaunchKernelGGL(k_force_sphere_flat<false>, dim3(grid), dim3(b), lds, s,
+                       pos_in, pos_out, cidx, cown, wtot, ncnt, n, tile, maxn,
                        col, boxes, g0, fp, fc, fc_oid, vmax, err, ls.remap);
   return hipGetLastError();
 }
 
 hipError_t launch_force_general(DynArrays in, DynArrays out, StaticArrays st,
-                                const int32_t *cidx, const uint8_t *cown,
-                                const int32_t *wtot, int8_t *redo_tile,
-                                const int32_t *nbr, const int32_t *ncnt,
-                                int64_t ncap, int64_t n, int32_t maxn,
+                                FlatRows flat, int8_t *redo_tile,
+                                const int32_t *ncnt, int64_t n, int32_t maxn,
                                 const BoxGeom *boxes, BoxGeom g0, int multi,
                                 ForceParams fp, double *fc, double *vmax,
                                 int32_t *err, LaunchShape ls, hipStream_t s) {
   if (n <= 0) return hipSuccess;
   const int b = ls.block > 256 ? 256 : ls.block;
-  const int64_t tiles = (n + kGTile - 1) / kGTile;
-  const int grid = grid_for(tiles, b / kWave);
+  const int grid = force_blocks(n, flat.tile, b);
   const size_t lds = (size_t)(b / kWave) * kGenWaveBytes;
   if (multi) {
     hipLaunchKernelGGL(k_force_general_flat<true>, dim3(grid), dim3(b), lds, s,
-                       in, out, st, cidx, cown, wtot, redo_tile, ncnt, n, maxn,
-                       boxes, g0, fp, fc, vmax, err, ls.remap);
+                       in, out, st, flat.cidx, flat.cown, flat.tot, redo_tile,
+                       ncnt, n, flat.tile, maxn, boxes, g0, fp, fc, vmax, err,
+                       ls.remap);
     hipLaunchKernelGGL(k_force_general_redo<true>, dim3(grid_for(n, 256)),
-                       dim3(256), 0, s, in, out, st, redo_tile, nbr, ncnt,
-                       ncap, n, boxes, g0, fp, fc, vmax, err);
+                       dim3(256), 0, s, in, out, st, redo_tile, flat, maxn,
+                       ncnt, n, boxes, g0, fp, fc, vmax, err);
   } else {
     hipLaunchKernelGGL(k_force_general_flat<false>, dim3(grid), dim3(b), lds, s,
-                       in, out, st, cidx, cown, wtot, redo_tile, ncnt, n, maxn,
-                       boxes, g0, fp, fc, vmax, err, ls.remap);
+                       in, out, st, flat.cidx, flat.cown, flat.tot, redo_tile,
+                       ncnt, n, flat.tile, maxn, boxes, g0, fp, fc, vmax, err,
+                       ls.remap);
     hipLaunchKernelGGL(k_force_general_redo<false>, dim3(grid_for(n, 256)),
-                       dim3(256), 0, s, in, out, st, redo_tile, nbr, ncnt,
-                       ncap, n, boxes, g0, fp, fc, vmax, err);
+                       dim3(256), 0, s, in, out, st, redo_tile, flat, maxn,
+                       ncnt, n, boxes, g0, fp, fc, vmax, err);
   }
   return hipGetLastError();
 }
 
-int flat_tile(int segments) { return segments ? kGTile : kWave; }
+// Particles per tile, one wave per tile of the force pass.  A wave's time
+// grows with the windows of 128 entries its tile holds, and every wave pays
+// its own start and end, so a tile holds about one window, as long as the
+// waves are resident at once (6 per SIMD: 6,144); beyond that, tiles grow
+// until they are few enough or hold four windows, where the share of start
+// and end is small.  Force pass, us, tiles of 64 / 32 / 16 / 8 / 4:
+//   rows of 1:  n = 24,000: 4.2 / 4.4 / 4.8 / 5.3 / 7.1; 1M: 18.7 / 26.7 / 44
+//   rows of 8:  24,000: 11.9 / 8.5 / 7.2 / 6.0 / 7.9;
+//               120,000: 15.3 / 13.6 / 15.0 / 16.1; 1M: 59 / 62 / 74 / 92
+//   rows of 72: 24,000: 57 / 32 / 21 / 15.0 / 14.0; 120,000: 73 / 52 / 45 / 42.5 / 47
+// Segment pairs are far heavier than a wave's start and end (and their rows
+// hold about ten): tiles of 32 / 16 / 8 / 4
+//   2,000: 57 / 40 / 29 / 24; 20,000: 89 / 64 / 49 / 46;
+//   60,000: 96 / 77 / 77 / 90; 200,000: 160 / 157 / 185 / 247
+int flat_tile(int segments, int64_t n, double row) {
+  int t = 4;
+  if (segments) {
+    while (t < 16 && n > (int64_t)t * 5120) t *= 2;
+    return t;
+  }
+  while (t < kWave && 2 * t * row <= kFlatWin) t *= 2;
+  while (t < kWave && n > (int64_t)t * 6144 && t * row < 4 * kFlatWin) t *= 2;
+  return t;
+}
 int64_t flat_entries(int64_t ncap, int tile, int32_t maxn) {
   // + one window: the force pass reads a window before it knows the count
   return (ncap + tile - 1) / tile * (int64_t)tile * maxn + kFlatWin;
 }
 
-hipError_t launch_init_bonds(DynArrays dy, StaticArrays st, const int32_t *nbr,
-                             const int32_t *ncnt, int64_t ncap, int64_t n,
+hipError_t launch_init_bonds(DynArrays dy, StaticArrays st, FlatRows flat,
+                             int32_t maxn, const int32_t *ncnt, int64_t n,
                              const BoxGeom *boxes, BoxGeom g0, int multi,
                              ForceParams fp, int32_t *err, hipStream_t s) {
   if (n <= 0) return hipSuccess;
   if (multi)
     hipLaunchKernelGGL(k_init_bonds<true>, dim3(grid_for(n, 128)), dim3(128),
-                       0, s, dy, st, nbr, ncnt, ncap, n, boxes, g0, fp, err);
+                       0, s, dy, st, flat, maxn, ncnt, n, boxes, g0, fp, err);
   else
     hipLaunchKernelGGL(k_init_bonds<false>, dim3(grid_for(n, 128)), dim3(128),
-                       0, s, dy, st, nbr, ncnt, ncap, n, boxes, g0, fp, err);
+                       0, s, dy, st, flat, maxn, ncnt, n, boxes, g0, fp, err);
   return hipGetLastError();
 }
 

@@ -96,7 +96,8 @@ typedef struct {
 /* Launch shape of the pair kernels (the autotuner's search space).
    A new context uses {64, 1}. */
 typedef struct {
-  int32_t block_size;     /* threads per block: 64, 128, 256, 512 */
+  int32_t block_size;     /* threads per block of the force passes: 64, 128,
+                             256, 512 */
   int32_t xcd_remap;      /* 1: give each of the 8 XCDs a contiguous range
                              of particle tiles */
 } bmx_launch_params;
