@@ -732,14 +732,12 @@ bmx_status drop_chem(bmx_ctx *c) {
 }
 
 bmx_status pack_records(bmx_ctx *c) {
+  // the bin ranks are scratch between rebuilds
   HIPCHK(launch_aos_pack(c->recs, c->lay, c->n, static_arrays(c, c->cs),
-                         dyn_arrays(c, c->cd), c->d_fc.p, c->mobility,
-                         c->wrote_step ? 1 : 0, c->any_fungi ? 1 : 0, c->stream));
-  if (c->have_chem)
-    HIPCHK(launch_chem_pack(c->recs, c->lay, c->n, chem_rel(c),
-                            c->d_chemst[c->cc].p, c->oid[c->cs].p,
-                            c->type[c->cs].p, c->pos[c->cd].p, c->rod[c->cd].p,
-                            c->stream));
+                         dyn_arrays(c, c->cd), c->d_fc.p,
+                         c->have_chem ? c->d_chemst[c->cc].p : nullptr,
+                         chem_rel(c), c->mobility, c->wrote_step ? 1 : 0,
+                         c->any_fungi ? 1 : 0, c->d_rank.p, c->stream));
   return BMX_OK;
 }
 

@@ -55,10 +55,13 @@ hipError_t launch_aos_refresh(const uint8_t *aos, AosLayout lay, int64_t n,
                               const BoxGeom *boxes, StaticArrays st,
                               DynArrays dy, uint32_t fields,
                               unsigned long long *stats, hipStream_t s);
-// sorted SoA -> AoS at original positions (fields the force pass writes)
+// sorted SoA -> AoS (fields the force pass writes; with state, the chemistry
+// state's too, and each particle's radius and length); inv: n words of
+// scratch
 hipError_t launch_aos_pack(uint8_t *aos, AosLayout lay, int64_t n,
                            StaticArrays st, DynArrays dy, const double *fc,
-                           double mob, int wrote_step, int any_fungi,
+                           const double *state, int has_rel, double mob,
+                           int wrote_step, int any_fungi, int32_t *inv,
                            hipStream_t s);
 
 // The displacement check of a Verlet period folded into the first two
