@@ -104,6 +104,7 @@ struct bmx_ctx {
   DevBuf<double> bscale[2];
   DevBuf<double4> pos[2], rod[2], trig[2];
   DevBuf<Topo> topo[2];
+  DevBuf<SegNear> near[2];  // contexts with segments
   int cs = 0;  // current static buffer
   int cd = 0;  // current dynamic buffer
 
@@ -252,6 +253,7 @@ DynArrays dyn_arrays(bmx_ctx *c, int k) {
   d.rod = c->rod[k].p;
   d.trig = c->trig[k].p;
   d.topo = c->topo[k].p;
+  d.near = c->any_fungi ? c->near[k].p : nullptr;
   return d;
 }
 
@@ -579,8 +581,11 @@ bmx_status enqueue_step(bmx_ctx *c, double dt, bool write_fc) {
         multi ? c->col[c->cs].p : nullptr, c->d_boxes.p, c->boxes[0], multi,
         fp, fc, c->oid[c->cs].p, vm, c->d_err.p, shape(c), s));
   } else {
+    // the next step reads what this one leaves only where it keeps the list
+    DynArrays next = dyn_arrays(c, 1 - c->cd);
+    if (c->nbp.rebuild_every == 1) next.near = nullptr;
     HIPCHK(launch_force_general(
-        dyn_arrays(c, c->cd), dyn_arrays(c, 1 - c->cd), static_arrays(c, c->cs),
+        dyn_arrays(c, c->cd), next, static_arrays(c, c->cs),
         flat_rows(c), c->d_redo.p, c->d_ncnt.p, c->n, c->maxn, c->d_boxes.p,
         c->boxes[0], multi, fp, fc, vm, c->d_err.p, shape(c), s));
   }
@@ -868,6 +873,8 @@ bmx_status bind_common(bmx_ctx *c, const void *aos, const int64_t *cstart,
   std::memcpy(&c->lmax, &hs[1], sizeof(double));
   c->any_yeast = hs[2] != 0;
   c->any_fungi = hs[3] != 0;
+  if (c->any_fungi)
+    for (auto &b : c->near) HIPCHK(b.alloc(cap));
   bmx_status bs = setup_boxes(c);
   if (bs != BMX_OK) return bs;
   bs = ensure_rows(c);
@@ -960,6 +967,7 @@ void bmx_ctx_destroy(bmx_ctx *c) {
     c->rod[k].release();
     c->trig[k].release();
     c->topo[k].release();
+    c->near[k].release();
   }
   c->d_boxes.release();
   c->d_col_in.release();
@@ -2745,6 +2753,7 @@ constexpr size_t kNaBytes =
     + 2 * na_align(8 * kNaParticles)             // bscale
     + 2 * 3 * na_align(32 * kNaParticles)        // pos, rod, trig
     + 2 * na_align(sizeof(Topo) * kNaParticles)  // topo
+    + 2 * na_align(sizeof(SegNear) * kNaParticles)  // near
     + 2 * na_align(4 * kNaParticles)             // keytmp, rank
     + na_align(8 * kNaParticles)                 // permk
     + na_align(8 * 6 * kNaParticles)             // fc
@@ -2798,6 +2807,7 @@ bmx_status na_setup(NaDevice &d, int dev) {
     na_slice(c.rod[k], cur, N);
     na_slice(c.trig[k], cur, N);
     na_slice(c.topo[k], cur, N);
+    na_slice(c.near[k], cur, N);
     c.col[k].fixed = true;  // one box: never used
   }
   na_slice(c.d_keytmp, cur, N);

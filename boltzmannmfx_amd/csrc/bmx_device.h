@@ -107,6 +107,110 @@ __device__ __forceinline__ void sphere_pair(double d0, double d1, double d2,
 
 // ---------------------------------------------------------------- rods ----
 
+// bmx_sin and bmx_cos of one angle with one reduction and no branch on the
+// quadrant (lanes of a wave are in all four), and bmx_acos with one series
+// evaluation instead of one per branch: the same operations on the same
+// values, so the same bits.
+__device__ __forceinline__ void sin_cos(double x, double &s, double &c) {
+  int q;
+  const double r = bmx_reduce_pio2(x, &q);
+  const double a = bmx_sin_kernel(r), b = bmx_cos_kernel(r);
+  const double sv = (q & 1) ? b : a, cv = (q & 1) ? a : b;
+  s = (q & 2) ? -sv : sv;
+  c = ((q + 1) & 2) ? -cv : cv;
+}
+__device__ __forceinline__ double acos_of(double x) {
+  if (!(x >= -1.0 && x <= 1.0)) return (x - x) / (x - x); /* NaN, as acos */
+  const double a = fabs(x);
+  const bool mid = a <= 0.5;
+  const double k = bmx_asin_kernel(mid ? x : sqrt((1.0 - a) * 0.5));
+  return mid ? BMX_PIO2 - k : (x > 0.0 ? 2.0 * k : BMX_PI - 2.0 * k);
+}
+__device__ __forceinline__ double4 trig_of(double theta, double phi) {
+  double st, ct, sp, cp;
+  sin_cos(theta, st, ct);
+  sin_cos(phi, sp, cp);
+  return make_double4(ct, st, cp, sp);
+}
+
+// 16-bit hash of an (id, cpu) pair, never 0.
+__device__ __forceinline__ uint32_t id_hash(int32_t id, int32_t cpu) {
+  const uint32_t h = (uint32_t)id * 0x9E3779B1u ^ (uint32_t)cpu * 0x85EBCA6Bu;
+  return 1u + (uint32_t)__umulhi(h, 65535u);
+}
+// (All scalars: local vectors and structs of arrays ended up in LDS.)
+__device__ __forceinline__ SegNear near_of(
+    double x, double y, double z, double rad, int type, double len, double ct,
+    double st, double cp, double sp, int n_bnds, int id0, int id1, int id2,
+    int id3, int cpu0, int cpu1, int cpu2, int cpu3, int self_id, int self_cpu) {
+  SegNear q;
+  q.x = x;
+  q.y = y;
+  q.z = z;
+  const bool seg = type == rec::FUNGI;
+  q.reach = seg ? len : rad;
+  q.nx = (float)(st * cp);
+  q.ny = (float)(st * sp);
+  q.nz = (float)ct;
+  q.rad = (float)rad;
+  const uint32_t s0 = seg && n_bnds > 0 ? id_hash(id0, cpu0) : 0u;
+  const uint32_t s1 = seg && n_bnds > 1 ? id_hash(id1, cpu1) : 0u;
+  const uint32_t s2 = seg && n_bnds > 2 ? id_hash(id2, cpu2) : 0u;
+  const uint32_t s3 = seg && n_bnds > 3 ? id_hash(id3, cpu3) : 0u;
+  q.bonds = (unsigned long long)(s2 | s3 << 16) << 32 | (s0 | s1 << 16);
+  q.self = seg ? id_hash(self_id, self_cpu) : 0u;
+  q.type = type;
+  return q;
+}
+__device__ __forceinline__ SegNear near_of(const double4 &p, int type,
+                                           const double4 &rod,
+                                           const double4 &tr, const Topo &tp) {
+  return near_of(p.x, p.y, p.z, p.w, type, rod.x, tr.x, tr.y, tr.z, tr.w, tp.n_bnds,
+                 tp.seg_id[0], tp.seg_id[1], tp.seg_id[2], tp.seg_id[3], tp.seg_cpu[0],
+                 tp.seg_cpu[1], tp.seg_cpu[2], tp.seg_cpu[3], tp.self_id, tp.self_cpu);
+}
+// Whether some bond slot may name the particle with the given hash (never
+// false when one does).
+__device__ __forceinline__ bool may_bond(unsigned long long slots, uint32_t self) {
+  const uint32_t r = self * 0x10001u;
+  const uint32_t lo = (uint32_t)slots ^ r, hi = (uint32_t)(slots >> 32) ^ r;
+  // a zero 16-bit half leaves its top bit set
+  return (((lo - 0x10001u) & ~lo) | ((hi - 0x10001u) & ~hi)) & 0x80008000u;
+}
+
+// True only if the contact force of two unbonded segments is exactly zero,
+// because every point of one is farther from every point of the other than
+// the sum of radii and the adhesion band.  d: separation of the centres.
+// The closest points are found in float, so the distance found is that of
+// two points of the segments up to rounding, above the smallest one by at
+// most a few eps (h_i + h_j)^2 in its square (near parallel axes the split is
+// ill-conditioned, but there the distance hardly depends on it); the margin
+// is 160 eps.  Left to the pair law: axes within 1e-4 of perpendicular (at
+// exactly perpendicular ones the law's points may lie outside the
+// segments), lengths that vanish beside the separation, sizes whose squares
+// come near the float range, and NaN.
+__device__ __forceinline__ bool cannot_touch(const SegNear &a, const SegNear &b,
+                                             double d0, double d1, double d2,
+                                             float wa) {
+  const float dx = (float)d0, dy = (float)d1, dz = (float)d2;
+  const float hi = 0.5f * (float)a.reach, hj = 0.5f * (float)b.reach;
+  const float c = a.nx * b.nx + a.ny * b.ny + a.nz * b.nz;
+  const float di = dx * a.nx + dy * a.ny + dz * a.nz;
+  const float dj = dx * b.nx + dy * b.ny + dz * b.nz;
+  const float det = fmaxf(1.0f - c * c, 1.0e-12f);
+  float s = (c * dj - di) * __builtin_amdgcn_rcpf(det);
+  s = fminf(fmaxf(s, -hi), hi);
+  const float t = fminf(fmaxf(c * s + dj, -hj), hj);
+  s = fminf(fmaxf(c * t - di, -hi), hi);
+  const float ex = dx + s * a.nx - t * b.nx, ey = dy + s * a.ny - t * b.ny,
+              ez = dz + s * a.nz - t * b.nz;
+  const float r2 = ex * ex + ey * ey + ez * ez;
+  const float ra = a.rad + b.rad + wa, h = hi + hj;
+  const float lim = 1.02f * ra * ra + 1.0e-5f * h * h;
+  return r2 > lim && lim > 1.0e-30f && fabsf(c) > 1.0e-4f &&
+         hi * hi > 1.0e-10f * (dx * dx + dy * dy + dz * dz);
+}
+
 __device__ __forceinline__ bool in01(double t) { return t >= 0.0 && t <= 1.0; }
 
 // Closest points of two segments (K.H:51-221).
@@ -269,22 +373,16 @@ __device__ inline void rod_mobility(double area, double c_length, double visc,
   }
   // D <- R D R^T with D diagonal, in the reference's summation order:
   // tmp[a][b] = sum_k D[a][k] R[b][k]; out[a][b] = sum_k R[a][k] tmp[k][b].
+  // The products with D's zeros add +-0 to a sum that starts at +0, which
+  // leaves D[a][a] R[b][a] + 0.
   double D0[3] = {d0, d0, d0}, D1[3] = {e0, e1, e1};
   double t0[3][3], t1[3][3];
 #pragma unroll
   for (int a = 0; a < 3; a++)
 #pragma unroll
     for (int b = 0; b < 3; b++) {
-      double s0 = 0.0, s1 = 0.0;
-#pragma unroll
-      for (int k = 0; k < 3; k++) {
-        double m0 = (a == k) ? D0[a] : 0.0;
-        double m1 = (a == k) ? D1[a] : 0.0;
-        s0 += m0 * R[b][k];
-        s1 += m1 * R[b][k];
-      }
-      t0[a][b] = s0;
-      t1[a][b] = s1;
+      t0[a][b] = D0[a] * R[b][a] + 0.0;
+      t1[a][b] = D1[a] * R[b][a] + 0.0;
     }
 #pragma unroll
   for (int a = 0; a < 3; a++)
@@ -360,40 +458,38 @@ __device__ inline void rod_pair_forces(const double d[3], const RodSelf &S,
   double rA = rS + fp.WA;
   double scale = S.bs * bsj;
   double kb = fp.kb;
-  int j_id[4], j_cpu[4], j_site[4];
-#pragma unroll
-  for (int b = 0; b < 4; b++) {
-    j_id[b] = tj.seg_id[b];
-    j_cpu[b] = tj.seg_cpu[b];
-    j_site[b] = tj.site[b];
-  }
-  int j_bnds = tj.n_bnds;
-  int iid = ti.self_id, icpu = ti.self_cpu;
-  int jid = tj.self_id, jcpu = tj.self_cpu;
+  const int jid = tj.self_id, jcpu = tj.self_cpu;
 
   // Bond tables hold at most 4 entries (n_bnds is checked to 0..4 at bind
-  // and a repair stops at 4).  Every lookup below runs over the 4 slots
-  // with constant indices, so the tables stay in registers; a search for
-  // the first match keeps the lowest matching slot.
+  // and a repair stops at 4).  Every lookup runs over the 4 slots with
+  // constant indices, so the tables stay in registers; mi and mj mark the
+  // slots of i that name j and of j that name i, and the lowest counts.
+  int mi = 0, mj = 0;
+#pragma unroll
+  for (int b = 0; b < 4; b++) {
+    if (b < ti.n_bnds && ti.seg_id[b] == jid && ti.seg_cpu[b] == jcpu) mi |= 1 << b;
+    if (b < tj.n_bnds && tj.seg_id[b] == ti.self_id && tj.seg_cpu[b] == ti.self_cpu)
+      mj |= 1 << b;
+  }
+  int si = 0, sj = 0;
+#pragma unroll
+  for (int b = 3; b >= 0; b--) {
+    if (mi >> b & 1) si = ti.site[b];
+    if (mj >> b & 1) sj = tj.site[b];
+  }
   // K.H:338-362
-  if (ti.position == rec::SECOND_1 || ti.position == rec::SECOND_2) {
-    int site = (ti.position == rec::SECOND_1) ? 1 : 2;
+  if (mi && (ti.position == rec::SECOND_1 || ti.position == rec::SECOND_2)) {
+    const int site = (ti.position == rec::SECOND_1) ? 1 : 2;
     bool hit = false;
 #pragma unroll
-    for (int b = 0; b < 4; b++)
-      hit = hit || (b < ti.n_bnds && ti.seg_id[b] == jid &&
-                    ti.seg_cpu[b] == jcpu && ti.site[b] == site);
+    for (int b = 0; b < 4; b++) hit = hit || ((mi >> b & 1) && ti.site[b] == site);
     if (hit && tj.position != rec::TIP) ti.position = rec::INTERIOR;
   }
   ti.dltd = 1;  // K.H:364-369
-  // K.H:372-545
-  bool i_to_j = false, j_to_i = false;
-#pragma unroll
-  for (int b = 0; b < 4; b++) {
-    i_to_j = i_to_j || (b < ti.n_bnds && ti.seg_id[b] == jid && ti.seg_cpu[b] == jcpu);
-    j_to_i = j_to_i || (b < j_bnds && j_id[b] == iid && j_cpu[b] == icpu);
-  }
-  if (!i_to_j && j_to_i) {
+  // K.H:372-545: a bond that only one side holds is added to the other
+  // (to j's copy, which this pair alone sees) where a slot is free
+  bool ihit = mi != 0, jhit = mj != 0;
+  if (!ihit && jhit) {
     int isite = (ti.fix_site == 0) ? ((ti.site[0] == 1) ? 2 : 1) : ti.fix_site;
     int nb = ti.n_bnds;
     if (nb >= 0 && nb <= 3) {
@@ -405,18 +501,13 @@ __device__ inline void rod_pair_forces(const double d[3], const RodSelf &S,
           ti.site[b] = isite;
         }
       ti.n_bnds = nb + 1;
+      ihit = true;
+      si = isite;
     }
-  } else if (i_to_j && !j_to_i) {
-    int jsite = (tj.fix_site == 0) ? ((tj.site[0] == 1) ? 2 : 1) : tj.fix_site;
-    if (j_bnds >= 0 && j_bnds <= 3) {
-#pragma unroll
-      for (int b = 0; b < 4; b++)
-        if (b == j_bnds) {
-          j_id[b] = iid;
-          j_cpu[b] = icpu;
-          j_site[b] = jsite;
-        }
-      j_bnds++;
+  } else if (ihit && !jhit) {
+    if (tj.n_bnds >= 0 && tj.n_bnds <= 3) {
+      jhit = true;
+      sj = (tj.fix_site == 0) ? ((tj.site[0] == 1) ? 2 : 1) : tj.fix_site;
     }
   }
 
@@ -436,19 +527,6 @@ __device__ inline void rod_pair_forces(const double d[3], const RodSelf &S,
   }
   bool bonded = false;
   // K.H:615-698
-  bool ihit = false, jhit = false;
-  int si = 0, sj = 0;
-#pragma unroll
-  for (int b = 3; b >= 0; b--) {  // descending: the lowest match is kept
-    if (b < ti.n_bnds && ti.seg_id[b] == jid && ti.seg_cpu[b] == jcpu) {
-      ihit = true;
-      si = ti.site[b];
-    }
-    if (b < j_bnds && j_id[b] == iid && j_cpu[b] == icpu) {
-      jhit = true;
-      sj = j_site[b];
-    }
-  }
   if (ihit && jhit) {
     int itip = ti.fuse_tip, jtip = tj.fuse_tip;
     if ((itip > 0 && itip == si) || (jtip > 0 && jtip == sj)) kb = scale * kb;
@@ -600,7 +678,8 @@ __device__ inline void rod_rotate(double &theta, double &phi,
   double ct = om[2], st = om[1];
   double orot[3][3] = {{1.0, 0.0, 0.0}, {0.0, ct, -st}, {0.0, st, ct}};
   double dth = on * subdt;
-  double nd[3] = {bmx_cos(dth), bmx_sin(dth), 0.0};
+  double nd[3] = {0.0, 0.0, 0.0};
+  sin_cos(dth, nd[1], nd[0]);
 #pragma unroll
   for (int a = 0; a < 3; a++) {
     double s = 0.0;
@@ -615,10 +694,10 @@ __device__ inline void rod_rotate(double &theta, double &phi,
     for (int b = 0; b < 3; b++) s += R[a][b] * om[b];
     nd[a] = s;
   }
-  theta = bmx_acos(nd[2]);
+  theta = acos_of(nd[2]);
   on = sqrt(nd[0] * nd[0] + nd[1] * nd[1]);
   if (on > 0.0) nd[0] /= on;
-  phi = bmx_acos(nd[0]);
+  phi = acos_of(nd[0]);
   if (nd[1] < 0.0) phi = 2.0 * kPi - phi;
 }
 

@@ -71,6 +71,22 @@ struct Topo {
 };
 static_assert(sizeof(Topo) == 80, "Topo layout");
 
+// What decides whether a neighbor can act on a segment, in one 64-byte
+// sector: position and reach as the pair test needs them, the axis and
+// radius in float for a distance bound, and hashes of the particle's own id
+// and of its bonds (16 bits each, never 0; 0 in an empty slot), equal
+// wherever the ids and cpus are.  Derived from the other arrays at every
+// rebuild and after every step that keeps its lists.
+struct SegNear {
+  double x, y, z;
+  double reach;  // c_length; the radius of a sphere
+  float nx, ny, nz, rad;
+  unsigned long long bonds;  // four 16-bit slots
+  uint32_t self;
+  int32_t type;
+};
+static_assert(sizeof(SegNear) == 64, "SegNear layout");
+
 // Per-particle arrays in sorted (binned) order.
 struct StaticArrays {  // permuted at rebuild only
   int32_t *oid;        // original index
@@ -84,6 +100,7 @@ struct DynArrays {     // rewritten every step (ping-pong)
   double4 *rod;        // c_length, theta, phi, area
   double4 *trig;       // cos(theta), sin(theta), cos(phi), sin(phi)
   Topo *topo;
+  SegNear *near;       // contexts with segments
 };
 
 // The level mesh of the particle <-> mesh coupling: n cells per axis,

@@ -27,7 +27,7 @@ __device__ __forceinline__ int64_t row_base(const FlatRows &f, int32_t maxn,
   return t / f.tile * f.tile * (int64_t)maxn + f.roff[t];
 }
 // Particles per tile for a context of n particles whose rows hold about
-// 'row' entries (4 to 64; segment and mixed contexts: 4 to 16).
+// 'row' entries (4 to 64; segment and mixed contexts: 4 to 32).
 int flat_tile(int segments, int64_t n, double row);
 // Entries to allocate for the flat rows of ncap particles.
 int64_t flat_entries(int64_t ncap, int tile, int32_t maxn);

@@ -120,7 +120,7 @@ __global__ void k_aos_unpack(const uint8_t *__restrict__ aos, AosLayout lay,
   if (dy.rod) {
     double L = rd[rec::c_length], th = rd[rec::theta], ph = rd[rec::phi];
     dy.rod[t] = make_double4(L, th, ph, rd[rec::area]);
-    dy.trig[t] = make_double4(bmx_cos(th), bmx_sin(th), bmx_cos(ph), bmx_sin(ph));
+    dy.trig[t] = trig_of(th, ph);
     st.bscale[t] = rd[rec::bond_scale];
     Topo tp;
     tp.n_bnds = id[rec::n_bnds];
@@ -204,8 +204,7 @@ __global__ void k_aos_refresh(const uint8_t *__restrict__ aos, AosLayout lay,
       if (fields & kFieldOrientations) {
         rr.y = rd[rec::theta];
         rr.z = rd[rec::phi];
-        dy.trig[t] = make_double4(bmx_cos(rr.y), bmx_sin(rr.y), bmx_cos(rr.z),
-                                  bmx_sin(rr.z));
+        dy.trig[t] = trig_of(rr.y, rr.z);
       }
       dy.rod[t] = rr;
       if (fields & kFieldBonds) {
@@ -230,6 +229,8 @@ __global__ void k_aos_refresh(const uint8_t *__restrict__ aos, AosLayout lay,
         const int nb = dy.topo[t].n_bnds;
         if (nb < 0 || nb > 4 || !(rr.x > 0.0)) bad = true;
       }
+      // lists that survive this call read it
+      if (dy.near) dy.near[t] = near_of(p, ty, rr, dy.trig[t], dy.topo[t]);
     }
     if (bad) nbad = 1;
   }
@@ -731,16 +732,35 @@ __global__ void k_sort_gather(const unsigned long long *__restrict__ permk,
     t = a;
     for (int64_t i = a; i < z; i++) t += permk[i] < e;
   }
-  dd.pos[t] = sd.pos[s];
+  // native vectors: double4's members and whole copies together keep it in
+  // memory (LDS)
+  typedef double double4v __attribute__((ext_vector_type(4)));
+  typedef int int4v __attribute__((ext_vector_type(4)));
+  const double4v p = reinterpret_cast<const double4v *>(sd.pos)[s];
+  const int32_t ty = ss.type[s];
+  reinterpret_cast<double4v *>(dd.pos)[t] = p;
   ds.oid[t] = ss.oid[s];
-  ds.type[t] = ss.type[s];
+  ds.type[t] = ty;
   ds.key[t] = b;
   if (multi) ds.col[t] = ss.col[s];
   if (rods) {
     ds.bscale[t] = ss.bscale[s];
-    dd.rod[t] = sd.rod[s];
-    dd.trig[t] = sd.trig[s];
-    dd.topo[t] = sd.topo[s];
+    const double4v rr = reinterpret_cast<const double4v *>(sd.rod)[s];
+    const double4v tr = reinterpret_cast<const double4v *>(sd.trig)[s];
+    reinterpret_cast<double4v *>(dd.rod)[t] = rr;
+    reinterpret_cast<double4v *>(dd.trig)[t] = tr;
+    const int4v *a = reinterpret_cast<const int4v *>(sd.topo + s);
+    int4v *b = reinterpret_cast<int4v *>(dd.topo + t);
+    const int4v x0 = a[0], x1 = a[1], x2 = a[2], x3 = a[3], x4 = a[4];
+    b[0] = x0;
+    b[1] = x1;
+    b[2] = x2;
+    b[3] = x3;
+    b[4] = x4;
+    // n_bnds, seg_id[4], seg_cpu[4], ..., self_id and self_cpu at 16 and 17
+    dd.near[t] = near_of(p[0], p[1], p[2], p[3], ty, rr[0], tr[0], tr[1], tr[2], tr[3],
+                         x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3], x2[0],
+                         x4[0], x4[1]);
   }
   if (chem_src) {  // the chemistry state's line (chem::stride doubles)
     const double4 *a = reinterpret_cast<const double4 *>(chem_src + s * chem::stride);
@@ -1454,10 +1474,16 @@ __device__ double general_finish(int64_t t, const BoxGeom &g,
     double w[3] = {acc[3], acc[4], acc[5]};
     rod_rotate(th, ph, tr_i, rod_i.x, w, fp.dt);
     out.rod[t] = make_double4(rod_i.x, th, ph, rod_i.w);
-    out.trig[t] = make_double4(bmx_cos(th), bmx_sin(th), bmx_cos(ph), bmx_sin(ph));
+    const double4 rod_o = make_double4(rod_i.x, th, ph, rod_i.w);
+    const double4 tr_o = trig_of(th, ph);
+    out.rod[t] = rod_o;
+    out.trig[t] = tr_o;
+    if (out.near) out.near[t] = near_of(make_double4(x, y, z, p.w), ty, rod_o, tr_o, ti);
   } else {
     out.rod[t] = rod_i;
     out.trig[t] = tr_i;
+    if (out.near)
+      out.near[t] = near_of(make_double4(x, y, z, p.w), ty, rod_i, tr_i, ti);
   }
   out.topo[t] = ti;
   if (fc) {  // original order
@@ -1473,69 +1499,61 @@ __device__ double general_finish(int64_t t, const BoxGeom &g,
 // ------------------------------------------------ flat general force ---
 //
 // Segments (and mixed colonies) over the flat row layout with tiles of at
-// most kGTile particles, one tile per wave.  Per window of 128 entries a light
-// pass (neighbor position, length and type) applies the interaction test;
-// the interacting entries are packed by ballot, in entry order, and only
-// they load the heavy data and run the pair law (rod_pair_i, sphere_pair),
-// each term into its LDS slot.  The tile's particles (the first lanes)
-// then add their runs of terms in row order.  The pair law is evaluated
+// most kGTile particles, one tile per wave.  Per window of 128 entries a
+// light pass reads one 64-byte sector per neighbor (SegNear), applies the
+// interaction test, and finds the entries that act: spheres, pairs that may
+// be bonded, and segments that may touch.  The other pairs' terms are zeros
+// (a zero force through a finite mobility), which adding leaves out.  The
+// entries that act queue up in LDS, in entry order; whenever 64 are queued
+// they load the heavy data and run the pair law (rod_pair_forces,
+// sphere_pair), each term into its LDS slot, and the tile's particles (the
+// first lanes) add their runs of terms in row order.  The pair law is evaluated
 // with the particle's record as it stands before its row; that is what the
 // row loop sees unless an earlier pair of the row repaired a bond.  A tile
 // where some pair repairs a bond is marked and recomputed row by row by
 // k_force_general_redo (general_rows), so every result is the row loop's;
-// keeping the row loop out of this kernel keeps its register budget low.  Promotion of a second segment and
-// the dltd reset do not depend on the order of the pairs.
+// keeping the row loop out of this kernel keeps its register budget low.
+// Promotion of a second segment and the dltd reset do not depend on the
+// order of the pairs.
+//
+// 200,000 segments (10.8 interacting pairs each, about three of which act):
+// 93 us, half of it issuing vector instructions (28.5 M per launch), the
+// rest waiting on dependent loads at three waves per SIMD.  With every
+// interacting pair through the law it was 157 us and 55.3 M instructions.
+// At 4 waves per SIMD 16 registers spill: 115 us.
 constexpr int kGTile = 32;
 constexpr int kGWin = 2 * kWave;
-constexpr int kGPass = kWave;  // packed pairs per pass
-// LDS per wave: the terms of one pass (6 x 64), the tile's mobility
-// matrices (18 x 32, formed once per segment) and the window's packed
-// pairs (neighbor, owner, promotion flag: 3 x 128)
-constexpr size_t kGenWaveBytes = 6 * kGPass * sizeof(double) +
-                                 18 * kGTile * sizeof(double) +
-                                 3 * kGWin * sizeof(int32_t);
-
-template <bool MULTI>
-__device__ __forceinline__ bool general_test(
-    int64_t ti_, int64_t u, bool valid, const DynArrays &in,
-    const StaticArrays &st, const BoxGeom *__restrict__ boxes,
-    const BoxGeom &g0, const ForceParams &fp) {
-  if (!valid) return false;
-  const int ty = st.type[ti_], tyj = st.type[u];
-  if (ty != tyj || (ty != rec::YEAST && ty != rec::FUNGI)) return false;
-  const BoxGeom &g = MULTI ? boxes[st.col[ti_]] : g0;
-  const double4 p = in.pos[ti_], o = in.pos[u];
-  const double d0 = sep_axis(p.x, o.x, g.L[0], g.halfL[0], g.periodic[0]);
-  const double d1 = sep_axis(p.y, o.y, g.L[1], g.halfL[1], g.periodic[1]);
-  const double d2 = sep_axis(p.z, o.z, g.L[2], g.halfL[2], g.periodic[2]);
-  const double r2 = d0 * d0 + d1 * d1 + d2 * d2;
-  double lim;
-  if (ty == rec::YEAST) {
-    lim = p.w + o.w + fp.WA - 1.0e-15;
-  } else {
-    const double rlm = 1.5 * (in.rod[ti_].x + in.rod[u].x) + fp.WA;  // K.H:33-37
-    lim = rlm - 1.0e-15;
-  }
-  return r2 <= lim * lim;
+constexpr int kGPass = kWave;           // packed pairs per pass
+constexpr int kGQueue = kGWin + kGPass; // entries that act, waiting
+// LDS of an owner's SegNear, padded off the bank period
+constexpr int kGNear = 80;
+// LDS per wave: the terms of one pass (6 x 64), the tile's mobility matrices
+// (18 per particle, formed once) and its SegNear, the queue (neighbor,
+// owner) and the pass's promotion flags
+size_t general_lds(int tile) {
+  return 6 * kGPass * sizeof(double) +
+         (size_t)tile * (18 * sizeof(double) + kGNear) +
+         (2 * kGQueue + kGPass) * sizeof(int32_t);
 }
 
 template <bool MULTI>
-__global__ __launch_bounds__(256, 4) void k_force_general_flat(
+__global__ __launch_bounds__(256, 3) void k_force_general_flat(
     DynArrays in, DynArrays out, StaticArrays st,
     const int32_t *__restrict__ cidx, const uint8_t *__restrict__ cown,
     const int32_t *__restrict__ wtot, int8_t *__restrict__ redo_tile,
     const int32_t *__restrict__ ncnt, int64_t n, int tsize, int32_t maxn,
     const BoxGeom *__restrict__ boxes, BoxGeom g0,
     ForceParams fp, double *__restrict__ fc, double *__restrict__ vmax,
-    int32_t *__restrict__ err, int remap) {
+    int32_t *__restrict__ err, int remap, int wave_bytes) {
   extern __shared__ __align__(16) unsigned char gen_lds[];
   const int lane = threadIdx.x & (kWave - 1);
   const int wv = threadIdx.x / kWave, nwv = blockDim.x / kWave;
-  double *res = reinterpret_cast<double *>(gen_lds + wv * kGenWaveBytes);
-  double *mob = res + 6 * kGPass;  // mob[m * kGTile + owner]: dii (m < 9), dij
-  int32_t *pu = reinterpret_cast<int32_t *>(mob + 18 * kGTile);
-  int32_t *po = pu + kGWin;
-  int32_t *pf = po + kGWin;
+  double *res = reinterpret_cast<double *>(gen_lds + wv * wave_bytes);
+  double *mob = res + 6 * kGPass;  // mob[m * tsize + owner]: dii (m < 9), dij
+  unsigned char *own = reinterpret_cast<unsigned char *>(mob + 18 * tsize);
+  int32_t *qu = reinterpret_cast<int32_t *>(own + kGNear * tsize);
+  int32_t *qo = qu + kGQueue;
+  int32_t *pf = qo + kGQueue;
   const int64_t tile = tile_of(remap) * nwv + wv;
   const int64_t t0 = tile * tsize;
   const int64_t t = t0 + lane;
@@ -1546,110 +1564,182 @@ __global__ __launch_bounds__(256, 4) void k_force_general_flat(
     B = t0 * maxn;
     T = wtot[tile];
   }
-  const int c = active ? row_len(ncnt[t]) : 0;
+  const int32_t raw = active ? ncnt[t] : 0;
+  const int c = row_len(raw);
+  const int img = wave_or3(row_img(raw));  // axes that can need an image
   const int P = wave_incl_scan64(c) - c;
-  if (active && st.type[t] == rec::FUNGI && c > 0) {
-    // the two-site mobility of the segment, once (the pairs read it)
-    RodSelf S;
-    rod_self_geom(S, in.rod[t], in.trig[t], in.pos[t].w, st.bscale[t]);
-    rod_self_mob(S, in.trig[t], fp.visc);
+  if (active) {
+    SegNear q = in.near[t];
+    if (q.type == rec::FUNGI && c > 0) {
+      // the two-site mobility of the segment, once (the pairs read it)
+      RodSelf S;
+      rod_self_geom(S, in.rod[t], in.trig[t], in.pos[t].w, st.bscale[t]);
+      rod_self_mob(S, in.trig[t], fp.visc);
+      double sum = 0.0;
 #pragma unroll
-    for (int a = 0; a < 3; a++)
+      for (int a = 0; a < 3; a++)
 #pragma unroll
-      for (int b = 0; b < 3; b++) {
-        mob[(3 * a + b) * kGTile + lane] = S.dii[a][b];
-        mob[(9 + 3 * a + b) * kGTile + lane] = S.dij[a][b];
-      }
+        for (int b = 0; b < 3; b++) {
+          mob[(3 * a + b) * tsize + lane] = S.dii[a][b];
+          mob[(9 + 3 * a + b) * tsize + lane] = S.dij[a][b];
+          sum += S.dii[a][b] + S.dij[a][b];
+        }
+      // a zero force leaves no term only through a finite mobility: with an
+      // infinite radius here every pair goes through the law
+      if (!isfinite(sum)) q.rad = __builtin_huge_valf();
+    }
+    *reinterpret_cast<SegNear *>(own + kGNear * lane) = q;
   }
   wave_lds_sync();
   const unsigned long long below = (1ull << lane) - 1ull;
   double acc[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
   bool paired = false, promoted = false, repair = false;
-  for (int w0 = 0; w0 < T; w0 += kGWin) {
-    const int e0 = w0 + lane, e1 = e0 + kWave;
-    const bool v0 = e0 < T, v1 = e1 < T;
-    int u0 = 0, u1 = 0, o0 = 0, o1 = 0;
-    if (v0) {
-      u0 = cidx[B + e0];
-      o0 = cown[B + e0];
+  int a_lo = 0, a_hi = 0;      // this owner's queued entries, counted from 0
+  int queued = 0, passed = 0;  // entries queued and evaluated so far
+  const float wa = (float)fp.WA;
+  // bit 0: the pair interacts; bit 1: it acts
+  auto light = [&](int o, int u, bool valid) -> int {
+    if (!valid) return 0;
+    const SegNear a = *reinterpret_cast<const SegNear *>(own + kGNear * o);
+    const SegNear b = in.near[u];
+    if (a.type != b.type || (a.type != rec::YEAST && a.type != rec::FUNGI)) return 0;
+    const BoxGeom &g = MULTI ? boxes[st.col[t0 + o]] : g0;
+    double d0 = a.x - b.x, d1 = a.y - b.y, d2 = a.z - b.z;
+    if (img) {
+      d0 = sep_axis(a.x, b.x, g.L[0], g.halfL[0], g.periodic[0]);
+      d1 = sep_axis(a.y, b.y, g.L[1], g.halfL[1], g.periodic[1]);
+      d2 = sep_axis(a.z, b.z, g.L[2], g.halfL[2], g.periodic[2]);
     }
-    if (v1) {
-      u1 = cidx[B + e1];
-      o1 = cown[B + e1];
-    }
-    const bool i0 = general_test<MULTI>(t0 + o0, u0, v0, in, st, boxes, g0, fp);
-    const bool i1 = general_test<MULTI>(t0 + o1, u1, v1, in, st, boxes, g0, fp);
-    const unsigned long long b0 = __ballot(i0), b1 = __ballot(i1);
-    const int n0 = __popcll(b0), ni = n0 + __popcll(b1);
-    if (i0) {
-      const int k = __popcll(b0 & below);
-      pu[k] = u0;
-      po[k] = o0;
-    }
-    if (i1) {
-      const int k = n0 + __popcll(b1 & below);
-      pu[k] = u1;
-      po[k] = o1;
-    }
-    wave_lds_sync();
-    const int lo = P > w0 ? P : w0;
-    const int hi = P + c < w0 + kGWin ? P + c : w0 + kGWin;
-    const int klo = lo < hi ? packed_before(lo - w0, b0, b1, n0) : 0;
-    const int khi = lo < hi ? packed_before(hi - w0, b0, b1, n0) : 0;
-    for (int k0 = 0; k0 < ni; k0 += kGPass) {  // pair laws, packed
-      const int k = k0 + lane;
-      if (k < ni) {
-        const int64_t u = pu[k], ti_ = t0 + po[k];
-        const BoxGeom &g = MULTI ? boxes[st.col[ti_]] : g0;
-        const double4 p = in.pos[ti_], o = in.pos[u];
-        double d[3];
-        d[0] = sep_axis(p.x, o.x, g.L[0], g.halfL[0], g.periodic[0]);
-        d[1] = sep_axis(p.y, o.y, g.L[1], g.halfL[1], g.periodic[1]);
-        d[2] = sep_axis(p.z, o.z, g.L[2], g.halfL[2], g.periodic[2]);
-        double f[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-        int flag = 0;
-        if (st.type[ti_] == rec::YEAST) {
-          const double r2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
-          sphere_pair(d[0], d[1], d[2], r2, p.w + o.w, fp, f[0], f[1], f[2]);
-        } else {
-          RodSelf S;
-          rod_self_geom(S, in.rod[ti_], in.trig[ti_], p.w, st.bscale[ti_]);
-          Topo tio = in.topo[ti_];
-          const int pos0 = tio.position, nb0 = tio.n_bnds;
-          double f1[3], f2[3], ri[3];
-          {
-            const Topo tj = in.topo[u];
-            rod_pair_forces(d, S, tio, tj, in.rod[u].x, o.w, st.bscale[u],
-                            in.trig[u], fp, f1, f2, ri);
-          }
-          if (tio.n_bnds != nb0) repair = true;
-          if (tio.position != pos0) flag = 1;
-          const int ow = po[k];
-#pragma unroll
-          for (int a = 0; a < 3; a++)
-#pragma unroll
-            for (int b = 0; b < 3; b++) {
-              S.dii[a][b] = mob[(3 * a + b) * kGTile + ow];
-              S.dij[a][b] = mob[(9 + 3 * a + b) * kGTile + ow];
-            }
-          rod_pair_mobility(S, f1, f2, ri, f);
+    const double r2 = d0 * d0 + d1 * d1 + d2 * d2;
+    const bool seg = a.type == rec::FUNGI;
+    // K.H:33-37 and the sphere's r_lm
+    const double lim = (seg ? 1.5 * (a.reach + b.reach) + fp.WA
+                            : a.reach + b.reach + fp.WA) - 1.0e-15;
+    if (!(r2 <= lim * lim)) return 0;
+    if (seg && !may_bond(a.bonds, b.self) && !may_bond(b.bonds, a.self) &&
+        cannot_touch(a, b, d0, d1, d2, wa))
+      return 1;
+    return 3;
+  };
+  // evaluates the first min(64, waiting) queued entries
+  auto pass = [&]() {
+    const int m = queued - passed < kGPass ? queued - passed : kGPass;
+    if (lane < m) {
+      const int ow = qo[lane];
+      const int64_t u = qu[lane], ti_ = t0 + ow;
+      const BoxGeom &g = MULTI ? boxes[st.col[ti_]] : g0;
+      const double4 p = in.pos[ti_], o = in.pos[u];
+      double d[3];
+      d[0] = sep_axis(p.x, o.x, g.L[0], g.halfL[0], g.periodic[0]);
+      d[1] = sep_axis(p.y, o.y, g.L[1], g.halfL[1], g.periodic[1]);
+      d[2] = sep_axis(p.z, o.z, g.L[2], g.halfL[2], g.periodic[2]);
+      double f[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+      int flag = 0;
+      if (st.type[ti_] == rec::YEAST) {
+        const double r2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
+        sphere_pair(d[0], d[1], d[2], r2, p.w + o.w, fp, f[0], f[1], f[2]);
+      } else {
+        RodSelf S;
+        rod_self_geom(S, in.rod[ti_], in.trig[ti_], p.w, st.bscale[ti_]);
+        Topo tio = in.topo[ti_];
+        const int pos0 = tio.position, nb0 = tio.n_bnds;
+        double f1[3], f2[3], ri[3];
+        {
+          const Topo tj = in.topo[u];
+          rod_pair_forces(d, S, tio, tj, in.rod[u].x, o.w, st.bscale[u],
+                          in.trig[u], fp, f1, f2, ri);
         }
+        if (tio.n_bnds != nb0) repair = true;
+        if (tio.position != pos0) flag = 1;
 #pragma unroll
-        for (int q = 0; q < 6; q++) res[q * kGPass + lane] = f[q];
-        pf[k] = flag;
+        for (int a = 0; a < 3; a++)
+#pragma unroll
+          for (int b = 0; b < 3; b++) {
+            S.dii[a][b] = mob[(3 * a + b) * tsize + ow];
+            S.dij[a][b] = mob[(9 + 3 * a + b) * tsize + ow];
+          }
+        rod_pair_mobility(S, f1, f2, ri, f);
+      }
+#pragma unroll
+      for (int q = 0; q < 6; q++) res[q * kGPass + lane] = f[q];
+      pf[lane] = flag;
+    }
+    wave_lds_sync();
+    const int k0 = a_lo > passed ? a_lo - passed : 0;
+    const int k1 = a_hi < passed + m ? a_hi - passed : m;
+    for (int k = k0; k < k1; k++) {
+#pragma unroll
+      for (int q = 0; q < 6; q++) acc[q] += res[q * kGPass + k];
+      promoted = promoted || pf[k] != 0;
+    }
+    passed += m;
+    wave_lds_sync();
+  };
+  for (int w0 = 0;;) {
+    if (w0 < T) {
+      const int e0 = w0 + lane, e1 = e0 + kWave;
+      const bool v0 = e0 < T, v1 = e1 < T;
+      int u0 = 0, u1 = 0, o0 = 0, o1 = 0;
+      if (v0) {
+        u0 = cidx[B + e0];
+        o0 = cown[B + e0];
+      }
+      if (v1) {
+        u1 = cidx[B + e1];
+        o1 = cown[B + e1];
+      }
+      const int l0 = light(o0, u0, v0), l1 = light(o1, u1, v1);
+      const unsigned long long i0 = __ballot(l0 & 1), i1 = __ballot(l1 & 1);
+      const unsigned long long b0 = __ballot(l0 & 2), b1 = __ballot(l1 & 2);
+      const int n0 = __popcll(b0), ni = n0 + __popcll(b1);
+      const int qn = queued - passed;  // fewer than 64 wait here
+      if (l0 & 2) {
+        const int k = qn + __popcll(b0 & below);
+        qu[k] = u0;
+        qo[k] = o0;
+      }
+      if (l1 & 2) {
+        const int k = qn + n0 + __popcll(b1 & below);
+        qu[k] = u1;
+        qo[k] = o1;
+      }
+      const int lo = P > w0 ? P : w0;
+      const int hi = P + c < w0 + kGWin ? P + c : w0 + kGWin;
+      if (lo < hi) {
+        const int m0 = __popcll(i0);
+        paired = paired || packed_before(hi - w0, i0, i1, m0) >
+                               packed_before(lo - w0, i0, i1, m0);
+        if (lo == P) a_lo = queued + packed_before(lo - w0, b0, b1, n0);
+        a_hi = queued + packed_before(hi - w0, b0, b1, n0);
+      }
+      queued += ni;
+      wave_lds_sync();
+      w0 += kGWin;
+    }
+    const bool last = w0 >= T;
+    while (queued - passed >= kGPass || (last && queued > passed)) {
+      pass();
+      // the entries behind the pass move to the front
+      const int left = queued - passed;
+      int u[2], o[2];
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        const int k = h * kWave + lane;
+        u[h] = k < left ? qu[kGPass + k] : 0;
+        o[h] = k < left ? qo[kGPass + k] : 0;
       }
       wave_lds_sync();
-      const int a0 = klo > k0 ? klo : k0;
-      const int a1 = khi < k0 + kGPass ? khi : k0 + kGPass;
-      for (int k2 = a0; k2 < a1; k2++) {
 #pragma unroll
-        for (int q = 0; q < 6; q++) acc[q] += res[q * kGPass + (k2 - k0)];
-        promoted = promoted || pf[k2] != 0;
-        paired = true;
+      for (int h = 0; h < 2; h++) {
+        const int k = h * kWave + lane;
+        if (k < left) {
+          qu[k] = u[h];
+          qo[k] = o[h];
+        }
       }
       wave_lds_sync();
     }
-    wave_lds_sync();
+    if (last) break;
   }
   // A tile with a bond repair is left to k_force_general_redo.
   const bool redo = __any(repair);
@@ -2143,12 +2233,13 @@ hipError_t launch_force_general(DynArrays in, DynArrays out, StaticArrays st,
   if (n <= 0) return hipSuccess;
   const int b = ls.block > 256 ? 256 : ls.block;
   const int grid = force_blocks(n, flat.tile, b);
-  const size_t lds = (size_t)(b / kWave) * kGenWaveBytes;
+  const int wave_bytes = (int)general_lds(flat.tile);
+  const size_t lds = (size_t)(b / kWave) * wave_bytes;
   if (multi) {
     hipLaunchKernelGGL(k_force_general_flat<true>, dim3(grid), dim3(b), lds, s,
                        in, out, st, flat.cidx, flat.cown, flat.tot, redo_tile,
                        ncnt, n, flat.tile, maxn, boxes, g0, fp, fc, vmax, err,
-                       ls.remap);
+                       ls.remap, wave_bytes);
     hipLaunchKernelGGL(k_force_general_redo<true>, dim3(grid_for(n, 256)),
                        dim3(256), 0, s, in, out, st, redo_tile, flat, maxn,
                        ncnt, n, boxes, g0, fp, fc, vmax, err);
@@ -2156,7 +2247,7 @@ hipError_t launch_force_general(DynArrays in, DynArrays out, StaticArrays st,
     hipLaunchKernelGGL(k_force_general_flat<false>, dim3(grid), dim3(b), lds, s,
                        in, out, st, flat.cidx, flat.cown, flat.tot, redo_tile,
                        ncnt, n, flat.tile, maxn, boxes, g0, fp, fc, vmax, err,
-                       ls.remap);
+                       ls.remap, wave_bytes);
     hipLaunchKernelGGL(k_force_general_redo<false>, dim3(grid_for(n, 256)),
                        dim3(256), 0, s, in, out, st, redo_tile, flat, maxn,
                        ncnt, n, boxes, g0, fp, fc, vmax, err);
@@ -2174,14 +2265,15 @@ hipError_t launch_force_general(DynArrays in, DynArrays out, StaticArrays st,
 //   rows of 8:  24,000: 11.9 / 8.5 / 7.2 / 6.0 / 7.9;
 //               120,000: 15.3 / 13.6 / 15.0 / 16.1; 1M: 59 / 62 / 74 / 92
 //   rows of 72: 24,000: 57 / 32 / 21 / 15.0 / 14.0; 120,000: 73 / 52 / 45 / 42.5 / 47
-// Segment pairs are far heavier than a wave's start and end (and their rows
-// hold about ten): tiles of 32 / 16 / 8 / 4
-//   2,000: 57 / 40 / 29 / 24; 20,000: 89 / 64 / 49 / 46;
-//   60,000: 96 / 77 / 77 / 90; 200,000: 160 / 157 / 185 / 247
+// Segment waves carry far more per particle, so their tiles are as small as
+// keeps the waves resident at once (3 per SIMD), 64 / 32 / 16 / 8 / 4:
+//   5,000: - / 34 / 25 / 21.8 / 20.8; 20,000: 58 / 39 / 30 / 27.9 / 37;
+//   40,000: 63 / 47 / 36 / 42; 60,000: 63 / 45 / 48 / 55;
+//   200,000: 116 / 93 / 106 / 144
 int flat_tile(int segments, int64_t n, double row) {
   int t = 4;
   if (segments) {
-    while (t < 16 && n > (int64_t)t * 5120) t *= 2;
+    while (t < kGTile && n > (int64_t)t * 3072) t *= 2;
     return t;
   }
   while (t < kWave && 2 * t * row <= kFlatWin) t *= 2;

@@ -427,7 +427,7 @@ bmx_status bmx_fusion(bmx_ctx *ctx, const bmx_fusion_params *params,
  * forbid hipMalloc): one call does what bmx_bind_particles_aos (device
  * records) + bmx_evolve(dt, nsteps) + bmx_sync_to_aos do on a context, on
  * the caller's device records in place, with every working array in a
- * static device scratch the library holds per GPU (about 40 MB, from load
+ * static device scratch the library holds per GPU (about 45 MB, from load
  * to process end).  It calls no allocating routine.  Limits: n <=
  * BMX_NOALLOC_MAX_PARTICLES, max_neighbors <= BMX_NOALLOC_MAX_NEIGHBORS
  * (0 = that), rebuild_every <= BMX_NOALLOC_MAX_REBUILD_EVERY, at most

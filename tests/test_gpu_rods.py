@@ -242,3 +242,152 @@ def test_skin_check_sees_the_last_tiles(bmx, gpu, block):
     with pytest.raises(bmx.BMXError) as e:
         run(2.0 * 0.99 * bound, 2)
     assert e.value.code == 6                   # BMX_ERR_SKIN
+
+
+def contact_pairs(bmx, seed, n_side=11):
+    """Two segments per cell of a cubic grid: lengths over a factor of 60,
+    relative orientations from random over near parallel and near
+    perpendicular to exactly parallel, collinear and exactly perpendicular,
+    closest distances from overlap over both sides of the adhesion range to
+    well apart; some pairs bonded (on both sides, or stretched far beyond
+    contact)."""
+    rng = np.random.default_rng(seed)
+    gap = 2.2e-2
+    m = n_side ** 3
+    hi = np.full(3, n_side * gap)
+    recs = bmx.generate_hyphae(2 * m, 2 * m, 30e-4, 2e-4, 0.0, 30.0, 60.0, seed,
+                               [0, 0, 0], hi, 0.0)
+    cell = np.stack(np.unravel_index(np.arange(m), (n_side,) * 3), 1)
+    centre = (cell + 0.5) * gap
+    kind = rng.integers(0, 8, m)
+    u = rng.normal(size=(m, 3))
+    u /= np.linalg.norm(u, axis=1)[:, None]
+    axis = np.eye(3)[rng.integers(0, 3, m)]
+    u[kind >= 5] = axis[kind >= 5]
+    w = rng.normal(size=(m, 3))                      # a direction across u
+    other = np.eye(3)[(axis.argmax(1) + 1) % 3]
+    w[kind >= 5] = other[kind >= 5]
+    w -= (w * u).sum(1)[:, None] * u
+    w /= np.linalg.norm(w, axis=1)[:, None]
+    v = rng.normal(size=(m, 3))                      # 0, 1: any
+    eps = 10.0 ** rng.uniform(-9, -2, m)
+    near_par, near_perp = (kind == 2) | (kind == 3), kind == 4
+    v[near_par] = (u + eps[:, None] * w)[near_par]
+    v[near_perp] = (w + eps[:, None] * u)[near_perp]
+    v[kind == 5] = u[kind == 5]                      # parallel
+    v[kind == 6] = u[kind == 6]                      # collinear
+    v[kind == 7] = w[kind == 7]                      # perpendicular
+    v /= np.linalg.norm(v, axis=1)[:, None]
+    L = 10.0 ** rng.uniform(-4.0, -2.22, (2, m))
+    r = rng.uniform(1e-4, 3e-4, (2, m))
+    ra = r.sum(0) + 1.0e-4                           # radii + adhesion band
+    dist = ra * rng.choice([0.3, 0.9, 0.999, 1.0, 1.001, 1.005, 1.02, 1.1, 2.0], m)
+    off = np.cross(u, v)
+    bad = np.linalg.norm(off, axis=1) < 1e-6
+    off[bad] = w[bad]
+    off[kind == 6] = u[kind == 6]                    # end to end
+    off /= np.linalg.norm(off, axis=1)[:, None]
+    along = rng.uniform(-0.6, 0.6, m) * L[0]
+    d = off * dist[:, None] + along[:, None] * u
+    d[kind == 6] = (u * (0.5 * L.sum(0) + dist)[:, None])[kind == 6]
+    for k, (x, nrm) in enumerate(((centre, u), (centre + d, v))):
+        s = slice(k * m, (k + 1) * m)
+        recs["pos"][s] = x
+        recs["rdata"][s, 0] = r[k]
+        recs["rdata"][s, 1] = L[k]
+        recs["rdata"][s, 2] = np.arccos(np.clip(nrm[:, 2], -1, 1))
+        recs["rdata"][s, 3] = np.mod(np.arctan2(nrm[:, 1], nrm[:, 0]), 2 * np.pi)
+        recs["rdata"][s, 4] = 2 * np.pi * r[k] * L[k]
+    ids = recs["idata"]
+    for p in np.nonzero(rng.random(m) < 0.25)[0]:
+        for a, b, site in ((p, p + m, 1), (p + m, p, 2)):
+            ids[a, 6] = 1
+            ids[a, 7], ids[a, 11], ids[a, 15] = ids[b, 33], ids[b, 34], site
+    ids[::5, 34] = 3                                 # other cpu words
+    recs["cpu"][::5] = 3
+    for p in range(2 * m):                           # bonds name them as they are now
+        if ids[p, 6]:
+            ids[p, 11] = 3 if (ids[p, 7] - 1) % 5 == 0 else 0
+    return recs, hi
+
+
+@pytest.mark.parametrize("seed", [1, 2, 3])
+def test_pairs_around_contact_match_oracle(bmx, oracle, gpu, seed):
+    """Pairs are left out of the pair law only where their force is zero:
+    every orientation and length ratio, on both sides of the contact range,
+    bonded and not."""
+    recs, hi = contact_pairs(bmx, seed)
+    fpar = W.hyphae_fpar(-1.0)                       # the surface far below
+    ctx = bmx.Context(0)
+    ctx.set_force_params(fpar)
+    ctx.set_geometry([0, 0, 0], hi, (1, 1, 0))
+    ctx.set_neighbor_params(mode=bmx.NBR_VERLET, rebuild_every=1, skin=1e-4,
+                            max_neighbors=64)
+    ctx.bind(recs.copy())
+    orecs = recs.copy()
+    g = oracle.make_geom([0, 0, 0], hi, (1, 1, 0), ctx.bin_dims())
+    st = oracle.State(orecs, g, fpar, oracle.NBR_PAIR, 1e-4, 1)
+    for _ in range(2):
+        ctx.evolve(1e-3, 1)
+        fo = st.evolve(1e-3, 1)
+        assert np.array_equal(ctx.fc(), fo)
+    assert np.array_equal(ctx.int_fields(), orecs["idata"])
+    assert 0.1 < (np.abs(fo[:2]).sum(0) > 0).mean() < 0.9   # both kinds are there
+    ctx.close()
+    st.close()
+
+
+def test_infinite_mobility_is_still_an_error(bmx, gpu):
+    """Without viscous drag every interacting pair gives a non-finite term,
+    also one whose force is zero."""
+    recs, hi = contact_pairs(bmx, 4, n_side=4)
+    fpar = W.hyphae_fpar(-1.0)
+    fpar[8] = 0.0
+    two = recs[:2].copy()                            # placed far from contact
+    two["idata"][:, 6] = 0
+    two["rdata"][:, 1] = 6e-3
+    two["pos"] = [[0.03, 0.03, 0.03], [0.03, 0.03, 0.035]]
+    two["rdata"][:, 2] = 0.5 * np.pi
+    two["rdata"][:, 3] = [0.3, 0.9]
+    ctx = bmx.Context(0)
+    ctx.set_force_params(fpar)
+    ctx.set_geometry([0, 0, 0], hi, (1, 1, 0))
+    ctx.set_neighbor_params(mode=bmx.NBR_VERLET, rebuild_every=1, skin=1e-4)
+    ctx.bind(two)
+    with pytest.raises(bmx.BMXError) as e:
+        ctx.evolve(1e-3, 1)
+    assert e.value.code == 4
+    ctx.close()
+
+
+def test_refreshed_orientations_and_bonds_are_seen_by_kept_lists(bmx, oracle, gpu):
+    """A refresh that keeps the lists (orientations, bonds) reaches the data
+    the pair selection reads."""
+    recs, hi = contact_pairs(bmx, 6, n_side=6)
+    fpar = W.hyphae_fpar(-1.0)
+    ctx = bmx.Context(0)
+    ctx.set_force_params(fpar)
+    ctx.set_geometry([0, 0, 0], hi, (1, 1, 0))
+    ctx.set_neighbor_params(mode=bmx.NBR_VERLET, rebuild_every=10, skin=1e-3,
+                            max_neighbors=64)
+    grecs = recs.copy()
+    ctx.bind(grecs)
+    orecs = recs.copy()
+    g = oracle.make_geom([0, 0, 0], hi, (1, 1, 0), ctx.bin_dims())
+    st = oracle.State(orecs, g, fpar, oracle.NBR_PAIR, 1e-3, 10)
+    ctx.evolve(1e-3, 2)
+    st.evolve(1e-3, 2)
+    ctx.sync()
+    assert np.array_equal(grecs["pos"], orecs["pos"])
+    rng = np.random.default_rng(8)
+    th, ph = rng.uniform(0.1, 3.0, len(recs)), rng.uniform(0.0, 6.2, len(recs))
+    for r in (grecs, orecs):
+        r["rdata"][:, 2], r["rdata"][:, 3] = th, ph
+        r["idata"][:, 6] = 0                         # every bond is cut
+    ctx.refresh(bmx.FIELD_ORIENTATIONS | bmx.FIELD_BONDS)
+    for k in (1, 3):
+        ctx.evolve(1e-3, k)
+        fo = st.evolve(1e-3, k)
+        assert np.array_equal(ctx.fc(), fo)
+    ctx.close()
+    st.close()
