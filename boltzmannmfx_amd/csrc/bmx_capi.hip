@@ -2078,9 +2078,11 @@ extern "C" bmx_status bmx_exchange(bmx_ctx *c, const double xpar[3], double dt) 
   // the rows are rebuilt at the current positions (xchng.cpp:68-77)
   st = rebuild(c);
   if (st != BMX_OK) return st;
-  HIPCHK(launch_exchange(c->pos[c->cd].p, c->type[c->cs].p, c->topo[c->cd].p,
-                         flat_rows(c), c->maxn, c->d_ncnt.p, c->n,
-                         c->d_chemst[c->cc].p, xpar, dt, s));
+  // only segments exchange
+  if (c->any_fungi)
+    HIPCHK(launch_exchange(c->pos[c->cd].p, c->type[c->cs].p, c->near[c->cd].p,
+                           c->topo[c->cd].p, flat_rows(c), c->maxn, c->d_ncnt.p,
+                           c->n, c->d_chemst[c->cc].p, xpar, dt, s));
   return check_flags(c);
 }
 

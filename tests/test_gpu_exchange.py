@@ -105,3 +105,24 @@ def test_exchange_leaves_spheres_alone(bmx, gpu):
     ctx.sync()
     assert np.array_equal(recs["rdata"][:, 25:31], col.recs["rdata"][:, 25:31])
     ctx.close()
+
+
+@pytest.mark.parametrize("n", [3, 20_483, 70_001])
+def test_exchange_at_every_tile_size(bmx, oracle, gpu, n):
+    """Tiles of 4, 8 and 32 segments, the last one partly empty; rows longer
+    than a window of 64 entries per tile."""
+    col = mat(n=n, nroots=max(1, n // 100), seed=31)
+    if n == 3:
+        col.prob_hi, col.n_cell = np.array([0.04, 0.04, 0.016]), (20, 20, 8)
+    ctx, grecs, st, orecs = pair(bmx, oracle, col, 1, 1)
+    ctx.init_bonds()
+    assert st.init_bonds() == 0
+    for _ in range(2):
+        ctx.evolve(col.dt, 1)
+        st.evolve(col.dt, 1)
+        ctx.exchange(XPAR, 1.0)
+        st.exchange(XPAR, 1.0)
+    ctx.sync()
+    assert np.array_equal(grecs["rdata"][:, 25:31], orecs["rdata"][:, 25:31])
+    assert np.abs(orecs["rdata"][:, 28:31]).max() > 0
+    ctx.close()
