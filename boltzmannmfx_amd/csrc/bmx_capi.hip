@@ -93,7 +93,7 @@ struct bmx_ctx {
   std::vector<bmx_geometry> colony_geom;
   std::vector<int64_t> colony_start;
   std::vector<BoxGeom> boxes, boxes_next;
-  DevBuf<BoxGeom> d_boxes;
+  DevBuf<BoxGeom> d_boxes;  // several boxes (one box goes to kernels by value)
   DevBuf<int32_t> d_col_in;
   bool bound = false;
   bool any_fungi = false, any_yeast = false;
@@ -164,8 +164,14 @@ struct bmx_ctx {
   bool have_chem = false;
   // particle <-> mesh coupling: bins over the level mesh, staged fields
   DevBuf<int32_t> d_mkey, d_mrank, d_mcount, d_mstart, d_mscan;
+  size_t mcount_clear = 0;  // d_mcount.n while it holds zeros (the scan
+                            // leaves them)
   DevBuf<unsigned long long> d_mperm;
   DevBuf<double> d_mout, d_min;
+  // division and fusion: decisions and offsets of every particle
+  DevBuf<int32_t> w_cnt, w_start, w_scan, w_one, w_tgt, w_flag;
+  DevBuf<int4> w_dec;
+  DevBuf<double> w_tau, w_dtau;
   int32_t n_real = 0, n_int = 0;
   bool have_list = false;
   int64_t step = 0, last_build = -1;
@@ -179,10 +185,11 @@ struct bmx_ctx {
   DevBuf<unsigned long long> d_slotmax;  // per-slot maxima (skin check)
   int32_t vmax_slots = 1;
   int32_t vstride = 1;         // tiles (flat_tile) of ncap particles
-  int32_t row_nblk = 0;        // blocks of the last row build
-  // pinned: err, max row, total (2 words), ..., guard periods' errors
-  // (8, 9), the chemistry's size maxima (16..19), the adjoint forward's
-  // error word (20)
+  int32_t row_nblk = 0;        // blocks of a row build not yet reported
+  // pinned (32 words): err, max row, total (2 words), ..., guard periods'
+  // errors (8, 9), the chemistry's size maxima (16..19), the adjoint
+  // forward's error word (20), counts of split and fused particles (21), the
+  // bind statistics (22..31)
   int32_t *h_flags = nullptr;
   int32_t *h_flags_dev = nullptr;  // h_flags as the device addresses it
 
@@ -390,10 +397,13 @@ bmx_status setup_boxes(bmx_ctx *c) {
                                      std::to_string(c->nbins) +
                                      ") than the fixed scratch holds");
   }
-  hipError_t e = c->d_boxes.alloc(c->ncol);
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(c->d_boxes.p, c->boxes.data(), sizeof(BoxGeom) * c->ncol,
-                       hipMemcpyHostToDevice, c->stream);
+  hipError_t e = hipSuccess;
+  if (c->ncol > 1) {
+    e = c->d_boxes.alloc(c->ncol);
+    if (e == hipSuccess)
+      e = hipMemcpyAsync(c->d_boxes.p, c->boxes.data(), sizeof(BoxGeom) * c->ncol,
+                         hipMemcpyHostToDevice, c->stream);
+  }
   if (e == hipSuccess) e = c->d_count.alloc(c->nbins + 1);
   if (e == hipSuccess) e = c->d_start.alloc(c->nbins + 1);
   if (e == hipSuccess) e = c->d_scan.alloc(scan_scratch_elems(c->nbins) + 1);
@@ -623,22 +633,16 @@ bmx_status enqueue_flags(bmx_ctx *c) {
     bmx_status st = close_run(c);
     if (st != BMX_OK) return st;
   }
-  if (c->h_flags_dev) {
-    // one launch writes the words into host memory the device maps
-    HIPCHK(launch_flags_out(c->d_bstats.p, c->row_nblk, c->d_stats.p,
-                            c->d_total.p, c->d_err.p, c->h_flags_dev, s));
-    return BMX_OK;
-  }
-  if (c->row_nblk > 0)
-    HIPCHK(launch_reduce_rowstats(c->d_bstats.p, c->row_nblk, c->d_stats.p,
-                                  c->d_total.p, s));
-  HIPCHK(hipMemcpyAsync(c->h_flags, c->d_err.p, sizeof(int32_t),
-                        hipMemcpyDeviceToHost, s));
-  HIPCHK(hipMemcpyAsync(c->h_flags + 1, c->d_stats.p, sizeof(int32_t),
-                        hipMemcpyDeviceToHost, s));
-  HIPCHK(hipMemcpyAsync(c->h_flags + 2, c->d_total.p, sizeof(unsigned long long),
-                        hipMemcpyDeviceToHost, s));
-  HIPCHK(launch_fill_i32(c->d_err.p, 1, 0, s));
+  // one launch leaves the words in host memory the device maps, or beside
+  // the statistics, from where one copy brings them
+  const bool mapped = c->h_flags_dev != nullptr;
+  HIPCHK(launch_flags_out(c->d_bstats.p, c->row_nblk, c->d_stats.p, c->d_total.p,
+                          c->d_err.p, mapped ? c->h_flags_dev : c->d_stats.p + 4,
+                          mapped ? 1 : 0, s));
+  c->row_nblk = 0;
+  if (!mapped)
+    HIPCHK(hipMemcpyAsync(c->h_flags, c->d_stats.p + 4, 4 * sizeof(int32_t),
+                          hipMemcpyDeviceToHost, s));
   return BMX_OK;
 }
 
@@ -841,11 +845,11 @@ bmx_status bind_common(bmx_ctx *c, const void *aos, const int64_t *cstart,
       b.dxi[d] = 1.0;
     }
   }
-  HIPCHK(c->d_boxes.alloc(ncol));
-  HIPCHK(hipMemcpyAsync(c->d_boxes.p, c->boxes.data(), sizeof(BoxGeom) * ncol,
-                        hipMemcpyHostToDevice, s));
   const int32_t *dcol = nullptr;
   if (ncol > 1) {
+    HIPCHK(c->d_boxes.alloc(ncol));
+    HIPCHK(hipMemcpyAsync(c->d_boxes.p, c->boxes.data(), sizeof(BoxGeom) * ncol,
+                          hipMemcpyHostToDevice, s));
     std::vector<int32_t> hc((size_t)n);
     for (int k = 0; k < ncol; k++)
       for (int64_t i = cstart[k]; i < cstart[k + 1]; i++) hc[i] = k;
@@ -860,11 +864,13 @@ bmx_status bind_common(bmx_ctx *c, const void *aos, const int64_t *cstart,
   HIPCHK(launch_fill_u64(c->d_ustats.p, 8, 0ull, s));
   StaticArrays st = static_arrays(c, 0);
   DynArrays dy = dyn_arrays(c, 0);
-  HIPCHK(launch_aos_unpack(c->recs, c->lay, n, dcol, c->d_boxes.p, st, dy,
-                           c->d_ustats.p, s));
-  unsigned long long hs[8];
-  HIPCHK(hipMemcpyAsync(hs, c->d_ustats.p, sizeof hs, hipMemcpyDeviceToHost, s));
+  HIPCHK(launch_aos_unpack(c->recs, c->lay, n, dcol, c->d_boxes.p, c->boxes[0], st,
+                           dy, c->d_ustats.p, s));
+  unsigned long long hs[5];
+  HIPCHK(hipMemcpyAsync(c->h_flags + 22, c->d_ustats.p, sizeof hs,
+                        hipMemcpyDeviceToHost, s));
   HIPCHK(hipStreamSynchronize(s));
+  std::memcpy(hs, c->h_flags + 22, sizeof hs);
   if (hs[4] != 0)
     return fail(BMX_ERR_BAD_ARG,
                 "particle records with negative radius, non-finite position, "
@@ -883,7 +889,8 @@ bmx_status bind_common(bmx_ctx *c, const void *aos, const int64_t *cstart,
   bs = alloc_partials(c);
   if (bs != BMX_OK) return bs;
   c->row_nblk = 0;
-  HIPCHK(hipStreamSynchronize(s));
+  // (setup_boxes copies several boxes from a host array)
+  if (ncol > 1) HIPCHK(hipStreamSynchronize(s));
   c->step = 0;
   c->last_build = -1;
   c->rebuilds_total = 0;
@@ -934,7 +941,7 @@ bmx_status bmx_ctx_create(bmx_ctx **out, int32_t device) {
     e = hipEventCreateWithFlags(&c->done_ev, hipEventDisableTiming);
   if (e == hipSuccess) e = hipHostMalloc((void **)&c->h_flags, 128);
   if (e == hipSuccess) e = c->d_err.alloc(1) ;
-  if (e == hipSuccess) e = c->d_stats.alloc(4);
+  if (e == hipSuccess) e = c->d_stats.alloc(8);
   if (e == hipSuccess) e = c->d_total.alloc(1);
   if (e != hipSuccess) {
     bmx_ctx_destroy(c);
@@ -994,6 +1001,11 @@ void bmx_ctx_destroy(bmx_ctx *c) {
   c->d_slotmax.release();
   c->d_ustats.release();
   for (auto &b : c->d_chemst) b.release();
+  for (auto *b : {&c->w_cnt, &c->w_start, &c->w_scan, &c->w_one, &c->w_tgt, &c->w_flag})
+    b->release();
+  c->w_dec.release();
+  c->w_tau.release();
+  c->w_dtau.release();
   c->d_mkey.release();
   c->d_mrank.release();
   c->d_mcount.release();
@@ -1544,12 +1556,14 @@ bmx_status bmx_refresh_from_aos(bmx_ctx *c, const void *aos, uint32_t fields) {
       HIPCHK(hipMemcpyAsync(c->recs, src, (size_t)c->n * stride, kind, s));
   }
   HIPCHK(launch_fill_u64(c->d_ustats.p, 8, 0ull, s));
-  HIPCHK(launch_aos_refresh(c->recs, c->lay, c->n, c->d_boxes.p,
+  HIPCHK(launch_aos_refresh(c->recs, c->lay, c->n, c->boxes[0],
                             static_arrays(c, c->cs), dyn_arrays(c, c->cd),
                             fields, c->d_ustats.p, s));
-  unsigned long long hs[8];
-  HIPCHK(hipMemcpyAsync(hs, c->d_ustats.p, sizeof hs, hipMemcpyDeviceToHost, s));
+  unsigned long long hs[5];
+  HIPCHK(hipMemcpyAsync(c->h_flags + 22, c->d_ustats.p, sizeof hs,
+                        hipMemcpyDeviceToHost, s));
   HIPCHK(hipStreamSynchronize(s));
+  std::memcpy(hs, c->h_flags + 22, sizeof hs);
   if (hs[4] != 0) {
     c->bound = false;
     return fail(BMX_ERR_BAD_ARG,
@@ -1661,6 +1675,7 @@ bmx_status bmx_evolve_graph(bmx_ctx *c, double dt, int32_t nsteps) {
       if (c->have_chem) c->cc = 1 - c->cc;
       c->have_list = true;
       c->last_build = c->step;
+      c->row_nblk = tile_count(c->n, c->flat_tile);
       c->rebuilds_total++;
     }
     c->cd = 1 - c->cd;
@@ -2365,7 +2380,8 @@ int64_t mesh_cells(const MeshGeom &g, int ghost) {
 // Bins the particles (current sorted arrays) over the level mesh.  The
 // records are not needed: the positions are the sorted ones and the
 // deposited fields (vol, rdata[31..33]) are only changed in the records.
-bmx_status mesh_bin(bmx_ctx *c, const MeshGeom &g, int tri, int sorted) {
+bmx_status mesh_bin(bmx_ctx *c, const MeshGeom &g, int tri, int sorted,
+                    unsigned long long *clear2 = nullptr) {
   (void)hipSetDevice(c->device);
   int64_t nb = 1;
   for (int d = 0; d < 3; d++)
@@ -2377,21 +2393,35 @@ bmx_status mesh_bin(bmx_ctx *c, const MeshGeom &g, int tri, int sorted) {
   HIPCHK(c->d_mcount.alloc((size_t)nb + 1));
   HIPCHK(c->d_mstart.alloc((size_t)nb + 1));
   HIPCHK(c->d_mscan.alloc((size_t)scan_scratch_elems(nb) + 1));
+  if (c->mcount_clear != c->d_mcount.n)
+    HIPCHK(launch_fill_i32(c->d_mcount.p, (int64_t)c->d_mcount.n, 0, c->stream));
+  c->mcount_clear = 0;
   HIPCHK(launch_mesh_bin(c->pos[c->cd].p, c->oid[c->cs].p, c->n, g, tri,
                          c->d_mkey.p, c->d_mrank.p, c->d_mcount.p,
                          c->d_mstart.p, c->d_mscan.p, c->d_mperm.p, sorted,
-                         c->d_err.p, c->stream));
+                         c->d_err.p, clear2, c->stream));
+  c->mcount_clear = c->d_mcount.n;
   return BMX_OK;
 }
 
-// Reads and clears the error word after the mesh kernels.
-bmx_status mesh_flags(bmx_ctx *c) {
+// Reads and clears the error word after the mesh kernels; with maxima, also
+// brings the chemistry's size maxima (h_flags 16..19).
+bmx_status mesh_flags(bmx_ctx *c, const unsigned long long *maxima = nullptr) {
   hipStream_t s = c->stream;
-  HIPCHK(hipMemcpyAsync(c->h_flags, c->d_err.p, sizeof(int32_t),
-                        hipMemcpyDeviceToHost, s));
-  HIPCHK(launch_fill_i32(c->d_err.p, 1, 0, s));
+  if (c->h_flags_dev) {
+    HIPCHK(launch_mesh_out(c->d_err.p, maxima, c->h_flags_dev,
+                           reinterpret_cast<unsigned long long *>(c->h_flags_dev + 16), s));
+  } else {
+    HIPCHK(hipMemcpyAsync(c->h_flags, c->d_err.p, sizeof(int32_t),
+                          hipMemcpyDeviceToHost, s));
+    if (maxima)
+      HIPCHK(hipMemcpyAsync(c->h_flags + 16, maxima, 2 * sizeof(unsigned long long),
+                            hipMemcpyDeviceToHost, s));
+    HIPCHK(launch_fill_i32(c->d_err.p, 1, 0, s));
+  }
   HIPCHK(hipStreamSynchronize(s));
   const int32_t err = c->h_flags[0];
+  c->h_flags[0] = 0;
   if (err & ERRBIT_MESH)
     return fail(BMX_ERR_MESH,
                 "a particle lies outside the level mesh, or one cell holds "
@@ -2489,7 +2519,7 @@ extern "C" bmx_status bmx_calc_txfr_particle(bmx_ctx *c, const double chempar[10
   MeshGeom g;
   st = mesh_geom(c, g);
   if (st != BMX_OK) return st;
-  st = mesh_bin(c, g, 0, 0);  // particles per cell
+  st = mesh_bin(c, g, 0, 0, c->d_ustats.p);  // particles per cell
   if (st != BMX_OK) return st;
   hipStream_t s = c->stream;
   const int64_t ng = mesh_cells(g, 1);
@@ -2509,16 +2539,13 @@ extern "C" bmx_status bmx_calc_txfr_particle(bmx_ctx *c, const double chempar[10
   // next step for the new reaches
   st = load_chem(c);
   if (st != BMX_OK) return st;
-  HIPCHK(launch_fill_u64(c->d_ustats.p, 8, 0ull, s));
   HIPCHK(launch_mesh_to_particle(c->d_chemst[c->cc].p, c->n, g, c->d_mstart.p,
                                  c->type[c->cs].p,
                                  c->any_fungi ? c->topo[c->cd].p : nullptr,
                                  c->pos[c->cd].p, c->rod[c->cd].p, X, V,
                                  cnc_scheme, vf_scheme, chempar, dt, nloop,
                                  c->d_ustats.p, c->d_err.p, s));
-  HIPCHK(hipMemcpyAsync(c->h_flags + 16, c->d_ustats.p, 2 * sizeof(unsigned long long),
-                        hipMemcpyDeviceToHost, s));
-  st = mesh_flags(c);  // synchronizes the stream
+  st = mesh_flags(c, c->d_ustats.p);  // synchronizes the stream
   if (st == BMX_ERR_HIP) return st;
   // the sorted sizes have changed either way: new bins, rows rebuilt
   std::memcpy(&c->rmax, c->h_flags + 16, sizeof(double));
@@ -2595,17 +2622,16 @@ extern "C" bmx_status bmx_split_particles(bmx_ctx *c, const bmx_split_params *sp
   st = pack_records(c);
   if (st != BMX_OK) return st;
   const int64_t n = c->n;
-  DevBuf<int32_t> cnt, start, scratch;
-  Releaser<int32_t> r1{cnt}, r2{start}, r3{scratch};
+  DevBuf<int32_t> &cnt = c->w_cnt, &start = c->w_start, &scratch = c->w_scan;
   HIPCHK(cnt.alloc((size_t)n + 1));
   HIPCHK(start.alloc((size_t)n + 1));
   HIPCHK(scratch.alloc((size_t)scan_scratch_elems(n) + 1));
   HIPCHK(launch_split_count(c->recs, c->lay, n, p, seed, call, cnt.p, s));
   HIPCHK(launch_scan(cnt.p, start.p, n, scratch.p, s));
-  int32_t total = 0;
-  HIPCHK(hipMemcpyAsync(&total, start.p + n, sizeof total,
+  HIPCHK(hipMemcpyAsync(c->h_flags + 21, start.p + n, sizeof(int32_t),
                         hipMemcpyDeviceToHost, s));
   HIPCHK(hipStreamSynchronize(s));
+  const int32_t total = c->h_flags[21];
   *n_new = total;
   if (total > 0) {
     if ((int64_t)next_id + total > (int64_t)INT32_MAX)
@@ -2659,10 +2685,8 @@ extern "C" bmx_status bmx_fusion(bmx_ctx *c, const bmx_fusion_params *fp,
   const BoxGeom g0 = c->boxes[0];
   const double wa = c->fpar[0];
   const int64_t n = c->n;
-  DevBuf<int32_t> flag, tgt;
-  DevBuf<double> ttau;
-  Releaser<int32_t> rf{flag}, rt{tgt};
-  Releaser<double> rtt{ttau};
+  DevBuf<int32_t> &flag = c->w_flag, &tgt = c->w_tgt;
+  DevBuf<double> &ttau = c->w_tau;
   HIPCHK(flag.alloc(1));
   HIPCHK(tgt.alloc((size_t)n + 1));
   HIPCHK(ttau.alloc((size_t)n + 1));
@@ -2670,18 +2694,16 @@ extern "C" bmx_status bmx_fusion(bmx_ctx *c, const bmx_fusion_params *fp,
   HIPCHK(launch_tip_fusion(c->recs, c->lay, n, c->pos[c->cd].p,
                            c->oid[c->cs].p, flat_rows(c), c->maxn, c->d_ncnt.p, g0,
                            wa, fus, seed, call, tgt.p, ttau.p, flag.p, s));
-  int32_t any = 0;
-  HIPCHK(hipMemcpyAsync(&any, flag.p, sizeof any, hipMemcpyDeviceToHost, s));
+  HIPCHK(hipMemcpyAsync(c->h_flags + 21, flag.p, sizeof(int32_t),
+                        hipMemcpyDeviceToHost, s));
   HIPCHK(hipStreamSynchronize(s));
-  if (!any) return BMX_OK;  // no record changed
+  if (!c->h_flags[21]) return BMX_OK;  // no record changed
   *fused = 1;
   // interior fusion over the same rows, decisions then updates
-  DevBuf<int32_t> cnt, one, start, scratch;
-  DevBuf<int4> dec;
-  DevBuf<double> dtau;
-  Releaser<int32_t> r1{cnt}, r2{one}, r3{start}, r4{scratch};
-  Releaser<int4> r5{dec};
-  Releaser<double> r6{dtau};
+  DevBuf<int32_t> &cnt = c->w_cnt, &one = c->w_one, &start = c->w_start,
+                  &scratch = c->w_scan;
+  DevBuf<int4> &dec = c->w_dec;
+  DevBuf<double> &dtau = c->w_dtau;
   HIPCHK(cnt.alloc((size_t)n + 1));
   HIPCHK(one.alloc((size_t)n + 1));
   HIPCHK(start.alloc((size_t)n + 1));
@@ -2692,9 +2714,10 @@ extern "C" bmx_status bmx_fusion(bmx_ctx *c, const bmx_fusion_params *fp,
                                 c->oid[c->cs].p, flat_rows(c), c->maxn, c->d_ncnt.p,
                                 g0, wa, cnt.p, dec.p, dtau.p, one.p, s));
   HIPCHK(launch_scan(one.p, start.p, n, scratch.p, s));
-  int32_t total = 0;
-  HIPCHK(hipMemcpyAsync(&total, start.p + n, sizeof total, hipMemcpyDeviceToHost, s));
+  HIPCHK(hipMemcpyAsync(c->h_flags + 21, start.p + n, sizeof(int32_t),
+                        hipMemcpyDeviceToHost, s));
   HIPCHK(hipStreamSynchronize(s));
+  const int32_t total = c->h_flags[21];
   if ((int64_t)next_id + total > (int64_t)INT32_MAX)
     return fail(BMX_ERR_BAD_ARG, "particle ids would overflow int32");
   const size_t stride = (size_t)c->lay.stride;
@@ -2768,7 +2791,7 @@ constexpr size_t kNaBytes =
     + na_align(8 * kNaTiles * kNaRebuild)        // displacement slots
     + na_align(8 * kNaRebuild)                   // slot maxima
     + na_align(4 * 2 * kNaTiles)                 // row-build block stats
-    + na_align(4) + na_align(16) + na_align(8) + na_align(64)  // err, stats, total, ustats
+    + na_align(4) + na_align(32) + na_align(8) + na_align(64)  // err, stats, total, ustats
     + na_align(sizeof(BoxGeom));
 
 static __device__ __align__(256) uint8_t scratch[kNaBytes];
@@ -2777,7 +2800,7 @@ struct NaDevice {
   bool ready = false;
   uint8_t *ptr = nullptr;  // this device's copy of scratch
   bmx_ctx ctx;
-  int32_t flags[16];       // host words the error/statistics reads land in
+  alignas(8) int32_t flags[32];  // host words the error/statistics reads land in
 };
 NaDevice g_na[kNaDevices];
 
@@ -2830,7 +2853,7 @@ bmx_status na_setup(NaDevice &d, int dev) {
   na_slice(c.d_slotmax, cur, (size_t)kNaRebuild);
   na_slice(c.d_bstats, cur, 2 * kNaTiles);
   na_slice(c.d_err, cur, 1);
-  na_slice(c.d_stats, cur, 4);
+  na_slice(c.d_stats, cur, 8);
   na_slice(c.d_total, cur, 1);
   na_slice(c.d_ustats, cur, 8);
   na_slice(c.d_boxes, cur, 1);

@@ -37,11 +37,12 @@ hipError_t launch_fill_u64(unsigned long long *p, int64_t n,
                            unsigned long long v, hipStream_t s);
 
 // AoS -> sorted SoA (identity order), periodic wrap, per-box bounds stats.
+// g0: the box of every particle when col is null
 // stats: [0] max radius bits, [1] max c_length bits, [2] any yeast,
 // [3] any fungi, [4] bad record count
 hipError_t launch_aos_unpack(const uint8_t *aos, AosLayout lay, int64_t n,
                              const int32_t *col, const BoxGeom *boxes,
-                             StaticArrays st, DynArrays dy,
+                             BoxGeom g0, StaticArrays st, DynArrays dy,
                              unsigned long long *stats, hipStream_t s);
 // Fields bmx_refresh_from_aos re-reads (the BMX_FIELD_* values of the ABI).
 enum : uint32_t {
@@ -52,9 +53,9 @@ enum : uint32_t {
 // values there (stats as launch_aos_unpack: [0] max radius, [1] max
 // c_length, [4] bad records)
 hipError_t launch_aos_refresh(const uint8_t *aos, AosLayout lay, int64_t n,
-                              const BoxGeom *boxes, StaticArrays st,
-                              DynArrays dy, uint32_t fields,
-                              unsigned long long *stats, hipStream_t s);
+                              BoxGeom g, StaticArrays st, DynArrays dy,
+                              uint32_t fields, unsigned long long *stats,
+                              hipStream_t s);
 // sorted SoA -> AoS (fields the force pass writes; with state, the chemistry
 // state's too, and each particle's radius and length); inv: n words of
 // scratch
@@ -133,16 +134,17 @@ hipError_t launch_force_sphere_flat(const double4 *pos_in, double4 *pos_out,
                                     hipStream_t s);
 // tiles of n particles (at least one)
 int32_t tile_count(int64_t n, int tile);
-// The end of a call in one launch: row statistics (nblk > 0), then err,
-// longest row and entry total (low, high word) into host_out (host memory
-// mapped for the device), err cleared.
+// The end of a call in one launch: row statistics (nblk > 0), then err
+// (add: OR-ed to what is there), longest row and entry total (low, high
+// word) into out (4 words), err cleared.
 hipError_t launch_flags_out(const int32_t *bstats, int32_t nblk, int32_t *stats,
                             unsigned long long *total, int32_t *err,
-                            int32_t *host_out, hipStream_t s);
-// stats[0] = longest row, *total = entries, from the per-block partials
-hipError_t launch_reduce_rowstats(const int32_t *bstats, int32_t nblk,
-                                  int32_t *stats, unsigned long long *total,
-                                  hipStream_t s);
+                            int32_t *out, int add, hipStream_t s);
+// The end of a mesh call: err into out_err, cleared, and with maxima the
+// chemistry's two size maxima into out_max.
+hipError_t launch_mesh_out(int32_t *err, const unsigned long long *maxima,
+                           int32_t *out_err, unsigned long long *out_max,
+                           hipStream_t s);
 
 // ---- segment (and mixed) force + overdamped update, fused: fc and vmax
 // as for launch_force_sphere_flat.
@@ -239,14 +241,16 @@ hipError_t launch_exchange(const double4 *pos, const int32_t *type,
                            hipStream_t s);
 
 // ---- particle <-> mesh (bmx_mesh.hip), over the sorted arrays
-// Bins the particles by mesh cell, or by trilinear base cell (tri);
-// start[0..nb] from the counts; with 'sorted', perm lists each bin's
+// Bins the particles by mesh cell, or by trilinear base cell (tri); count:
+// zeros, left zero; start[0..nb] from the counts; clear2: two words set to
+// zero on the way (or null); with 'sorted', perm lists each bin's
 // particles as (original index << 32 | sorted index), ascending.
 hipError_t launch_mesh_bin(const double4 *pos, const int32_t *oid, int64_t n,
                            const MeshGeom &g, int tri, int32_t *key,
                            int32_t *rank, int32_t *count, int32_t *start,
                            int32_t *scan_scratch, unsigned long long *perm,
-                           int sorted, int32_t *err, hipStream_t s);
+                           int sorted, int32_t *err,
+                           unsigned long long *clear2, hipStream_t s);
 // mode 0: sums of rdata[comp0..comp0+ncomp); 1: volume fraction of the
 // deposited volume; 2: particles per cell (one-to-one bins).  The source
 // records are indexed by original index, or by sorted index with by_sorted

@@ -91,8 +91,9 @@ int grid_capped(int64_t n, int block) {
 
 __global__ void k_aos_unpack(const uint8_t *__restrict__ aos, AosLayout lay,
                              int64_t n, const int32_t *__restrict__ col,
-                             const BoxGeom *__restrict__ boxes, StaticArrays st,
-                             DynArrays dy, unsigned long long *stats) {
+                             const BoxGeom *__restrict__ boxes, BoxGeom g0,
+                             StaticArrays st, DynArrays dy,
+                             unsigned long long *stats) {
   __shared__ double shd[16];
   __shared__ unsigned long long shu[16];
   int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -103,7 +104,8 @@ __global__ void k_aos_unpack(const uint8_t *__restrict__ aos, AosLayout lay,
   const double *pos = reinterpret_cast<const double *>(r + lay.pos);
   const double *rd = reinterpret_cast<const double *>(r + lay.rdata);
   const int32_t *id = reinterpret_cast<const int32_t *>(r + lay.idata);
-  const BoxGeom &g = boxes[col ? col[t] : 0];
+  BoxGeom g = g0;
+  if (col) g = boxes[col[t]];
   double x = wrap_axis(pos[0], g.plo[0], g.phi[0], g.L[0], g.periodic[0]);
   double y = wrap_axis(pos[1], g.plo[1], g.phi[1], g.L[1], g.periodic[1]);
   double z = wrap_axis(pos[2], g.plo[2], g.phi[2], g.L[2], g.periodic[2]);
@@ -168,8 +170,8 @@ __global__ void k_aos_unpack(const uint8_t *__restrict__ aos, AosLayout lay,
 // arrays and everything not selected are kept.  stats as in k_aos_unpack
 // (maxima over the particles after the update, bad records).
 __global__ void k_aos_refresh(const uint8_t *__restrict__ aos, AosLayout lay,
-                              int64_t n, const BoxGeom *__restrict__ boxes,
-                              StaticArrays st, DynArrays dy, uint32_t fields,
+                              int64_t n, BoxGeom g, StaticArrays st,
+                              DynArrays dy, uint32_t fields,
                               unsigned long long *stats) {
   __shared__ double shd[16];
   __shared__ unsigned long long shu[16];
@@ -182,7 +184,6 @@ __global__ void k_aos_refresh(const uint8_t *__restrict__ aos, AosLayout lay,
     const double *pos = reinterpret_cast<const double *>(r + lay.pos);
     const double *rd = reinterpret_cast<const double *>(r + lay.rdata);
     const int32_t *id = reinterpret_cast<const int32_t *>(r + lay.idata);
-    const BoxGeom &g = boxes[st.col ? st.col[t] : 0];
     double4 p = dy.pos[t];
     if (fields & kFieldPositions) {
       p.x = wrap_axis(pos[0], g.plo[0], g.phi[0], g.L[0], g.periodic[0]);
@@ -1123,28 +1124,6 @@ __global__ __launch_bounds__(256, 8) void k_build_rows(
   }
 }
 
-// Reduces the per-block row statistics of the last build.
-__global__ __launch_bounds__(1024) void k_reduce_rowstats(
-    const int32_t *__restrict__ bstats, int32_t nblk,
-    int32_t *__restrict__ stats, unsigned long long *__restrict__ total) {
-  __shared__ int32_t shi[16];
-  __shared__ unsigned long long shu[16];
-  int m = 0;
-  unsigned long long sm = 0;
-  for (int b = threadIdx.x; b < nblk; b += blockDim.x) {
-    int v = bstats[2 * b];
-    m = v > m ? v : m;
-    sm += (unsigned long long)bstats[2 * b + 1];
-  }
-  m = block_max(m, shi);
-  __syncthreads();
-  sm = block_sum(sm, shu);
-  if (threadIdx.x == 0) {
-    stats[0] = m;
-    *total = sm;
-  }
-}
-
 // ------------------------------------------------------- force + update ---
 
 // Separation of two spheres along the axes, with the image test of sep_m.
@@ -1967,20 +1946,20 @@ hipError_t launch_fill_u64(unsigned long long *p, int64_t n,
 
 hipError_t launch_aos_unpack(const uint8_t *aos, AosLayout lay, int64_t n,
                              const int32_t *col, const BoxGeom *boxes,
-                             StaticArrays st, DynArrays dy,
+                             BoxGeom g0, StaticArrays st, DynArrays dy,
                              unsigned long long *stats, hipStream_t s) {
   if (n <= 0) return hipSuccess;
   hipLaunchKernelGGL(k_aos_unpack, dim3(grid_for(n, 256)), dim3(256), 0, s,
-                     aos, lay, n, col, boxes, st, dy, stats);
+                     aos, lay, n, col, boxes, g0, st, dy, stats);
   return hipGetLastError();
 }
 hipError_t launch_aos_refresh(const uint8_t *aos, AosLayout lay, int64_t n,
-                              const BoxGeom *boxes, StaticArrays st,
-                              DynArrays dy, uint32_t fields,
-                              unsigned long long *stats, hipStream_t s) {
+                              BoxGeom g, StaticArrays st, DynArrays dy,
+                              uint32_t fields, unsigned long long *stats,
+                              hipStream_t s) {
   if (n <= 0) return hipSuccess;
   hipLaunchKernelGGL(k_aos_refresh, dim3(grid_for(n, 256)), dim3(256), 0, s,
-                     aos, lay, n, boxes, st, dy, fields, stats);
+                     aos, lay, n, g, st, dy, fields, stats);
   return hipGetLastError();
 }
 
@@ -2142,15 +2121,16 @@ hipError_t launch_build_nbr(const double4 *pos, const int32_t *col,
 }
 
 
-// The tail of a call in one launch: the row statistics of the last build
-// (nblk > 0), then the error word (OR-ed in: calls enqueued back to back
-// add up until the host reads and clears it), the longest row and the entry
-// total written straight into host memory mapped for the device (out: 4
-// words), and the device's error word cleared.
+// The tail of a call in one launch: the row statistics of a build since the
+// last one (nblk > 0), then the error word (add: OR-ed in, so that calls
+// enqueued back to back add up until the host reads and clears it), the
+// longest row and the entry total (out: 4 words, in host memory mapped for
+// the device where there is such memory), and the device's error word
+// cleared.
 __global__ __launch_bounds__(1024) void k_flags_out(
     const int32_t *__restrict__ bstats, int32_t nblk,
     int32_t *__restrict__ stats, unsigned long long *__restrict__ total,
-    int32_t *__restrict__ err, int32_t *__restrict__ out) {
+    int32_t *__restrict__ err, int32_t *__restrict__ out, int add) {
   __shared__ int32_t shi[16];
   __shared__ unsigned long long shu[16];
   if (nblk > 0) {
@@ -2171,7 +2151,7 @@ __global__ __launch_bounds__(1024) void k_flags_out(
   }
   if (threadIdx.x == 0) {
     const unsigned long long tot = *total;
-    out[0] |= *err;  // the host clears the word when it reads it
+    out[0] = add ? out[0] | *err : *err;
     out[1] = stats[0];
     out[2] = (int32_t)(uint32_t)(tot & 0xffffffffull);
     out[3] = (int32_t)(uint32_t)(tot >> 32);
@@ -2179,19 +2159,32 @@ __global__ __launch_bounds__(1024) void k_flags_out(
   }
 }
 
-hipError_t launch_flags_out(const int32_t *bstats, int32_t nblk, int32_t *stats,
-                            unsigned long long *total, int32_t *err,
-                            int32_t *host_out, hipStream_t s) {
-  hipLaunchKernelGGL(k_flags_out, dim3(1), dim3(1024), 0, s, bstats, nblk,
-                     stats, total, err, host_out);
+// The error word of a mesh call, cleared behind it, and (maxima) the two
+// size maxima of the chemistry, into mapped host memory.
+__global__ void k_mesh_out(int32_t *__restrict__ err,
+                           const unsigned long long *__restrict__ maxima,
+                           int32_t *__restrict__ out_err,
+                           unsigned long long *__restrict__ out_max) {
+  out_err[0] = *err;
+  *err = 0;
+  if (maxima) {
+    out_max[0] = maxima[0];
+    out_max[1] = maxima[1];
+  }
+}
+hipError_t launch_mesh_out(int32_t *err, const unsigned long long *maxima,
+                           int32_t *out_err, unsigned long long *out_max,
+                           hipStream_t s) {
+  hipLaunchKernelGGL(k_mesh_out, dim3(1), dim3(1), 0, s, err, maxima, out_err,
+                     out_max);
   return hipGetLastError();
 }
 
-hipError_t launch_reduce_rowstats(const int32_t *bstats, int32_t nblk,
-                                  int32_t *stats, unsigned long long *total,
-                                  hipStream_t s) {
-  hipLaunchKernelGGL(k_reduce_rowstats, dim3(1), dim3(1024), 0, s, bstats,
-                     nblk, stats, total);
+hipError_t launch_flags_out(const int32_t *bstats, int32_t nblk, int32_t *stats,
+                            unsigned long long *total, int32_t *err,
+                            int32_t *out, int add, hipStream_t s) {
+  hipLaunchKernelGGL(k_flags_out, dim3(1), dim3(nblk > 0 ? 1024 : kWave), 0, s,
+                     bstats, nblk, stats, total, err, out, add);
   return hipGetLastError();
 }
 

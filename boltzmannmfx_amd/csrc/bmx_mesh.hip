@@ -54,8 +54,10 @@ template <int TRI>
 __global__ __launch_bounds__(256) void k_mesh_key(
     const double4 *__restrict__ pos, int64_t n, MeshGeom g,
     int32_t *__restrict__ key, int32_t *__restrict__ rank,
-    int32_t *__restrict__ count, int32_t *__restrict__ err) {
+    int32_t *__restrict__ count, int32_t *__restrict__ err,
+    unsigned long long *__restrict__ clear2) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (clear2 && t < 2) clear2[t] = 0ull;
   int32_t k = -1;
   if (t < n) {
     const double4 p = pos[t];
@@ -606,20 +608,20 @@ hipError_t launch_mesh_bin(const double4 *pos, const int32_t *oid, int64_t n,
                            const MeshGeom &g, int tri, int32_t *key,
                            int32_t *rank, int32_t *count, int32_t *start,
                            int32_t *scan_scratch, unsigned long long *perm,
-                           int sorted, int32_t *err, hipStream_t s) {
+                           int sorted, int32_t *err,
+                           unsigned long long *clear2, hipStream_t s) {
   int64_t nb = 1;
   for (int d = 0; d < 3; d++)
     nb *= (tri && !g.periodic[d]) ? g.n[d] + 1 : g.n[d];
-  hipError_t e = launch_fill_i32(count, nb, 0, s);
+  // (launched without particles too, for clear2)
+  if (tri)
+    hipLaunchKernelGGL(k_mesh_key<1>, dim3(grid_of(n)), dim3(256), 0, s, pos, n,
+                       g, key, rank, count, err, clear2);
+  else
+    hipLaunchKernelGGL(k_mesh_key<0>, dim3(grid_of(n)), dim3(256), 0, s, pos, n,
+                       g, key, rank, count, err, clear2);
+  hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  if (n > 0) {
-    if (tri)
-      hipLaunchKernelGGL(k_mesh_key<1>, dim3(grid_of(n)), dim3(256), 0, s, pos,
-                         n, g, key, rank, count, err);
-    else
-      hipLaunchKernelGGL(k_mesh_key<0>, dim3(grid_of(n)), dim3(256), 0, s, pos,
-                         n, g, key, rank, count, err);
-  }
   e = launch_scan(count, start, nb, scan_scratch, s);
   if (e != hipSuccess) return e;
   if (!sorted || n <= 0) return hipGetLastError();

@@ -308,3 +308,29 @@ def test_negative_fluid_concentration_is_an_error(bmx, oracle, gpu):
         ctx.txfr_particle(CHEMPAR, X, vf, 0.25, 4)
     assert e.value.code == 12
     ctx.close()
+
+
+def test_alternating_schemes_and_an_error_between(bmx, oracle, gpu):
+    """The cell counts a call leaves behind serve the next one: calls of both
+    schemes in turn, and after a call that failed on a particle outside the
+    mesh."""
+    col = spheres(seed=6)
+    ctx, grecs, g = setup(bmx, oracle, col)
+    for scheme in (0, 1, 1, 0, 1):
+        want, _ = oracle.volume_fraction(grecs, g, scheme)
+        assert np.array_equal(ctx.volume_fraction(scheme), want)
+    z = grecs["pos"][5, 2]
+    grecs["pos"][5, 2] = col.prob_hi[2] + 1e-4
+    ctx.refresh(bmx.FIELD_POSITIONS)
+    for scheme in (1, 0):
+        with pytest.raises(bmx.BMXError) as e:
+            ctx.volume_fraction(scheme)
+        assert e.value.code == 11
+    grecs["pos"][5, 2] = z
+    ctx.refresh(bmx.FIELD_POSITIONS)
+    for scheme in (0, 1):
+        want, _ = oracle.volume_fraction(grecs, g, scheme)
+        assert np.array_equal(ctx.volume_fraction(scheme), want)
+    want, _ = oracle.count_per_cell(grecs, g)
+    assert np.array_equal(ctx.count_per_cell(), want)
+    ctx.close()

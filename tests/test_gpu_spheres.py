@@ -332,3 +332,29 @@ def test_guard_takes_violating_periods_again(bmx, gpu):
     assert moved > 1e-9                # the skin was exceeded many times over
     for c in (g, every, sten):
         c.close()
+
+
+def test_row_statistics_follow_every_kind_of_call(bmx, gpu):
+    """The entry count and the longest row are those of the last build, after
+    eager, asynchronous and replayed steps that built rows and after steps
+    that kept them."""
+    col = W.sphere_colony(3000, 0.3, 3, W_A=5e-5, skin=2e-5)
+    ctx, _ = gpu_ctx(bmx, col, K=4)
+
+    def check():
+        off, _ = ctx.neighbors()
+        t = ctx.timing()
+        assert (t.neighbor_entries, t.max_row) == (off[-1], np.diff(off).max())
+
+    ctx.evolve(W.DT, 1)
+    check()
+    ctx.evolve(W.DT, 2)       # keeps the rows
+    check()
+    for _ in range(3):        # the second call builds
+        ctx.evolve_async(W.DT, 1)
+    ctx.wait()
+    check()
+    for _ in range(3):        # capture, then replays
+        ctx.evolve_graph(40 * W.DT, 4)
+        check()
+    ctx.close()
