@@ -504,8 +504,10 @@ bmx_status close_run(bmx_ctx *c) {
 // in force, the displacements since that list was built are checked against
 // skin/2 first and their partials cleared, so every caller that rebuilds
 // (steps, exchange, fusion, InitBonds) starts the next period from zero.
-// check_skin = false is for passes that repeat checked arithmetic.
-bmx_status rebuild(bmx_ctx *c, bool check_skin = true) {
+// check_skin = false is for passes that repeat checked arithmetic.  The rows
+// and their lengths go to the context's arrays, or to those given.
+bmx_status rebuild(bmx_ctx *c, bool check_skin = true,
+                   const FlatRows *rows = nullptr, int32_t *ncnt = nullptr) {
   hipStream_t s = c->stream;
   if (c->timing) {
     bmx_status st = close_run(c);
@@ -550,8 +552,9 @@ bmx_status rebuild(bmx_ctx *c, bool check_skin = true) {
                           multi, c->any_fungi ? 1 : 0, c->d_start.p, st.key,
                           c->n, c->nbp.mode == BMX_NBR_STENCIL ? 1 : 0,
                           c->crit, c->fpar[0], c->nbp.skin, c->d_nbr.p,
-                          c->d_ncnt.p, c->ncap, c->maxn, c->d_err.p,
-                          c->d_bstats.p, flat_rows(c), c->lp.xcd_remap, s));
+                          ncnt ? ncnt : c->d_ncnt.p, c->ncap, c->maxn, c->d_err.p,
+                          c->d_bstats.p, rows ? *rows : flat_rows(c),
+                          c->lp.xcd_remap, s));
   c->row_nblk = tile_count(c->n, c->flat_tile);
   if (c->timing) {
     HIPCHK(hipEventRecord(e1, s));
@@ -1814,26 +1817,23 @@ bmx_status bmx_adjoint(bmx_ctx *c, double dt, int32_t nsteps,
         if (t > 0)
           HIPCHK(hipMemcpyAsync(c->pos[c->cd].p, H.pos.p + (size_t)t * cap,
                                 sizeof(double4) * cap, hipMemcpyDeviceToDevice, s));
-        st = rebuild(c, false);
+        // the rows straight into the history
+        const int r = t / K;
+        const FlatRows rows{c->flat_tile, H.idx.p + (size_t)r * rowbuf,
+                            H.own.p + (size_t)r * rowbuf,
+                            H.tot.p + (size_t)r * tilebuf, c->d_roff.p};
+        st = rebuild(c, false, &rows, H.cnt.p + (size_t)r * cap);
         if (st != BMX_OK) return st;
         HIPCHK(hipMemcpyAsync(H.pos.p + (size_t)t * cap, c->pos[c->cd].p,
                               sizeof(double4) * cap, hipMemcpyDeviceToDevice, s));
-        const int r = t / K;
-        HIPCHK(hipMemcpyAsync(H.idx.p + (size_t)r * rowbuf, c->d_cidx.p,
-                              sizeof(int32_t) * rowbuf, hipMemcpyDeviceToDevice, s));
-        HIPCHK(hipMemcpyAsync(H.own.p + (size_t)r * rowbuf, c->d_cown.p, rowbuf,
-                              hipMemcpyDeviceToDevice, s));
-        HIPCHK(hipMemcpyAsync(H.tot.p + (size_t)r * tilebuf, c->d_wtot.p,
-                              sizeof(int32_t) * tilebuf, hipMemcpyDeviceToDevice, s));
-        HIPCHK(hipMemcpyAsync(H.cnt.p + (size_t)r * cap, c->d_ncnt.p,
-                              sizeof(int32_t) * cap, hipMemcpyDeviceToDevice, s));
         HIPCHK(hipMemcpyAsync(H.oid.p + (size_t)r * cap, c->oid[c->cs].p,
                               sizeof(int32_t) * cap, hipMemcpyDeviceToDevice, s));
       }
       if (t + 1 < len)  // the last state of the segment is not needed
         HIPCHK(launch_force_sphere_flat(
             H.pos.p + (size_t)t * cap, H.pos.p + (size_t)(t + 1) * cap,
-            c->d_cidx.p, c->d_cown.p, c->d_wtot.p, c->d_ncnt.p, c->n,
+            H.idx.p + (size_t)(t / K) * rowbuf, H.own.p + (size_t)(t / K) * rowbuf,
+            H.tot.p + (size_t)(t / K) * tilebuf, H.cnt.p + (size_t)(t / K) * cap, c->n,
             c->flat_tile, c->maxn, nullptr, c->d_boxes.p, c->boxes[0], 0, fp, nullptr,
             nullptr, nullptr, c->d_err.p, shape(c), s));
     }
