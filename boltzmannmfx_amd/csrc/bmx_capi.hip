@@ -177,7 +177,13 @@ struct bmx_ctx {
   int64_t step = 0, last_build = -1;
 
   // outputs and flags
-  DevBuf<double> d_fc;  // last step's fc: original order, 6 per particle
+  // last step's fc, 6 per particle.  Segment steps write d_fc in original
+  // order; sphere steps in the order of the step, oid[fc_cs] (a rebuild leaves
+  // that order standing, the one after it does not), until keep_fc puts it
+  // into d_fco in original order
+  DevBuf<double> d_fc, d_fco;
+  int fc_cs = 0;
+  bool fc_orig = false;  // in original order: d_fco for spheres
   bool wrote_step = false;
   DevBuf<int32_t> d_err, d_stats, d_bstats;
   DevBuf<unsigned long long> d_total, d_ustats;
@@ -567,6 +573,25 @@ bmx_status rebuild(bmx_ctx *c, bool check_skin = true,
 }
 
 
+// The last step's fc into original order, if the particles are no longer in
+// the order it was written in: before a reader, and before a second reorder
+// that no step of the same call follows.  always: also when they still are
+// (several reorders follow).
+bmx_status keep_fc(bmx_ctx *c, bool always = false) {
+  if (!c->wrote_step || c->fc_orig || (!always && c->fc_cs == c->cs)) return BMX_OK;
+  HIPCHK(c->d_fco.alloc(6 * (size_t)c->ncap));
+  HIPCHK(launch_fc_to_orig(c->d_fc.p, c->oid[c->fc_cs].p, c->n, c->d_fco.p, c->stream));
+  c->fc_orig = true;
+  return BMX_OK;
+}
+
+// The array that holds the last step's fc.
+const double *fc_now(const bmx_ctx *c) {
+  return c->fc_orig && !c->any_fungi ? c->d_fco.p : c->d_fc.p;
+}
+
+// A step that rebuilds reorders the particles; the call's last step writes fc
+// anew (write_fc).
 bmx_status enqueue_step(bmx_ctx *c, double dt, bool write_fc) {
   hipStream_t s = c->stream;
   bool need = !c->have_list ||
@@ -592,7 +617,7 @@ bmx_status enqueue_step(bmx_ctx *c, double dt, bool write_fc) {
         c->pos[c->cd].p, c->pos[1 - c->cd].p, c->d_cidx.p, c->d_cown.p,
         c->d_wtot.p, c->d_ncnt.p, c->n, c->flat_tile, c->maxn,
         multi ? c->col[c->cs].p : nullptr, c->d_boxes.p, c->boxes[0], multi,
-        fp, fc, c->oid[c->cs].p, vm, c->d_err.p, shape(c), s));
+        fp, fc, vm, c->d_err.p, shape(c), s));
   } else {
     // the next step reads what this one leaves only where it keeps the list
     DynArrays next = dyn_arrays(c, 1 - c->cd);
@@ -605,7 +630,13 @@ bmx_status enqueue_step(bmx_ctx *c, double dt, bool write_fc) {
   if (c->timing) c->run_n++;
   c->cd = 1 - c->cd;
   c->step++;
-  if (write_fc) c->wrote_step = true;
+  if (write_fc) {
+    c->wrote_step = true;
+    c->fc_orig = c->any_fungi;
+    c->fc_cs = c->cs;
+  } else if (need && !c->any_fungi) {
+    c->wrote_step = false;  // until the call's last step
+  }
   return BMX_OK;
 }
 
@@ -620,8 +651,7 @@ bmx_status enqueue_force_only(bmx_ctx *c, double dt, int slot) {
   HIPCHK(launch_force_sphere_flat(
       c->pos[c->cd].p, c->pos[1 - c->cd].p, c->d_cidx.p, c->d_cown.p,
       c->d_wtot.p, c->d_ncnt.p, c->n, c->flat_tile, c->maxn, nullptr, c->d_boxes.p,
-      c->boxes[0], 0, fp, nullptr, nullptr, vm, c->d_err.p, shape(c),
-      c->stream));
+      c->boxes[0], 0, fp, nullptr, vm, c->d_err.p, shape(c), c->stream));
   c->cd = 1 - c->cd;
   c->step++;
   return BMX_OK;
@@ -744,9 +774,12 @@ bmx_status drop_chem(bmx_ctx *c) {
 }
 
 bmx_status pack_records(bmx_ctx *c) {
+  bmx_status st = keep_fc(c);
+  if (st != BMX_OK) return st;
   // the bin ranks are scratch between rebuilds
   HIPCHK(launch_aos_pack(c->recs, c->lay, c->n, static_arrays(c, c->cs),
-                         dyn_arrays(c, c->cd), c->d_fc.p,
+                         dyn_arrays(c, c->cd), fc_now(c),
+                         c->fc_orig ? 1 : 0,
                          c->have_chem ? c->d_chemst[c->cc].p : nullptr,
                          chem_rel(c), c->mobility, c->wrote_step ? 1 : 0,
                          c->any_fungi ? 1 : 0, c->d_rank.p, c->stream));
@@ -996,6 +1029,7 @@ void bmx_ctx_destroy(bmx_ctx *c) {
   c->d_cidx.release();
   c->d_cown.release();
   c->d_fc.release();
+  c->d_fco.release();
   c->d_err.release();
   c->d_stats.release();
   c->d_bstats.release();
@@ -1256,6 +1290,8 @@ bmx_status bmx_init_bonds(bmx_ctx *c) {
   if (st != BMX_OK) return st;
   (void)hipSetDevice(c->device);
   reset_graph(c);
+  st = keep_fc(c);
+  if (st != BMX_OK) return st;
   st = rebuild(c);
   if (st != BMX_OK) return st;
   if (c->any_fungi)
@@ -1685,6 +1721,8 @@ bmx_status bmx_evolve_graph(bmx_ctx *c, double dt, int32_t nsteps) {
     c->step++;
   }
   c->wrote_step = true;
+  c->fc_orig = c->any_fungi;
+  c->fc_cs = c->cs;
   return check_flags(c);
 }
 
@@ -1706,6 +1744,7 @@ bmx_status bmx_adjoint(bmx_ctx *c, double dt, int32_t nsteps,
   (void)hipSetDevice(c->device);
   reset_graph(c);
   st = drop_chem(c);  // the checkpoints hold positions only
+  if (st == BMX_OK) st = keep_fc(c, true);
   if (st != BMX_OK) return st;
   hipStream_t s = c->stream;
   const int64_t n = c->n, cap = c->ncap;
@@ -1835,7 +1874,7 @@ bmx_status bmx_adjoint(bmx_ctx *c, double dt, int32_t nsteps,
             H.idx.p + (size_t)(t / K) * rowbuf, H.own.p + (size_t)(t / K) * rowbuf,
             H.tot.p + (size_t)(t / K) * tilebuf, H.cnt.p + (size_t)(t / K) * cap, c->n,
             c->flat_tile, c->maxn, nullptr, c->d_boxes.p, c->boxes[0], 0, fp, nullptr,
-            nullptr, nullptr, c->d_err.p, shape(c), s));
+            nullptr, c->d_err.p, shape(c), s));
     }
     HIPCHK(hipEventRecord(A.rdone[hs], s));
     HIPCHK(hipStreamWaitEvent(s2, A.rdone[hs], 0));
@@ -1903,9 +1942,13 @@ bmx_status bmx_get_fc(bmx_ctx *c, double *out) {
   if (!out && c->n > 0) return fail(BMX_ERR_BAD_ARG, "null output");
   if (!c->wrote_step) return fail(BMX_ERR_STATE, "no step has run");
   (void)hipSetDevice(c->device);
+  st = keep_fc(c);
+  if (st != BMX_OK) return st;
   DevBuf<double> tmp;
   HIPCHK(tmp.alloc(6 * (size_t)std::max<int64_t>(c->n, 1)));
-  HIPCHK(launch_export_fc(c->d_fc.p, c->n, tmp.p, c->stream));
+  HIPCHK(launch_export_fc(fc_now(c),
+                          c->fc_orig ? nullptr : c->oid[c->cs].p, c->n, tmp.p,
+                          c->stream));
   if (c->n)
     HIPCHK(hipMemcpyAsync(out, tmp.p, sizeof(double) * 6 * c->n,
                           hipMemcpyDeviceToHost, c->stream));
@@ -2091,6 +2134,8 @@ extern "C" bmx_status bmx_exchange(bmx_ctx *c, const double xpar[3], double dt) 
   st = load_chem(c);
   if (st != BMX_OK) return st;
   // the rows are rebuilt at the current positions (xchng.cpp:68-77)
+  st = keep_fc(c);
+  if (st != BMX_OK) return st;
   st = rebuild(c);
   if (st != BMX_OK) return st;
   // only segments exchange
@@ -2676,6 +2721,8 @@ extern "C" bmx_status bmx_fusion(bmx_ctx *c, const bmx_fusion_params *fp,
   hipStream_t s = c->stream;
   reset_graph(c);
   // records and rows at the current positions (EvaluateTipFusion rebuilds)
+  st = keep_fc(c);
+  if (st != BMX_OK) return st;
   st = pack_records(c);
   if (st != BMX_OK) return st;
   st = rebuild(c);

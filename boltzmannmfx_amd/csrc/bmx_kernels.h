@@ -58,10 +58,10 @@ hipError_t launch_aos_refresh(const uint8_t *aos, AosLayout lay, int64_t n,
                               hipStream_t s);
 // sorted SoA -> AoS (fields the force pass writes; with state, the chemistry
 // state's too, and each particle's radius and length); inv: n words of
-// scratch
+// scratch; fc_orig: fc is in original order, else in the sorted one
 hipError_t launch_aos_pack(uint8_t *aos, AosLayout lay, int64_t n,
                            StaticArrays st, DynArrays dy, const double *fc,
-                           const double *state, int has_rel, double mob,
+                           int fc_orig, const double *state, int has_rel, double mob,
                            int wrote_step, int any_fungi, int32_t *inv,
                            hipStream_t s);
 
@@ -119,17 +119,15 @@ hipError_t launch_build_nbr(const double4 *pos, const int32_t *col,
                             int32_t *bstats, FlatRows flat, int remap,
                             hipStream_t s);
 // Sphere force + overdamped update, fused, over the flat row layout.  fc
-// (6*ncap, original order: fc[oid + c*ncap]) is written when non-null,
-// with fc_oid the original index of each sorted row; vmax[tile] receives
-// the tile's max dt*|vel| when non-null.
+// (six doubles per particle, sorted order) is written when non-null;
+// vmax[tile] receives the tile's max dt*|vel| when non-null.
 hipError_t launch_force_sphere_flat(const double4 *pos_in, double4 *pos_out,
                                     const int32_t *cidx, const uint8_t *cown,
                                     const int32_t *wtot, const int32_t *ncnt,
                                     int64_t n, int tile, int32_t maxn,
                                     const int32_t *col,
                                     const BoxGeom *boxes, BoxGeom g0, int multi,
-                                    ForceParams fp, double *fc,
-                                    const int32_t *fc_oid, double *vmax,
+                                    ForceParams fp, double *fc, double *vmax,
                                     int32_t *err, LaunchShape ls,
                                     hipStream_t s);
 // tiles of n particles (at least one)
@@ -147,7 +145,7 @@ hipError_t launch_mesh_out(int32_t *err, const unsigned long long *maxima,
                            hipStream_t s);
 
 // ---- segment (and mixed) force + overdamped update, fused: fc and vmax
-// as for launch_force_sphere_flat.
+// as for launch_force_sphere_flat, but fc in original order.
 hipError_t launch_force_general(DynArrays in, DynArrays out, StaticArrays st,
                                 FlatRows flat, int8_t *redo_tile,
                                 const int32_t *ncnt, int64_t n, int32_t maxn,
@@ -170,8 +168,11 @@ hipError_t launch_skin_check(double *vpart, int32_t nslots, int32_t stride,
                              hipStream_t s);
 
 // ---- exports to original order
-hipError_t launch_export_fc(const double *fc, int64_t n, double *out,
-                            hipStream_t s);
+// (oid: the sorted order fc is in; null: fc is in original order)
+hipError_t launch_export_fc(const double *fc, const int32_t *oid, int64_t n,
+                            double *out, hipStream_t s);
+hipError_t launch_fc_to_orig(const double *fc, const int32_t *oid, int64_t n,
+                             double *out, hipStream_t s);
 hipError_t launch_export_pos(const double4 *pos, const int32_t *oid, int64_t n,
                              double *out, hipStream_t s);
 hipError_t launch_export_orient(const double4 *rod, const int32_t *oid,

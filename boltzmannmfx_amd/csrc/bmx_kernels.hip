@@ -247,23 +247,40 @@ __global__ void k_aos_refresh(const uint8_t *__restrict__ aos, AosLayout lay,
   }
 }
 
-// fc of the last step is kept in original particle order, six doubles per
-// particle (force, then torque) in one 48-byte run: a step that writes it
-// stores three 16-byte pieces per particle where the component-major
-// layout of the export would scatter six 8-byte words.
-__device__ __forceinline__ void store_fc(double *__restrict__ fc, int64_t o,
+// fc of the last step, six doubles per particle (force, then torque) in one
+// 48-byte run at index t.  Sphere steps keep it in the order of the step, so
+// that their stores are whole lines: 307,201 spheres 12.0 us for the pass
+// that writes it and 17.4 for the pack that reads it, against 13.1 and 22.5
+// in original order; 1M spheres with the chemistry state 34 against 48 for
+// the writing pass.  A reorder before its use has it put into the original
+// order (k_fc_to_orig).  Segment steps store it in original order: their
+// passes reorder between a step and its readers (exchange, fusion), and
+// beside the pair law the scattered store does not show.
+__device__ __forceinline__ void store_fc(double *__restrict__ fc, int64_t t,
                                          double f0, double f1, double f2,
                                          double f3, double f4, double f5) {
-  double2 *q = reinterpret_cast<double2 *>(fc + o * 6);
+  double2 *q = reinterpret_cast<double2 *>(fc + t * 6);
   q[0] = make_double2(f0, f1);
   q[1] = make_double2(f2, f3);
   q[2] = make_double2(f4, f5);
 }
+__global__ void k_fc_to_orig(const double *__restrict__ fc,
+                             const int32_t *__restrict__ oid, int64_t n,
+                             double *__restrict__ out) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n) return;
+  const double2 *a = reinterpret_cast<const double2 *>(fc + t * 6);
+  double2 *b = reinterpret_cast<double2 *>(out + (int64_t)oid[t] * 6);
+  const double2 x = a[0], y = a[1], z = a[2];
+  b[0] = x;
+  b[1] = y;
+  b[2] = z;
+}
 
 __global__ void k_aos_pack(uint8_t *__restrict__ aos, AosLayout lay, int64_t n,
                            StaticArrays st, DynArrays dy,
-                           const double *__restrict__ fc, double mob,
-                           int wrote_step, int any_fungi) {
+                           const double *__restrict__ fc, int fc_orig,
+                           double mob, int wrote_step, int any_fungi) {
   int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= n) return;
   int64_t o = st.oid[t];
@@ -276,7 +293,7 @@ __global__ void k_aos_pack(uint8_t *__restrict__ aos, AosLayout lay, int64_t n,
   pos[1] = p.y;
   pos[2] = p.z;
   if (wrote_step) {
-    const double *f = fc + o * 6;  // original order, six per particle
+    const double *f = fc + (fc_orig ? o : t) * 6;
     rd[rec::velx] = mob * f[0];
     rd[rec::vely] = mob * f[1];
     rd[rec::velz] = mob * f[2];
@@ -324,6 +341,7 @@ __global__ void k_inverse(const int32_t *__restrict__ oid, int64_t n,
 // 225 against 332 with the chemistry state.
 struct PackWhat {
   int step;  // a step has run: velocities and flags
+  int fc_orig;  // its fc is in original order
   int rel;   // CHEM: the layout holds the amounts taken from the fluid
 };
 template <bool FUNGI, bool CHEM>
@@ -397,7 +415,7 @@ __global__ __launch_bounds__(kWave) void k_aos_pack_wide(
       v[c++] = a.w;  // vol
     }
     if (what.step) {
-      const double *f = fc + o * 6;  // original order, six per particle
+      const double *f = fc + (what.fc_orig ? o : t) * 6;
       v[c++] = mob * f[0];
       v[c++] = mob * f[1];
       v[c++] = mob * f[2];
@@ -1271,8 +1289,8 @@ __global__ __launch_bounds__(512, 6) void k_force_sphere_flat(
     const int32_t *__restrict__ wtot, const int32_t *__restrict__ ncnt,
     int64_t n, int tsize, int32_t maxn, const int32_t *__restrict__ col,
     const BoxGeom *__restrict__ boxes, BoxGeom g0, ForceParams fp,
-    double *__restrict__ fc, const int32_t *__restrict__ fc_oid,
-    double *__restrict__ vmax, int32_t *__restrict__ err, int remap) {
+    double *__restrict__ fc, double *__restrict__ vmax,
+    int32_t *__restrict__ err, int remap) {
   extern __shared__ __align__(16) unsigned char flat_lds[];
   const int lane = threadIdx.x & (kWave - 1);
   const int wv = threadIdx.x / kWave, nwv = blockDim.x / kWave;
@@ -1363,9 +1381,7 @@ __global__ __launch_bounds__(512, 6) void k_force_sphere_flat(
     y = wrap_axis(y, g.plo[1], g.phi[1], g.L[1], g.periodic[1]);
     z = wrap_axis(z, g.plo[2], g.phi[2], g.L[2], g.periodic[2]);
     pos_out[t] = make_double4(x, y, z, p.w);
-    if (fc) {  // original order, so a later rebuild does not reorder it
-      store_fc(fc, fc_oid[t], a0, a1, a2, 0.0, 0.0, 0.0);
-    }
+    if (fc) store_fc(fc, t, a0, a1, a2, 0.0, 0.0, 0.0);
     if (!(isfinite(a0) && isfinite(a1) && isfinite(a2))) atomicOr(err, ERRBIT_NAN);
     v2 = vx * vx + vy * vy + vz * vz;
   }
@@ -1883,13 +1899,15 @@ __global__ void k_skin_final(unsigned long long *__restrict__ slotmax,
 
 // ------------------------------------------------------------- exports ---
 
-// fc from its kept layout (original order, six per particle) to the
-// reference's component-major fc[i + c * n]
-__global__ void k_export_fc(const double *__restrict__ fc, int64_t n,
+// fc from its kept layout (oid: the order of the step; null: original) to
+// the reference's component-major fc[i + c * n]
+__global__ void k_export_fc(const double *__restrict__ fc,
+                            const int32_t *__restrict__ oid, int64_t n,
                             double *__restrict__ out) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  for (int c = 0; c < 6; c++) out[c * n + i] = fc[i * 6 + c];
+  int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n) return;
+  const int64_t o = oid ? oid[t] : t;
+  for (int c = 0; c < 6; c++) out[c * n + o] = fc[t * 6 + c];
 }
 __global__ void k_export_pos(const double4 *__restrict__ pos,
                              const int32_t *__restrict__ oid, int64_t n,
@@ -1986,19 +2004,19 @@ constexpr int64_t kPackWide = 320ll << 20;
 
 hipError_t launch_aos_pack(uint8_t *aos, AosLayout lay, int64_t n,
                            StaticArrays st, DynArrays dy, const double *fc,
-                           const double *state, int has_rel, double mob,
+                           int fc_orig, const double *state, int has_rel, double mob,
                            int wrote_step, int any_fungi, int32_t *inv,
                            hipStream_t s) {
   if (n <= 0) return hipSuccess;
   if (n * (int64_t)lay.stride <= kPackWide) {
     hipLaunchKernelGGL(k_aos_pack, dim3(grid_for(n, 256)), dim3(256), 0, s, aos,
-                       lay, n, st, dy, fc, mob, wrote_step, any_fungi);
+                       lay, n, st, dy, fc, fc_orig, mob, wrote_step, any_fungi);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || !state) return e;
     return launch_chem_pack(aos, lay, n, has_rel, state, st.oid, st.type, dy.pos,
                             dy.rod, s);
   }
-  const PackWhat what{wrote_step, has_rel};
+  const PackWhat what{wrote_step, fc_orig, has_rel};
   hipLaunchKernelGGL(k_inverse, dim3(grid_for(n, 256)), dim3(256), 0, s, st.oid,
                      n, inv);
 #define BMX_PACK(F, C)                                                        \
@@ -2212,8 +2230,7 @@ hipError_t launch_force_sphere_flat(const double4 *pos_in, double4 *pos_out,
                                     int64_t n, int tile, int32_t maxn,
                                     const int32_t *col,
                                     const BoxGeom *boxes, BoxGeom g0, int multi,
-                                    ForceParams fp, double *fc,
-                                    const int32_t *fc_oid, double *vmax,
+                                    ForceParams fp, double *fc, double *vmax,
                                     int32_t *err, LaunchShape ls,
                                     hipStream_t s) {
   if (n <= 0) return hipSuccess;
@@ -2223,11 +2240,11 @@ hipError_t launch_force_sphere_flat(const double4 *pos_in, double4 *pos_out,
   if (multi)
     hipLaunchKernelGGL(k_force_sphere_flat<true>, dim3(grid), dim3(b), lds, s,
                        pos_in, pos_out, cidx, cown, wtot, ncnt, n, tile, maxn,
-                       col, boxes, g0, fp, fc, fc_oid, vmax, err, ls.remap);
+                       col, boxes, g0, fp, fc, vmax, err, ls.remap);
   else
     hipLaunchKernelGGL(k_force_sphere_flat<false>, dim3(grid), dim3(b), lds, s,
                        pos_in, pos_out, cidx, cown, wtot, ncnt, n, tile, maxn,
-                       col, boxes, g0, fp, fc, fc_oid, vmax, err, ls.remap);
+                       col, boxes, g0, fp, fc, vmax, err, ls.remap);
   return hipGetLastError();
 }
 
@@ -2319,11 +2336,18 @@ hipError_t launch_skin_check(double *vpart, int32_t nslots, int32_t stride,
   return hipGetLastError();
 }
 
-hipError_t launch_export_fc(const double *fc, int64_t n,
+hipError_t launch_fc_to_orig(const double *fc, const int32_t *oid, int64_t n,
+                             double *out, hipStream_t s) {
+  if (n <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_fc_to_orig, dim3(grid_for(n, 256)), dim3(256), 0, s, fc,
+                     oid, n, out);
+  return hipGetLastError();
+}
+hipError_t launch_export_fc(const double *fc, const int32_t *oid, int64_t n,
                             double *out, hipStream_t s) {
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_export_fc, dim3(grid_for(n, 256)), dim3(256), 0, s, fc, n,
-                     out);
+  hipLaunchKernelGGL(k_export_fc, dim3(grid_for(n, 256)), dim3(256), 0, s, fc,
+                     oid, n, out);
   return hipGetLastError();
 }
 hipError_t launch_export_pos(const double4 *pos, const int32_t *oid, int64_t n,

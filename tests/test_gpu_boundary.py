@@ -188,3 +188,43 @@ def test_chained_async_calls(bmx, gpu, col):
     assert ctx.timing().rebuilds_total == 3
     ctx.close()
     ref.close()
+
+
+def test_fc_survives_reorders_after_the_step(bmx, oracle, gpu):
+    """The forces of the last step, and the velocities a sync writes from
+    them, are the same whether they are read at once or after passes that
+    reorder the particles (one exchange, several, bond detection)."""
+    rng = np.random.default_rng(12)
+    for segments in (True, False):
+        col = (W.c3_hyphae(2003, nroots=20, seed=3) if segments
+               else W.sphere_colony(3001, 0.25, 3, skin=2e-5))
+        n = len(col.recs)
+        col.recs["rdata"][:, 5] = 1e-12
+        col.recs["rdata"][:, 25:28] = rng.uniform(0, 2e-5, (n, 3))
+        ctx = bmx.Context(0)
+        ctx.set_force_params(col.fpar)
+        ctx.set_geometry(col.prob_lo, col.prob_hi, col.periodic, col.n_cell)
+        if segments:
+            ctx.set_neighbor_params(mode=bmx.NBR_STENCIL, rebuild_every=1,
+                                    neighborhood=1.1 * (4e-4 + 1e-2), max_neighbors=256)
+        else:
+            ctx.set_neighbor_params(mode=bmx.NBR_VERLET, rebuild_every=10, skin=col.skin)
+        recs = col.recs.copy()
+        ctx.bind(recs)
+        ctx.evolve((100 if segments else 1) * col.dt, 3)
+        fc = ctx.fc()
+        ctx.sync()
+        vel = recs["rdata"][:, 6:12].copy()
+        assert np.abs(fc[:3]).max() > 0 and np.array_equal(vel, fc.T)
+        passes = [lambda: ctx.exchange([0.0] * 3, 1.0)] * 3
+        passes.append(ctx.init_bonds)
+        for k, call in enumerate(passes):
+            call()
+            assert np.array_equal(ctx.fc(), fc), k
+        recs["rdata"][:, 6:12] = 0.0
+        ctx.exchange([0.0] * 3, 1.0)
+        ctx.sync()
+        assert np.array_equal(recs["rdata"][:, 6:12], vel)
+        ctx.evolve(col.dt, 1)
+        assert not np.array_equal(ctx.fc(), fc)
+        ctx.close()
