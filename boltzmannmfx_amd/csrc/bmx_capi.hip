@@ -634,7 +634,7 @@ bmx_status enqueue_step(bmx_ctx *c, double dt, bool write_fc) {
     c->wrote_step = true;
     c->fc_orig = c->any_fungi;
     c->fc_cs = c->cs;
-  } else if (need && !c->any_fungi) {
+  } else if (need && !c->fc_orig) {
     c->wrote_step = false;  // until the call's last step
   }
   return BMX_OK;
@@ -1417,6 +1417,10 @@ bmx_status evolve_guarded(bmx_ctx *c, double dt, int32_t nsteps) {
   {
     // the snapshots hold the particle arrays only
     bmx_status sc = drop_chem(c);
+    if (sc != BMX_OK) return sc;
+    // an error in an early period ends the call before the step that writes
+    // fc, which then still is the call before's
+    if (nsteps > K) sc = keep_fc(c, true);
     if (sc != BMX_OK) return sc;
   }
   for (auto &z : c->gsnap)

@@ -228,3 +228,31 @@ def test_fc_survives_reorders_after_the_step(bmx, oracle, gpu):
         ctx.evolve(col.dt, 1)
         assert not np.array_equal(ctx.fc(), fc)
         ctx.close()
+
+
+def test_fc_of_the_call_before_a_failed_guarded_call(bmx, gpu):
+    """A guarded call that ends in its first period (a row over the capacity)
+    has not reached the step that writes the forces: those of the call before
+    are still there, in their particles' order."""
+    col = W.sphere_colony(3001, 0.25, 3, skin=2e-5)
+    ctx = bmx.Context(0)
+    ctx.set_force_params(col.fpar)
+    ctx.set_geometry(col.prob_lo, col.prob_hi, col.periodic, col.n_cell)
+    ctx.set_neighbor_params(mode=bmx.NBR_VERLET, rebuild_every=10, skin=col.skin,
+                            max_neighbors=24)
+    ctx.set_guard(True)
+    recs = col.recs.copy()
+    ctx.bind(recs)
+    dt = 1e-9 * col.dt
+    ctx.evolve(dt, 25)
+    fc = ctx.fc()
+    rng = np.random.default_rng(5)
+    recs["pos"] = recs["pos"][rng.permutation(len(recs))]
+    mid = 0.5 * (np.asarray(col.prob_lo) + np.asarray(col.prob_hi))
+    recs["pos"][:40] = mid + rng.uniform(-1e-5, 1e-5, (40, 3))
+    ctx.refresh(bmx.FIELD_POSITIONS, recs)
+    with pytest.raises(bmx.BMXError) as e:
+        ctx.evolve(dt, 45)
+    assert e.value.code == 5                          # a row over the capacity
+    assert np.array_equal(ctx.fc(), fc)
+    ctx.close()
