@@ -334,3 +334,27 @@ def test_alternating_schemes_and_an_error_between(bmx, oracle, gpu):
     want, _ = oracle.count_per_cell(grecs, g)
     assert np.array_equal(ctx.count_per_cell(), want)
     ctx.close()
+
+
+@pytest.mark.parametrize("scheme", [0, 1])
+def test_deposition_of_cells_with_few_and_many_particles(bmx, oracle, gpu, scheme):
+    """Cells of 0 to 19 particles (none, one, the edges of a batch of loads),
+    in shuffled order: volume fractions and fluid increments bit for bit."""
+    col = spheres()
+    nx, ny, nz = col.n_cell
+    lo, hi = np.asarray(col.prob_lo), np.asarray(col.prob_hi)
+    dx = (hi - lo) / np.array(col.n_cell)
+    rng = np.random.default_rng(8)
+    inner = rng.permutation(np.arange(nx * ny, nx * ny * (nz - 1)))
+    cells = [c for k, c in enumerate(inner[:190]) for _ in range(k % 20)]
+    col.recs = col.recs[:len(cells)].copy()
+    rng.shuffle(cells)
+    c = np.array(cells)
+    ijk = np.stack([c % nx, c // nx % ny, c // (nx * ny)], 1)
+    col.recs["pos"] = lo + (ijk + rng.uniform(0.05, 0.95, ijk.shape)) * dx
+    ctx, grecs, g = setup(bmx, oracle, col)
+    ovf, out = oracle.volume_fraction(grecs, g, scheme)
+    assert out == 0 and np.array_equal(ctx.volume_fraction(scheme), ovf)
+    orhs, _ = oracle.deposit(grecs, g, scheme, 31, 3)
+    assert np.array_equal(ctx.txfr_fluid(scheme), orhs)
+    ctx.close()
