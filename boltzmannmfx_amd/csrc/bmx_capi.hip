@@ -1665,11 +1665,12 @@ bmx_status bmx_evolve_graph(bmx_ctx *c, double dt, int32_t nsteps) {
                c->graph_nsteps == nsteps && c->graph_cs == c->cs &&
                c->graph_cd == c->cd && c->graph_step0 == phase &&
                c->graph_have_list == c->have_list;
-  int cs0 = c->cs, cd0 = c->cd;
+  int cs0 = c->cs, cd0 = c->cd, cc0 = c->cc;
   bool hl0 = c->have_list;
   if (!reuse) {
     reset_graph(c);
     int64_t save_step = c->step, save_last = c->last_build;
+    int64_t save_rebuilds = c->rebuilds_total;
     bool save_wrote = c->wrote_step;
     HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     bmx_status cst = BMX_OK;
@@ -1705,6 +1706,8 @@ bmx_status bmx_evolve_graph(bmx_ctx *c, double dt, int32_t nsteps) {
     c->wrote_step = save_wrote;
     c->cs = cs0;
     c->cd = cd0;
+    c->cc = cc0;  // a rebuild moves the chemistry state as well
+    c->rebuilds_total = save_rebuilds;
     c->have_list = hl0;
   }
   HIPCHK(hipGraphLaunch(c->graph_exec, c->stream));

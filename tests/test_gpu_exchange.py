@@ -71,6 +71,36 @@ def test_exchange_matches_oracle(bmx, oracle, gpu, mode, K, block):
     ctx.close()
 
 
+@pytest.mark.parametrize("mode,K,steps", [(1, 1, 4), (0, 10, 12)])
+def test_graph_steps_keep_each_particle_its_species(bmx, gpu, mode, K, steps):
+    """Graph replays with the chemistry state loaded move it with the
+    particles: as the same steps taken eagerly, after each of several replays
+    with an odd number of row builds (the capture included)."""
+    col = mat(seed=29)
+    ends = []
+    for graph in (False, True):
+        ctx = bmx.Context(0)
+        ctx.set_force_params(col.fpar)
+        ctx.set_geometry(col.prob_lo, col.prob_hi, col.periodic, col.n_cell)
+        ctx.set_neighbor_params(mode=mode, rebuild_every=K, skin=col.skin,
+                                neighborhood=HOOD, max_neighbors=384)
+        recs = col.recs.copy()
+        ctx.bind(recs)
+        ctx.init_bonds()
+        got = []
+        for _ in range(3):
+            ctx.exchange(XPAR, 1.0)  # loads the state; rows built here
+            (ctx.evolve_graph if graph else ctx.evolve)(col.dt, steps)
+            ctx.sync()
+            got.append([recs[f].copy() for f in ("pos", "rdata", "idata")] +
+                       [ctx.timing().rebuilds_total])
+        ends.append(got)
+        ctx.close()
+    for eager, replayed in zip(*ends):
+        for a, b in zip(eager, replayed):
+            assert np.array_equal(a, b)
+
+
 def test_exchange_conserves_species_with_symmetric_rows(bmx, gpu):
     """Verlet rows are symmetric and hold every bonded pair, so each flux
     leaves one segment and enters the other: sum(vol * c) is conserved."""
