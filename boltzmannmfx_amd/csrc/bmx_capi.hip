@@ -640,6 +640,32 @@ bmx_status enqueue_step(bmx_ctx *c, double dt, bool write_fc) {
   return BMX_OK;
 }
 
+// What enqueue_step changes on the host beside the launches it enqueues.
+struct StepMark {
+  int64_t step, last_build, rebuilds_total;
+  int cs, cd, cc, fc_cs;
+  int32_t row_nblk;
+  bool have_list, count_clear, wrote_step, fc_orig;
+};
+StepMark step_mark(const bmx_ctx *c) {
+  return {c->step, c->last_build, c->rebuilds_total, c->cs, c->cd, c->cc, c->fc_cs,
+          c->row_nblk, c->have_list, c->count_clear, c->wrote_step, c->fc_orig};
+}
+void step_restore(bmx_ctx *c, const StepMark &m) {
+  c->step = m.step;
+  c->last_build = m.last_build;
+  c->rebuilds_total = m.rebuilds_total;
+  c->cs = m.cs;
+  c->cd = m.cd;
+  c->cc = m.cc;
+  c->fc_cs = m.fc_cs;
+  c->row_nblk = m.row_nblk;
+  c->have_list = m.have_list;
+  c->count_clear = m.count_clear;
+  c->wrote_step = m.wrote_step;
+  c->fc_orig = m.fc_orig;
+}
+
 // One force launch without bookkeeping of rebuilds (the adjoint drives its
 // own rebuild schedule).  slot >= 0 records the step's displacement
 // partials for the skin check in that slot.
@@ -1665,13 +1691,9 @@ bmx_status bmx_evolve_graph(bmx_ctx *c, double dt, int32_t nsteps) {
                c->graph_nsteps == nsteps && c->graph_cs == c->cs &&
                c->graph_cd == c->cd && c->graph_step0 == phase &&
                c->graph_have_list == c->have_list;
-  int cs0 = c->cs, cd0 = c->cd, cc0 = c->cc;
-  bool hl0 = c->have_list;
   if (!reuse) {
     reset_graph(c);
-    int64_t save_step = c->step, save_last = c->last_build;
-    int64_t save_rebuilds = c->rebuilds_total;
-    bool save_wrote = c->wrote_step;
+    const StepMark before = step_mark(c);
     HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     bmx_status cst = BMX_OK;
     for (int32_t k = 0; k < nsteps && cst == BMX_OK; k++)
@@ -1682,6 +1704,9 @@ bmx_status bmx_evolve_graph(bmx_ctx *c, double dt, int32_t nsteps) {
                               c->d_err.p, c->stream);
     hipGraph_t g = nullptr;
     hipError_t e = hipStreamEndCapture(c->stream, &g);
+    // capture recorded the launches without running them: the bookkeeping
+    // goes back to where it was, whatever the capture came to
+    step_restore(c, before);
     if (cst != BMX_OK) {
       if (g) (void)hipGraphDestroy(g);
       return cst;
@@ -1695,20 +1720,10 @@ bmx_status bmx_evolve_graph(bmx_ctx *c, double dt, int32_t nsteps) {
                   std::string("instantiate: ") + hipGetErrorString(e));
     c->graph_dt = dt;
     c->graph_nsteps = nsteps;
-    c->graph_cs = cs0;
-    c->graph_cd = cd0;
+    c->graph_cs = c->cs;
+    c->graph_cd = c->cd;
     c->graph_step0 = phase;
-    c->graph_have_list = hl0;
-    // capture recorded the launches without running them: restore the
-    // bookkeeping to the pre-capture state, then replay below
-    c->step = save_step;
-    c->last_build = save_last;
-    c->wrote_step = save_wrote;
-    c->cs = cs0;
-    c->cd = cd0;
-    c->cc = cc0;  // a rebuild moves the chemistry state as well
-    c->rebuilds_total = save_rebuilds;
-    c->have_list = hl0;
+    c->graph_have_list = c->have_list;
   }
   HIPCHK(hipGraphLaunch(c->graph_exec, c->stream));
   // advance bookkeeping exactly as the eager loop would
@@ -1720,6 +1735,7 @@ bmx_status bmx_evolve_graph(bmx_ctx *c, double dt, int32_t nsteps) {
       c->cd = 1 - c->cd;
       if (c->have_chem) c->cc = 1 - c->cc;
       c->have_list = true;
+      c->count_clear = true;
       c->last_build = c->step;
       c->row_nblk = tile_count(c->n, c->flat_tile);
       c->rebuilds_total++;

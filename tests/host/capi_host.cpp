@@ -8,6 +8,7 @@
 
 #include <cstdlib>
 #include <functional>
+#include <tuple>
 
 namespace sim {
 bool capturing = false;
@@ -240,6 +241,13 @@ void check_buffers(bmx_ctx *c) {
   if (c->have_list) CHECK(c->d_cidx.p == sim::rows);
 }
 
+// What a step changes on the host.
+auto bookkeeping(const bmx_ctx *c) {
+  return std::make_tuple(c->step, c->last_build, c->rebuilds_total, c->row_nblk, c->cs,
+                         c->cd, c->cc, c->have_list, c->count_clear, c->wrote_step,
+                         c->fc_orig, c->fc_cs);
+}
+
 const double kXpar[3] = {0, 0, 0};
 
 void graph_with_chem() {
@@ -259,11 +267,36 @@ void graph_with_chem() {
   bmx_ctx_destroy(c);
 }
 
+// A capture that fails (in a launch, or when it is instantiated) and a graph
+// that does not launch leave the context where it was.
+void failed_capture() {
+  for (const char *where : {"force", "build", "instantiate", "graph"}) {
+    std::vector<uint8_t> recs;
+    sim::builds = 0;
+    bmx_ctx *c = bound(recs);
+    for (int32_t steps : {0, 4, kEvery}) {  // before the first row build, in
+      if (steps) CHECK(bmx_evolve(c, 1e-3, steps) == BMX_OK);  // a period, at its end
+      if (steps == 4) CHECK(bmx_exchange(c, kXpar, 1.0) == BMX_OK);
+      const auto m = bookkeeping(c);
+      sim::fail_at = where;
+      sim::fail_after = sim::fail_at == "force" ? 12 : 0;
+      CHECK(bmx_evolve_graph(c, 1e-3, 2 * kEvery) == BMX_ERR_HIP);
+      sim::fail_at.clear();
+      CHECK(bookkeeping(c) == m);
+      check_buffers(c);
+      CHECK(bmx_evolve_graph(c, 1e-3, 3) == BMX_OK);
+      check_buffers(c);
+    }
+    bmx_ctx_destroy(c);
+  }
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
   const std::string name = argc > 1 ? argv[1] : "";
   if (name == "graph_with_chem") graph_with_chem();
+  else if (name == "failed_capture") failed_capture();
   else return 2;
   return sim::bad ? 1 : 0;
 }
