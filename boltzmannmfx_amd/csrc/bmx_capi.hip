@@ -511,7 +511,8 @@ bmx_status close_run(bmx_ctx *c) {
 // skin/2 first and their partials cleared, so every caller that rebuilds
 // (steps, exchange, fusion, InitBonds) starts the next period from zero.
 // check_skin = false is for passes that repeat checked arithmetic.  The rows
-// and their lengths go to the context's arrays, or to those given.
+// and their lengths go to the context's arrays, or to those given; then the
+// context's own rows are those of an earlier order, and no list to step on.
 bmx_status rebuild(bmx_ctx *c, bool check_skin = true,
                    const FlatRows *rows = nullptr, int32_t *ncnt = nullptr) {
   hipStream_t s = c->stream;
@@ -549,6 +550,7 @@ bmx_status rebuild(bmx_ctx *c, bool check_skin = true,
   HIPCHK(launch_sort_gather(c->d_permk.p, c->d_start.p, c->n, ss, ds, sd, dd,
                             c->d_keytmp.p, multi, c->any_fungi ? 1 : 0,
                             c->d_err.p, s, chem_src, chem_dst));
+  c->have_list = false;  // another order: until its rows are built
   c->cs = 1 - c->cs;
   c->cd = 1 - c->cd;
   if (c->have_chem) c->cc = 1 - c->cc;
@@ -566,7 +568,7 @@ bmx_status rebuild(bmx_ctx *c, bool check_skin = true,
     HIPCHK(hipEventRecord(e1, s));
     c->ev_rebuild.push_back({e0, e1});
   }
-  c->have_list = true;
+  c->have_list = rows == nullptr;
   c->last_build = c->step;
   c->rebuilds_total++;
   return BMX_OK;

@@ -193,6 +193,9 @@ hipError_t launch_adj_step(const double4 *, const int32_t *, const uint8_t *, co
                            ForceParams, const double4 *, double4 *, double *, double *, hipStream_t) {
   return sim::op("adj_step", [] {});
 }
+hipError_t launch_export_counts(const int32_t *, const int32_t *, int64_t n, int64_t *out, hipStream_t) {
+  return sim::op("export", [=] { std::fill(out, out + n, 0); });
+}
 hipError_t launch_sum_partials(const double *, int64_t, int, double *, hipStream_t) {
   return sim::op("sum", [] {});
 }
@@ -291,12 +294,57 @@ void failed_capture() {
   }
 }
 
+// A row build that fails inside a list period leaves no list: the particles
+// are in another order than the rows.
+void failed_build() {
+  std::vector<uint8_t> recs;
+  bmx_ctx *c = bound(recs);
+  CHECK(bmx_evolve(c, 1e-3, 5) == BMX_OK);
+  sim::fail_at = "build";
+  sim::fail_after = 0;
+  CHECK(bmx_exchange(c, kXpar, 1.0) == BMX_ERR_HIP);
+  sim::fail_at.clear();
+  CHECK(!c->have_list);
+  CHECK(bmx_evolve(c, 1e-3, 1) == BMX_OK);
+  check_buffers(c);
+  CHECK(c->have_list && sim::builds == 2);
+  bmx_ctx_destroy(c);
+}
+
+// An adjoint call whose reverse pass fails: its recomputed rows went to the
+// history, so the context must not take its own rows as current.
+void adjoint_error() {
+  for (const char *where : {"adj_step", "force", "copy", "sum"}) {
+    std::vector<uint8_t> recs;
+    sim::builds = 0;
+    bmx_ctx *c = bound(recs);
+    CHECK(bmx_evolve(c, 1e-3, 5) == BMX_OK);
+    const std::vector<double> target(3 * kN, 0.0);
+    std::vector<double> grad_r(kN);
+    double loss = 0.0, grad[3];
+    sim::fail_at = where;
+    // past the forward pass: 40 steps of forces; 2 copies in, the error word
+    sim::fail_after = sim::fail_at == "force" ? 45 : sim::fail_at == "copy" ? 4 : 0;
+    CHECK(bmx_adjoint(c, 1e-3, 40, 2 * kEvery, target.data(), &loss, grad, grad_r.data(),
+                      nullptr) == BMX_ERR_HIP);
+    sim::fail_at.clear();
+    CHECK(sim::rows != c->d_cidx.p);  // the reverse pass had built rows
+    check_buffers(c);
+    int64_t total, offsets[kN + 1];
+    CHECK(bmx_get_neighbors(c, offsets, nullptr, 0, &total) == BMX_ERR_STATE);
+    bmx_ctx_destroy(c);
+  }
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
+  std::setvbuf(stdout, nullptr, _IONBF, 0);
   const std::string name = argc > 1 ? argv[1] : "";
   if (name == "graph_with_chem") graph_with_chem();
   else if (name == "failed_capture") failed_capture();
+  else if (name == "failed_build") failed_build();
+  else if (name == "adjoint_error") adjoint_error();
   else return 2;
   return sim::bad ? 1 : 0;
 }
