@@ -1446,8 +1446,11 @@ bmx_status evolve_guarded(bmx_ctx *c, double dt, int32_t nsteps) {
     // the snapshots hold the particle arrays only
     bmx_status sc = drop_chem(c);
     if (sc != BMX_OK) return sc;
-    // an error in an early period ends the call before the step that writes
-    // fc, which then still is the call before's
+    // Two periods are in flight: an error in a period before the last two
+    // ends the call before the step that writes fc, which then still is the
+    // call before's, and up to two reorders away from the order it was written
+    // in.  (An error in the last two, and so in any period of a call of at
+    // most K steps, leaves the fc of the call's last step.)
     if (nsteps > K) sc = keep_fc(c, true);
     if (sc != BMX_OK) return sc;
   }

@@ -256,3 +256,36 @@ def test_fc_of_the_call_before_a_failed_guarded_call(bmx, gpu):
     assert e.value.code == 5                          # a row over the capacity
     assert np.array_equal(ctx.fc(), fc)
     ctx.close()
+
+
+@pytest.mark.parametrize("nsteps", [7, 13, 20])
+def test_fc_of_a_guarded_call_that_fails_in_its_last_two_periods(bmx, gpu, nsteps):
+    """Two periods are in flight, so a guarded call that fails (a row over the
+    capacity) in one of its last two has taken the step that writes the
+    forces: those of the same steps without the guard, which fail alike."""
+    col = W.sphere_colony(3001, 0.25, 3, skin=2e-5)
+    rng = np.random.default_rng(5)
+    mid = 0.5 * (np.asarray(col.prob_lo) + np.asarray(col.prob_hi))
+    moved = col.recs["pos"][rng.permutation(len(col.recs))].copy()
+    moved[:40] = mid + rng.uniform(-1e-5, 1e-5, (40, 3))
+    dt = 1e-9 * col.dt
+    got = []
+    for guard in (False, True):
+        ctx = new_ctx(bmx, col, maxn=24)
+        ctx.set_guard(guard)
+        recs = col.recs.copy()
+        ctx.bind(recs)
+        ctx.evolve(dt, 25)
+        recs["pos"] = moved
+        ctx.refresh(bmx.FIELD_POSITIONS, recs)
+        with pytest.raises(bmx.BMXError) as e:
+            ctx.evolve(dt, nsteps)
+        assert e.value.code == 5                      # a row over the capacity
+        fc, pos = ctx.fc(), ctx.positions()
+        ctx.sync()
+        assert np.array_equal(recs["rdata"][:, 6:12], fc.T)
+        got.append((fc, pos))
+        ctx.close()
+    assert np.abs(got[0][0][:3]).max() > 0
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
