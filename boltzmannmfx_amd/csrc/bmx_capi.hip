@@ -485,6 +485,18 @@ bmx_status alloc_partials(bmx_ctx *c) {
   return BMX_OK;
 }
 
+// After setup_boxes has taken another reach (force parameters, re-read or
+// grown sizes): the rows' length, and with it the tile, may be another one.
+// Only a tile that changes costs anything.  24,000 spheres, us per force pass
+// with the tile of the old reach and of the new one: rows of 5 that become
+// rows of 0.8, 4.8 and 4.2; the other way round 8.7 and 5.6.
+bmx_status retile(bmx_ctx *c) {
+  if (flat_tile(c->any_fungi ? 1 : 0, c->n, row_estimate(c)) == c->flat_tile)
+    return BMX_OK;
+  bmx_status st = ensure_rows(c);
+  return st == BMX_OK ? alloc_partials(c) : st;
+}
+
 FlatRows flat_rows(bmx_ctx *c) {
   return FlatRows{c->flat_tile, c->d_cidx.p, c->d_cown.p, c->d_wtot.p, c->d_roff.p};
 }
@@ -1132,6 +1144,8 @@ bmx_status bmx_set_force_params(bmx_ctx *c, const double fpar[9]) {
       std::memcpy(c->fpar, old, sizeof old);
       return st;
     }
+    st = retile(c);
+    if (st != BMX_OK) return st;
   }
   c->have_fpar = true;
   return BMX_OK;
@@ -1658,6 +1672,7 @@ bmx_status bmx_refresh_from_aos(bmx_ctx *c, const void *aos, uint32_t fields) {
       c->rmax = rmax;
       c->lmax = lmax;
       st = setup_boxes(c);
+      if (st == BMX_OK) st = retile(c);
       if (st != BMX_OK) {
         c->bound = false;
         return st;
@@ -2625,6 +2640,7 @@ extern "C" bmx_status bmx_calc_txfr_particle(bmx_ctx *c, const double chempar[10
   std::memcpy(&c->lmax, c->h_flags + 18, sizeof(double));
   reset_graph(c);
   bmx_status sb = setup_boxes(c);
+  if (sb == BMX_OK) sb = retile(c);
   return st != BMX_OK ? st : sb;
 }
 

@@ -19,6 +19,7 @@ int fail_after = 0;   // ... after this many successful ones
 // left by the launches executed so far
 const void *chem = nullptr, *oid = nullptr, *rows = nullptr, *counts = nullptr;
 long builds = 0;
+double radius = 7e-5;  // the largest one the records hold
 bool counts_zero = false;
 int bad = 0;
 
@@ -93,7 +94,7 @@ void __hipRegisterVar(void **, void *, char *, char *, int, size_t, int, int) {}
 namespace bmx {
 int32_t tile_count(int64_t n, int tile) { return (int32_t)std::max<int64_t>(1, (n + tile - 1) / tile); }
 int64_t flat_entries(int64_t ncap, int, int32_t maxn) { return ncap * maxn + 128; }
-int flat_tile(int, int64_t, double row) { return row > 16.0 ? 4 : 64; }
+int flat_tile(int, int64_t, double row) { return row > 4.0 ? 4 : 64; }
 int64_t scan_scratch_elems(int64_t nb) { return nb / 2048 + 2; }
 int32_t adj_blocks(int64_t n, int tile) { return tile_count(n, 4 * tile); }
 int32_t adj_loss_blocks(int64_t n) { return tile_count(n, 256); }
@@ -111,11 +112,36 @@ hipError_t launch_aos_unpack(const uint8_t *, AosLayout, int64_t, const int32_t 
                              BoxGeom, StaticArrays st, DynArrays, unsigned long long *stats,
                              hipStream_t) {
   return sim::op("unpack", [=] {
-    const double r = 7e-5, l = 0.0;
-    std::memcpy(stats, &r, 8);
-    std::memcpy(stats + 1, &l, 8);
+    std::memcpy(stats, &sim::radius, 8);
+    stats[1] = 0;  // no segments
     stats[2] = 1;
     sim::oid = st.oid;
+  });
+}
+hipError_t launch_aos_refresh(const uint8_t *, AosLayout, int64_t, BoxGeom, StaticArrays, DynArrays,
+                              uint32_t, unsigned long long *stats, hipStream_t) {
+  return sim::op("refresh", [=] { std::memcpy(stats, &sim::radius, 8); });
+}
+hipError_t launch_mesh_bin(const double4 *, const int32_t *, int64_t, const MeshGeom &, int, int32_t *,
+                           int32_t *, int32_t *, int32_t *, int32_t *, unsigned long long *, int,
+                           int32_t *, unsigned long long *, hipStream_t) {
+  return sim::op("mesh_bin", [] {});
+}
+hipError_t launch_mesh_to_particle(double *, int64_t, const MeshGeom &, const int32_t *,
+                                   const int32_t *, const Topo *, double4 *, double4 *, const double *,
+                                   const double *, int, int, const double[10], double, int,
+                                   unsigned long long *maxima, int32_t *, hipStream_t) {
+  return sim::op("mesh", [=] {
+    std::memcpy(maxima, &sim::radius, 8);
+    maxima[1] = 0;
+  });
+}
+hipError_t launch_mesh_out(int32_t *err, const unsigned long long *maxima, int32_t *out_err,
+                           unsigned long long *out_max, hipStream_t) {
+  return sim::op("mesh_out", [=] {
+    *out_err = *err;
+    *err = 0;
+    if (maxima) std::memcpy(out_max, maxima, 16);
   });
 }
 hipError_t launch_bin_count(const double4 *, const int32_t *, const BoxGeom *, BoxGeom, int, int64_t,
@@ -336,6 +362,44 @@ void adjoint_error() {
   }
 }
 
+// The tile follows the reach, as a new bind with that reach would choose it,
+// and the arrays laid out by tiles with it.
+void check_tile(bmx_ctx *c, int tile) {
+  CHECK(c->flat_tile == tile && c->flat_tile == flat_tile(0, c->n, row_estimate(c)));
+  const size_t tiles = (size_t)tile_count(c->ncap, tile);
+  CHECK(c->vstride == (int32_t)tiles && c->d_vpart.n >= tiles * c->vmax_slots);
+  CHECK(c->d_wtot.n >= tiles && c->d_redo.n >= tiles && c->d_bstats.n >= 2 * tiles);
+  CHECK(bmx_evolve(c, 1e-3, 3) == BMX_OK);
+  check_buffers(c);
+  CHECK(bmx_evolve_graph(c, 1e-3, 3) == BMX_OK);
+  check_buffers(c);
+}
+void tile_follows_reach() {
+  std::vector<uint8_t> recs;
+  bmx_ctx *c = bound(recs);
+  check_tile(c, 64);
+  double fpar[9];
+  std::memcpy(fpar, kForce, sizeof fpar);
+  for (double band : {1.5e-4, 6e-6}) {  // the adhesion band W_A
+    fpar[0] = band;
+    CHECK(bmx_set_force_params(c, fpar) == BMX_OK);
+    check_tile(c, band > 1e-4 ? 4 : 64);
+  }
+  for (double radius : {1.3e-4, 7e-5}) {
+    sim::radius = radius;
+    CHECK(bmx_refresh_from_aos(c, nullptr, kFieldSizes) == BMX_OK);
+    check_tile(c, radius > 1e-4 ? 4 : 64);
+  }
+  const double chempar[10] = {};
+  const std::vector<double> x(3 * 6 * 6 * 6, 1.0);
+  for (double radius : {1.3e-4, 7e-5}) {
+    sim::radius = radius;
+    CHECK(bmx_calc_txfr_particle(c, chempar, x.data(), x.data(), 1.0, 1, 0, 0, 0) == BMX_OK);
+    check_tile(c, radius > 1e-4 ? 4 : 64);
+  }
+  bmx_ctx_destroy(c);
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -344,6 +408,7 @@ int main(int argc, char **argv) {
   if (name == "graph_with_chem") graph_with_chem();
   else if (name == "failed_capture") failed_capture();
   else if (name == "failed_build") failed_build();
+  else if (name == "tile_follows_reach") tile_follows_reach();
   else if (name == "adjoint_error") adjoint_error();
   else return 2;
   return sim::bad ? 1 : 0;

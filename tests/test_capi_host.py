@@ -28,7 +28,7 @@ def exe(tmp_path_factory):
 
 
 @pytest.mark.parametrize("case", ["graph_with_chem", "failed_capture", "failed_build",
-                                  "adjoint_error"])
+                                  "adjoint_error", "tile_follows_reach"])
 def test_bookkeeping_matches_the_launches(exe, case):
     p = subprocess.run([exe, case], capture_output=True, text=True, timeout=60)
     assert p.returncode == 0, p.stdout

@@ -130,3 +130,39 @@ def test_colonies_in_small_tiles(bmx, gpu):
         else:  # another order of the sums: 1e-16 of a force, 12 steps
             np.testing.assert_allclose(mine, alone, rtol=0, atol=1e-12 * col.prob_hi.max())
     both.close()
+
+
+@pytest.mark.parametrize("first,then", [(5e-5, 6e-6), (6e-6, 5e-5)])
+def test_tiles_follow_the_reach(bmx, gpu, first, then):
+    """A context whose adhesion band changes after steps lays its rows out in
+    the tiles of the new reach (32 and 16 here) and steps on as one bound there
+    with the new band."""
+    col = W.sphere_colony(24_001, 0.25, 5, W_A=5e-5, skin=2e-5, overlap_free=True)
+    dt = 1.0e-3 * W.DT
+    fpars = []
+    for band in (first, then):
+        f = np.array(col.fpar, float)
+        f[0] = band
+        fpars.append(f)
+    def bound(fpar, recs):
+        ctx = bmx.Context(0)
+        ctx.set_force_params(fpar)
+        ctx.set_geometry(col.prob_lo, col.prob_hi, col.periodic)
+        ctx.set_neighbor_params(mode=bmx.NBR_VERLET, rebuild_every=4, skin=2e-5, max_neighbors=192)
+        ctx.bind(recs)
+        return ctx
+    recs = col.recs.copy()
+    a = bound(fpars[0], recs)
+    a.evolve(dt, 5)
+    a.sync()
+    a.set_force_params(fpars[1])
+    b = bound(fpars[1], recs.copy())
+    for k in (3, 6):
+        a.evolve(dt, k)
+        b.evolve(dt, k)
+        assert np.array_equal(a.fc(), b.fc())
+        assert np.array_equal(a.positions(), b.positions())
+    for x, y in zip(a.neighbors(), b.neighbors()):
+        assert np.array_equal(x, y)
+    a.close()
+    b.close()
