@@ -2882,8 +2882,7 @@ constexpr size_t kNaBytes =
     + na_align(8 * kNaTiles * kNaRebuild)        // displacement slots
     + na_align(8 * kNaRebuild)                   // slot maxima
     + na_align(4 * 2 * kNaTiles)                 // row-build block stats
-    + na_align(4) + na_align(32) + na_align(8) + na_align(64)  // err, stats, total, ustats
-    + na_align(sizeof(BoxGeom));
+    + na_align(4) + na_align(32) + na_align(8) + na_align(64);  // err, stats, total, ustats
 
 static __device__ __align__(256) uint8_t scratch[kNaBytes];
 
@@ -2947,12 +2946,12 @@ bmx_status na_setup(NaDevice &d, int dev) {
   na_slice(c.d_stats, cur, 8);
   na_slice(c.d_total, cur, 1);
   na_slice(c.d_ustats, cur, 8);
-  na_slice(c.d_boxes, cur, 1);
   if ((size_t)(cur - ptr) > kNaBytes)
     return fail(BMX_ERR_HIP, "scratch layout exceeds the scratch array");
   // the record array is the caller's; a colony array is never needed
   c.d_aos.fixed = true;  // never used: the records are bound in place
   c.d_col_in.fixed = true;
+  c.d_boxes.fixed = true;  // one box: by value
   c.h_flags = d.flags;
   // host vectors reach their sizes here, not in a call
   c.colony_geom.reserve(1);

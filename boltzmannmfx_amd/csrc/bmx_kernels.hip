@@ -1482,7 +1482,6 @@ __device__ double general_finish(int64_t t, const BoxGeom &g,
     double th = rod_i.y, ph = rod_i.z;
     double w[3] = {acc[3], acc[4], acc[5]};
     rod_rotate(th, ph, tr_i, rod_i.x, w, fp.dt);
-    out.rod[t] = make_double4(rod_i.x, th, ph, rod_i.w);
     const double4 rod_o = make_double4(rod_i.x, th, ph, rod_i.w);
     const double4 tr_o = trig_of(th, ph);
     out.rod[t] = rod_o;
