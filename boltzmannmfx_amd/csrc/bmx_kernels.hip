@@ -2096,15 +2096,28 @@ int force_blocks(int64_t n, int tile, int block) {
 }
 // Lanes per particle of the row build.  More lanes shorten each particle's
 // chain of dependent loads, until the waves they make no longer fit the chip
-// at once.  Whole rebuilds, in us, 1.1-entry sphere rows unless said:
-//   n = 2,000:   16 lanes 29.6, 8 lanes 30.3, 4 lanes 32.0, 2 lanes 36.9
-//   24,000:      33.7, 32.8, 34.1, 37.7     (one lane per particle: 55)
-//   120,000:     8 lanes 49.5, 4 lanes 45.1, 2 lanes 46.1 (one lane: 58)
-//   300,000:     4 lanes 65.4, 2 lanes 67.2 (one lane: 68)
-//   1,000,000:   4 lanes 149.6, 2 lanes 139.1 (one lane: 146.8)
-//   segments, stencil rows, 20,000: 8 lanes 27.7, 4 lanes 29.8;
-//   200,000: 8 lanes 61.8, 4 lanes 55.8, 2 lanes 61.0
-// A block is one tile of at most 256 threads and at least one wave.
+// at once.  A block is one tile, at least one wave and at most 256 threads, so
+// the tile bounds the choice: tiles of 64 take 2 or 4 lanes, of 32 2 to 8, of
+// 16 4 to 16, of 8 8 or 16, and of 4 16 (the lines at 8,000 and 60,000 tell
+// the tiles below 64 apart; sparse spheres have 4 lanes up to 400,000).
+// Whole rebuilds, us, medians of runs that differ by 1 to 3, by lanes:
+//                                       16      8      4      2
+//   spheres, tiles of 64:    2,000                  33.7   36.8
+//                           24,000                  35.8   38.9
+//                          120,000                  43.9   45.2
+//                          300,000                  63.5   65.2
+//                        1,000,000                 136.9  134.7
+//   tiles of 32:             5,000           31.9   34.5   38.1
+//                           24,000           34.4   36.6   41.0
+//                          120,000           49.1   47.2   48.0
+//   tiles of 16:             5,000   33.5    35.4   39.9
+//                           24,000   36.1    36.7   40.5
+//                           90,000   54.2    50.0   50.1
+//   segments, stencil rows,
+//   tiles of 8:             20,000   28.2    28.2
+//   tiles of 16:            40,000   34.5    32.0   32.6
+//   tiles of 32:            60,000           35.1   35.3   38.8
+//                          200,000           63.5   58.4   61.4
 int build_lanes(int tile, int64_t n) {
   const int g = n > 400000 ? 2 : (n > 60000 ? 4 : (n > 8000 ? 8 : 16));
   return std::min(std::max(g, kWave / tile), 256 / tile);

@@ -2,8 +2,8 @@
 
 A context picks its tiles (particles per wave of a force pass) and the lanes
 per particle of the row build from its particle count and row length.  The
-cases below reach each of them, with counts that leave the last tile partly
-empty; rows, forces, positions and (segments) integer state must equal the
+cases below reach each pair of them but segments above 60,000 (tiles of 32 at
+4 and 2 lanes), with counts that leave the last tile partly empty; rows, forces, positions and (segments) integer state must equal the
 oracle's bit for bit, as everywhere else.
 """
 import numpy as np
@@ -29,14 +29,21 @@ def check(ctx, st, orecs, dt, steps, segments=False):
     st.close()
 
 
-# (n, phi, adhesion band, skin): tiles of 64 at 16, 8, 4 and 2 lanes per
-# particle (capped at 4 for 64-particle tiles), then 8 and 16 lanes at tiles
-# of 8, 16 and 32, and rows longer than what a tile stages on chip
-SPHERES = [(1, 0.01, 6e-6, 4e-6), (63, 0.05, 6e-6, 4e-6), (4097, 0.2, 6e-6, 4e-6),
-           (20_011, 0.2, 6e-6, 4e-6), (70_001, 0.15, 6e-6, 4e-6),
-           (410_003, 0.12, 6e-6, 4e-6), (3001, 0.2, 5e-5, 2e-5),
-           (30_001, 0.25, 5e-5, 2e-5), (61_001, 0.25, 5e-5, 2e-5),
-           (110_003, 0.25, 5e-5, 2e-5), (2503, 0.25, 5e-5, 1.5e-4)]
+# (n, phi, adhesion band, skin) and the tile and lanes per particle they get,
+# the last ones with rows longer than what a tile stages on chip
+SPHERES = [(1, 0.01, 6e-6, 4e-6),               # 64, 4
+           (63, 0.05, 6e-6, 4e-6),
+           (4097, 0.2, 6e-6, 4e-6),
+           (20_011, 0.2, 6e-6, 4e-6),
+           (70_001, 0.15, 6e-6, 4e-6),
+           (410_003, 0.12, 6e-6, 4e-6),         # 64, 2
+           (5003, 0.25, 5e-5, 5e-5),            # 8, 16
+           (3001, 0.2, 5e-5, 2e-5),             # 16, 16
+           (30_001, 0.25, 5e-5, 2e-5),          # 16, 8
+           (61_001, 0.25, 5e-5, 2e-5),          # 16, 4
+           (110_003, 0.25, 5e-5, 2e-5),         # 32, 4
+           (410_011, 0.25, 5e-5, 8e-5),         # 32, 2
+           (2503, 0.25, 5e-5, 1.5e-4)]          # 4, 16
 
 
 @pytest.mark.parametrize("n,phi,wa,skin", SPHERES)
@@ -58,7 +65,8 @@ def test_sphere_tiles(bmx, oracle, gpu, n, phi, wa, skin):
 
 @pytest.mark.parametrize("n", [5, 997, 25_003, 60_007])
 def test_stencil_sphere_tiles(bmx, oracle, gpu, n):
-    """The stencil policy's long rows: tiles of 4 and 8."""
+    """The stencil policy's rows: tiles of 32, 4, 8 and 16 (8, 16, 8 and 4
+    lanes)."""
     col = W.sphere_colony(n, 0.25, 9, W_A=5e-5, overlap_free=n < 50_000)
     hood = 1.1 * (2.0 * 7e-5 + 1e-2)
     if n == 5:
@@ -77,9 +85,10 @@ def test_stencil_sphere_tiles(bmx, oracle, gpu, n):
 
 
 @pytest.mark.parametrize("mode,K", [(1, 1), (0, 3)])
-@pytest.mark.parametrize("n", [7, 2051, 20_483, 41_003])
+@pytest.mark.parametrize("n", [7, 2051, 20_483, 41_003, 50_021])
 def test_segment_tiles(bmx, oracle, gpu, n, mode, K):
-    """Segments: tiles of 4, 8 and 16, either policy."""
+    """Segments: tiles of 4 (16 lanes), 8, 16 and 32 (8 lanes), either
+    policy."""
     col = W.c3_hyphae(n, nroots=max(1, n // 100), seed=3)
     hood = 1.1 * (2.0 * 2.0e-4 + 1.0e-2)
     ctx = bmx.Context(0)
