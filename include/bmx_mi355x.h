@@ -423,8 +423,8 @@ bmx_status bmx_fusion(bmx_ctx *ctx, const bmx_fusion_params *params,
 
 /* --- allocation-free evolve ---------------------------------------------
  * No counterpart in the reference.  For callers that cannot allocate device
- * memory (code under HIP graph capture, tight serving loops, harnesses that
- * forbid hipMalloc): one call does what bmx_bind_particles_aos (device
+ * memory (tight serving loops, harnesses that forbid hipMalloc; it waits for
+ * its stream, so it cannot itself be captured into a graph): one call does what bmx_bind_particles_aos (device
  * records) + bmx_evolve(dt, nsteps) + bmx_sync_to_aos do on a context, on
  * the caller's device records in place, with every working array in a
  * static device scratch the library holds per GPU (about 45 MB, from load
@@ -432,7 +432,8 @@ bmx_status bmx_fusion(bmx_ctx *ctx, const bmx_fusion_params *params,
  * BMX_NOALLOC_MAX_PARTICLES, max_neighbors <= BMX_NOALLOC_MAX_NEIGHBORS
  * (0 = that), rebuild_every <= BMX_NOALLOC_MAX_REBUILD_EVERY, at most
  * BMX_NOALLOC_MAX_BINS bins; beyond them BMX_ERR_BAD_ARG, before any GPU
- * work.  One box (no colonies).  stream: a hipStream_t, or NULL for the
+ * work (the bins, which follow from the sizes in the records, before any is
+ * changed).  One box (no colonies).  stream: a hipStream_t, or NULL for the
  * null stream; the call synchronizes it before returning.  Calls share
  * their GPU's scratch, which keeps the last call's contents: calls that
  * overlap on one GPU race. */
